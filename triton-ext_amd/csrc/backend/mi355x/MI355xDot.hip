@@ -226,6 +226,16 @@ const DecodeF8KernelFn kDecodeF8ScaledKernels[2][4] = {TX_DF8_SLICES(true, 0, 0,
                                                        TX_DF8_SLICES(true, 0, 0, true, false)};
 const DecodeF8KernelFn kDecodeI8KmajorKernels[4] = TX_DF8_SLICES(false, 0, 0, true, true);
 #undef TX_DF8_SLICES
+// MX operands: fp8 by [A e4m3 / e5m2][B e4m3 / e5m2][slice], and e2m1 by slice.
+#define TX_DMX_SLICES(FA, FB)                                                              \
+  {decode_f8_kernel<16, false, FA, FB, false, false, true>,                                \
+   decode_f8_kernel<32, false, FA, FB, false, false, true>,                                \
+   decode_f8_kernel<48, false, FA, FB, false, false, true>,                                \
+   decode_f8_kernel<64, false, FA, FB, false, false, true>}
+const DecodeF8KernelFn kDecodeMx8Kernels[2][2][4] = {
+    {TX_DMX_SLICES(0, 0), TX_DMX_SLICES(0, 1)}, {TX_DMX_SLICES(1, 0), TX_DMX_SLICES(1, 1)}};
+const DecodeF8KernelFn kDecodeMx4Kernels[4] = TX_DMX_SLICES(4, 4);
+#undef TX_DMX_SLICES
 // The 16-bit decode kernel by [B K-major][bf16][slice rows / 16 - 1], slices
 // of 16 .. 96 rows.
 typedef void (*Decode16KernelFn)(Decode16Args);
@@ -487,7 +497,8 @@ int64_t decode16Workspace(const tx_dot_desc &d, int ksplit) {
 // fp8 (e4m3 / e5m2 in any mix) with fp32 C; e4m3 x e4m3 with 128-block scales
 // and bf16 / fp32 C; with B K-major also int8 -> int32 and W8A8 at M <= 48
 // (past it the row kernel's K-major form; row-major int8 runs decode_i8.h);
-// M <= 64, one arrival counter per 128-column strip.
+// MX operands (e4m3 / e5m2 in any mix, or e2m1 on both sides) with bf16 / fp32
+// C; M <= 64, one arrival counter per 128-column strip.
 bool useDecodeF8(const tx_dot_desc &d) {
   const bool fa = d.a_type == TX_F8E4M3 || d.a_type == TX_F8E5M2;
   const bool fb = d.b_type == TX_F8E4M3 || d.b_type == TX_F8E5M2;
@@ -498,6 +509,9 @@ bool useDecodeF8(const tx_dot_desc &d) {
     return kmajor && d.M <= 48 &&
            ((d.scale_mode == TX_SCALE_NONE && d.c_type == TX_I32) ||
             (d.scale_mode == TX_SCALE_ROWCOL && d.c_type == TX_BF16));
+  if (d.scale_mode == TX_SCALE_MX32)
+    return ((fa && fb) || (d.a_type == TX_F4E2M1 && d.b_type == TX_F4E2M1)) && !kmajor &&
+           (d.c_type == TX_BF16 || d.c_type == TX_F32);
   if (!fa || !fb)
     return false;
   if (d.scale_mode == TX_SCALE_NONE)
@@ -505,14 +519,19 @@ bool useDecodeF8(const tx_dot_desc &d) {
   return d.scale_mode == TX_SCALE_BLOCK128 && d.a_type == TX_F8E4M3 &&
          d.b_type == TX_F8E4M3 && (d.c_type == TX_BF16 || d.c_type == TX_F32);
 }
-// Its tile: the slice (16 ceil(M / 16) rows) x a 128-column strip x 128-row
-// K batches (no 8-bit GEMM tile is narrower than 128 rows).
+// Its tile: the slice (16 ceil(M / 16) rows) x a 128-column strip x K batches
+// of 128 bytes a column: 128 elements, 256 of e2m1 (no 8-bit GEMM tile is
+// narrower than 128 rows).
+int decodeF8BatchK(const tx_dot_desc &d) {
+  return d.a_type == TX_F4E2M1 ? 2 * kDec8BatchK : kDec8BatchK;
+}
 bool decodeF8Tile(const tx_dot_desc &d) {
-  return d.block_m == decode16Rows(d) && d.block_n == kDec8StripN && d.block_k == kDec8BatchK;
+  return d.block_m == decode16Rows(d) && d.block_n == kDec8StripN &&
+         d.block_k == decodeF8BatchK(d);
 }
 int decodeF8Split(const tx_dot_desc &d) { // decode16Split's rule
   const int64_t strips = cdiv(d.N, kDec8StripN);
-  const int64_t batches = cdiv(d.K, kDec8BatchK);
+  const int64_t batches = cdiv(d.K, decodeF8BatchK(d));
   int ks = 1;
   while (ks < (int)kMaxSplit && strips * ks * 2 <= 256 && batches / (ks * 2) >= 4)
     ks *= 2;
@@ -1126,11 +1145,16 @@ int launchDecodeF8(const tx_dot_plan &plan, const void *A, const void *B, void *
   a.lda = d.lda;
   a.ldb = d.ldb;
   a.ldc = d.ldc;
-  a.sa_ld = (int32_t)cdiv(d.K, 128);
+  const bool mx = d.scale_mode == TX_SCALE_MX32, f4 = d.a_type == TX_F4E2M1;
+  if (f4) { // K and lda in bytes; B's packed rows
+    a.K = (int32_t)(d.K / 2);
+    a.lda = d.lda / 2;
+  }
+  a.sa_ld = (int32_t)(mx ? d.K / 32 : cdiv(d.K, 128));
   a.sb_ld = (int32_t)cdiv(d.N, 128);
   a.ksplit = ks;
-  a.batches_per_split = (int32_t)cdiv(cdiv(d.K, kDec8BatchK), ks);
-  a.k_main_batches = (int32_t)(plan.k_split / kDec8BatchK);
+  a.batches_per_split = (int32_t)cdiv(cdiv(d.K, decodeF8BatchK(d)), ks);
+  a.k_main_batches = (int32_t)(plan.k_split / decodeF8BatchK(d));
   a.counters = static_cast<uint32_t *>(ws);
   a.partials = need > 0 ? reinterpret_cast<float *>(static_cast<uint8_t *>(ws) +
                                                     kDecodeCounterBytes)
@@ -1139,6 +1163,8 @@ int launchDecodeF8(const tx_dot_plan &plan, const void *A, const void *B, void *
   const bool kmajor = (d.flags & TX_FLAG_B_KMAJOR) != 0;
   const DecodeF8KernelFn fn =
       d.a_type == TX_I8 ? kDecodeI8KmajorKernels[si]
+      : f4              ? kDecodeMx4Kernels[si]
+      : mx              ? kDecodeMx8Kernels[d.a_type == TX_F8E5M2][d.b_type == TX_F8E5M2][si]
       : scaled          ? kDecodeF8ScaledKernels[kmajor][si]
                         : kDecodeF8Kernels[kmajor][d.a_type == TX_F8E5M2][d.b_type == TX_F8E5M2][si];
   hipLaunchKernelGGL(fn, dim3(plan.grid_x), dim3(plan.block_threads), 0, stream, a);

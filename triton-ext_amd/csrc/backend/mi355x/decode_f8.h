@@ -62,11 +62,31 @@
 // scales, bf16 C, as decode_i8.h rounds it); per 16 x 16 block and batch two
 // v_mfma_i32_16x16x64_i8 on the same fragments (K bytes 32 G .. +15, then
 // +16 .. +31 of each lane), int32 partials, exact in any order.
+//
+// MX (tl.dot_scaled, row-major B): e4m3 / e5m2 in any mix, or e2m1 on both
+// sides, with e8m0 scales per 32 K that the MFMA applies.  A batch is 128
+// bytes of K: 128 fp8 elements (4 scale groups) or 256 fp4 ones (8), K, lda
+// and k0 counting bytes.  As on the 256x256 tile the scaled MFMA ties a
+// lane's scale byte to true K group l / 16, so fragments are read in that
+// order: A chunks G and 4 + G, B rows 16 G + {0, 8, 64, 72}.
+//   Scales: B's lie K / 32 bytes apart, one row a column, so a batch's 4 or 8
+// bytes a column would be a cache line each.  A segment's scales (SEG_B
+// batches; one segment is a whole split up to K = 4096) are staged at once,
+// before the ring's first loads: the strip's 128 columns and the slice's
+// rows, whole dwords from the row's first byte rounded down, rows an odd
+// number of dwords apart so that the 16 rows of a fragment fall in 16 banks.
+// Each further segment is loaded between two barriers.  Groups at or past
+// K / 32 (tail batch only) are replaced by 127: their data is zero, and only
+// a NaN scale could leak.
+//   Bound: HBM at N K large; a launch of few batches is the latency of the
+// scales, the ring's first batch and the split-K exchange in a row.  The
+// 256x256 tile covered N = 8192 with 32 workgroups here.
 #pragma once
 
 #include <type_traits>
 
 #include "decode16.h"
+#include "mfma_f4.h"
 
 namespace txk {
 
@@ -78,8 +98,8 @@ struct DecodeF8Args {
   const uint8_t *A;
   const uint8_t *B;
   void *C;
-  const float *sa;   // SCALED: [M][sa_ld]
-  const float *sb;   // SCALED: [ceil(K / 128)][sb_ld]
+  const float *sa;   // SCALED: [M][sa_ld]; MX: e8m0 bytes [M][sa_ld]
+  const float *sb;   // SCALED: [ceil(K / 128)][sb_ld]; MX: e8m0 bytes [N][sa_ld]
   int32_t c_f32;     // fp32 C (else bf16)
   int32_t acc_c;     // fp32 / int32 C: add the sums to C's contents (tl.dot's acc)
   int32_t rowcol;    // I8: W8A8, C = bf16((float(sum) * sa[m]) * sb[n]) (else int32 C)
@@ -97,14 +117,20 @@ __host__ __device__ constexpr int64_t decode_f8_split_bytes(int64_t strips, int 
   return strips * sr * kDec8StripN * 4;
 }
 
-template <int SR, bool SCALED> struct DecodeF8Cfg {
+template <int SR, bool SCALED, bool MX = false, bool F4 = false> struct DecodeF8Cfg {
   static constexpr int T = SR / 16;
   static constexpr int A_LOADS = (SR + 31) / 32;            // per wave: 8 rows a load
   static constexpr int A_OFF = kDec8BatchK * kDec8StripN;   // B's 16 KiB first
   static constexpr int SCL_OFF = A_OFF + kDecodeWaves * A_LOADS * 1024;
   static constexpr int SLOT = SCL_OFF + (SCALED ? 1024 : 0); // 256 bytes of scales a wave
-  static constexpr int S = 158 * 1024 / SLOT > 8 ? 8 : 158 * 1024 / SLOT;
+  // MX: scale groups a batch, batches a segment (128 groups), rows of scales
+  // (columns of the strip, then rows of the slice) and their LDS dwords.
+  static constexpr int GPB = F4 ? 8 : 4, SEG_B = 128 / GPB, SROWS = kDec8StripN + SR;
+  static constexpr int MXS_BYTES = MX ? SROWS * 33 * 4 : 0;
+  static constexpr int S_FIT = (158 * 1024 - MXS_BYTES) / SLOT;
+  static constexpr int S = S_FIT > 8 ? 8 : S_FIT;
   static constexpr int VPB = 4 + A_LOADS + (SCALED ? 1 : 0);
+  static_assert(!MX || (S - 1) * VPB + (SROWS * 33 + 255) / 256 <= 63, "vmcnt is 6 bits");
   static_assert(SR == 16 || SR == 32 || SR == 48 || SR == 64, "slices of 16 .. 64 rows");
   static_assert(S >= 3 && (S - 2) * VPB <= 63, "ring depth; vmcnt is 6 bits");
 };
@@ -114,54 +140,60 @@ template <int SR, bool SCALED> struct DecodeF8Cfg {
 // fragments (two 16-byte reads each, at a0 and a0 ^ 16, +2 KiB per tile),
 // waiting for them before the block ends.  Outputs are early-clobber: a
 // read lands while later reads of the block still use their address registers.
-#define TX_D8_TR                                                                           \
-  "ds_read_b64_tr_b8 %0, %[b0]\n\tds_read_b64_tr_b8 %1, %[b0] offset:1024\n\t"             \
-  "ds_read_b64_tr_b8 %2, %[b0] offset:2048\n\tds_read_b64_tr_b8 %3, %[b0] offset:3072\n\t" \
-  "ds_read_b64_tr_b8 %4, %[b1]\n\tds_read_b64_tr_b8 %5, %[b1] offset:1024\n\t"             \
-  "ds_read_b64_tr_b8 %6, %[b1] offset:2048\n\tds_read_b64_tr_b8 %7, %[b1] offset:3072\n\t"
+#define TX_D8_TR4(o1, o2, o3)                                                              \
+  "ds_read_b64_tr_b8 %0, %[b0]\n\tds_read_b64_tr_b8 %1, %[b0] offset:" o1 "\n\t"          \
+  "ds_read_b64_tr_b8 %2, %[b0] offset:" o2 "\n\tds_read_b64_tr_b8 %3, %[b0] offset:" o3 "\n\t" \
+  "ds_read_b64_tr_b8 %4, %[b1]\n\tds_read_b64_tr_b8 %5, %[b1] offset:" o1 "\n\t"          \
+  "ds_read_b64_tr_b8 %6, %[b1] offset:" o2 "\n\tds_read_b64_tr_b8 %7, %[b1] offset:" o3 "\n\t"
 #define TX_D8_OUT                                                                         \
   "=&v"(bq[0][0]), "=&v"(bq[0][1]), "=&v"(bq[0][2]), "=&v"(bq[0][3]), "=&v"(bq[1][0]),        \
       "=&v"(bq[1][1]), "=&v"(bq[1][2]), "=&v"(bq[1][3])
 #define TX_D8_IN [b0] "v"(b0), [b1] "v"(b1), [a0] "v"(a0), [a1] "v"(a1)
-template <int T>
-__device__ __forceinline__ void dec8_read(uint32_t b0, uint32_t b1, uint32_t a0, uint32_t a1,
-                                          v2i_t (&bq)[2][4], i32x4_t (&a)[T][2]) {
-  if constexpr (T == 1)
-    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"
-                          "s_waitcnt lgkmcnt(0)"
-                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1])
-                 : TX_D8_IN
-                 : "memory");
-  else if constexpr (T == 2)
-    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"
-                          "ds_read_b128 %10, %[a0] offset:2048\n\tds_read_b128 %11, %[a1] offset:2048\n\t"
-                          "s_waitcnt lgkmcnt(0)"
-                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1])
-                 : TX_D8_IN
-                 : "memory");
-  else if constexpr (T == 3)
-    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"
-                          "ds_read_b128 %10, %[a0] offset:2048\n\tds_read_b128 %11, %[a1] offset:2048\n\t"
-                          "ds_read_b128 %12, %[a0] offset:4096\n\tds_read_b128 %13, %[a1] offset:4096\n\t"
-                          "s_waitcnt lgkmcnt(0)"
-                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]),
-                   "=&v"(a[2][0]), "=&v"(a[2][1])
-                 : TX_D8_IN
-                 : "memory");
-  else
-    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"
-                          "ds_read_b128 %10, %[a0] offset:2048\n\tds_read_b128 %11, %[a1] offset:2048\n\t"
-                          "ds_read_b128 %12, %[a0] offset:4096\n\tds_read_b128 %13, %[a1] offset:4096\n\t"
-                          "ds_read_b128 %14, %[a0] offset:6144\n\tds_read_b128 %15, %[a1] offset:6144\n\t"
-                          "s_waitcnt lgkmcnt(0)"
-                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]),
-                   "=&v"(a[2][0]), "=&v"(a[2][1]), "=&v"(a[3][0]), "=&v"(a[3][1])
-                 : TX_D8_IN
-                 : "memory");
+// One asm statement per row-tile count, instantiated for the two row patterns
+// of the transposed reads (rows 8 apart; MX: 8, 64 and 72 further).
+#define TX_D8_READ(NAME, TX_D8_TR)                                                          \
+template <int T>                                                                                           \
+__device__ __forceinline__ void NAME(uint32_t b0, uint32_t b1, uint32_t a0, uint32_t a1,                   \
+                                          v2i_t (&bq)[2][4], i32x4_t (&a)[T][2]) {                         \
+  if constexpr (T == 1)                                                                                    \
+    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"                           \
+                          "s_waitcnt lgkmcnt(0)"                                                           \
+                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1])                                               \
+                 : TX_D8_IN                                                                                \
+                 : "memory");                                                                              \
+  else if constexpr (T == 2)                                                                               \
+    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"                           \
+                          "ds_read_b128 %10, %[a0] offset:2048\n\tds_read_b128 %11, %[a1] offset:2048\n\t" \
+                          "s_waitcnt lgkmcnt(0)"                                                           \
+                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1])               \
+                 : TX_D8_IN                                                                                \
+                 : "memory");                                                                              \
+  else if constexpr (T == 3)                                                                               \
+    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"                           \
+                          "ds_read_b128 %10, %[a0] offset:2048\n\tds_read_b128 %11, %[a1] offset:2048\n\t" \
+                          "ds_read_b128 %12, %[a0] offset:4096\n\tds_read_b128 %13, %[a1] offset:4096\n\t" \
+                          "s_waitcnt lgkmcnt(0)"                                                           \
+                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]),              \
+                   "=&v"(a[2][0]), "=&v"(a[2][1])                                                          \
+                 : TX_D8_IN                                                                                \
+                 : "memory");                                                                              \
+  else                                                                                                     \
+    asm volatile(TX_D8_TR "ds_read_b128 %8, %[a0]\n\tds_read_b128 %9, %[a1]\n\t"                           \
+                          "ds_read_b128 %10, %[a0] offset:2048\n\tds_read_b128 %11, %[a1] offset:2048\n\t" \
+                          "ds_read_b128 %12, %[a0] offset:4096\n\tds_read_b128 %13, %[a1] offset:4096\n\t" \
+                          "ds_read_b128 %14, %[a0] offset:6144\n\tds_read_b128 %15, %[a1] offset:6144\n\t" \
+                          "s_waitcnt lgkmcnt(0)"                                                           \
+                 : TX_D8_OUT, "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]),              \
+                   "=&v"(a[2][0]), "=&v"(a[2][1]), "=&v"(a[3][0]), "=&v"(a[3][1])                          \
+                 : TX_D8_IN                                                                                \
+                 : "memory");                                                                              \
 }
+TX_D8_READ(dec8_read, TX_D8_TR4("1024", "2048", "3072"))
+TX_D8_READ(dec8_read_mx, TX_D8_TR4("1024", "8192", "9216"))
+#undef TX_D8_READ
 #undef TX_D8_IN
 #undef TX_D8_OUT
-#undef TX_D8_TR
+#undef TX_D8_TR4
 
 // The same with B K-major: each column block's fragment is two 16-byte reads
 // (at b0 / b1 and their ^ 16, chunks 2 G and 2 G + 1), like A's, which are
@@ -210,17 +242,94 @@ __device__ __forceinline__ void dec8_read_kmajor(uint32_t b0, uint32_t b1, uint3
 #undef TX_D8K_O
 #undef TX_D8K_T
 
-// FA, FB: the MFMA format codes of A and B (0 e4m3, 1 e5m2); SCALED takes
-// e4m3 x e4m3 with block scales.  BT: B K-major; I8: int8 -> int32 (BT only).
-template <int SR, bool SCALED, int FA = 0, int FB = 0, bool BT = false, bool I8 = false>
+// MX scale operands of the wave's two column blocks (bytes at x0 / x1) and T
+// row tiles (at xa, `TB` bytes a tile): byte 0 the lane's group and, for fp4,
+// byte 1 the group four further (the second MFMA of a batch).  Reads and wait
+// in one block, early-clobber, as above.
+#define TX_MXS(i, addr) "ds_read_u8 %[v" #i "], " addr "\n\t"
+#define TX_MXS4(i, addr) TX_MXS(i, addr) "ds_read_u8 %[w" #i "], " addr " offset:4\n\t"
+#define TX_MXS_B(R) R(0, "%[x0]") R(1, "%[x1]")
+#define TX_MXS_O(i) [v##i] "=&v"(v[i])
+#define TX_MXS4_O(i) [v##i] "=&v"(v[i]), [w##i] "=&v"(w[i])
+#define TX_MXS_W "s_waitcnt lgkmcnt(0)"
+#define TX_MXS_IN [x0] "v"(x0), [x1] "v"(x1), [a0] "v"(xa)
+template <int T, bool F4>
+__device__ __forceinline__ void dec8_read_scales(uint32_t x0, uint32_t x1, uint32_t xa, uint32_t tb,
+                                                 int (&sc)[2 + T]) {
+  uint32_t v[6], w[6] = {0, 0, 0, 0, 0, 0};
+  const uint32_t xb = xa + tb, xc = xa + 2 * tb, xd = xa + 3 * tb;
+  if constexpr (T == 1 && !F4)
+    asm volatile(TX_MXS_B(TX_MXS) TX_MXS(2, "%[a0]") TX_MXS_W
+                 : TX_MXS_O(0), TX_MXS_O(1), TX_MXS_O(2)
+                 : TX_MXS_IN
+                 : "memory");
+  else if constexpr (T == 2 && !F4)
+    asm volatile(TX_MXS_B(TX_MXS) TX_MXS(2, "%[a0]") TX_MXS(3, "%[a1]") TX_MXS_W
+                 : TX_MXS_O(0), TX_MXS_O(1), TX_MXS_O(2), TX_MXS_O(3)
+                 : TX_MXS_IN, [a1] "v"(xb)
+                 : "memory");
+  else if constexpr (T == 3 && !F4)
+    asm volatile(TX_MXS_B(TX_MXS) TX_MXS(2, "%[a0]") TX_MXS(3, "%[a1]") TX_MXS(4, "%[a2]") TX_MXS_W
+                 : TX_MXS_O(0), TX_MXS_O(1), TX_MXS_O(2), TX_MXS_O(3), TX_MXS_O(4)
+                 : TX_MXS_IN, [a1] "v"(xb), [a2] "v"(xc)
+                 : "memory");
+  else if constexpr (!F4)
+    asm volatile(TX_MXS_B(TX_MXS) TX_MXS(2, "%[a0]") TX_MXS(3, "%[a1]") TX_MXS(4, "%[a2]")
+                 TX_MXS(5, "%[a3]") TX_MXS_W
+                 : TX_MXS_O(0), TX_MXS_O(1), TX_MXS_O(2), TX_MXS_O(3), TX_MXS_O(4), TX_MXS_O(5)
+                 : TX_MXS_IN, [a1] "v"(xb), [a2] "v"(xc), [a3] "v"(xd)
+                 : "memory");
+  else if constexpr (T == 1)
+    asm volatile(TX_MXS_B(TX_MXS4) TX_MXS4(2, "%[a0]") TX_MXS_W
+                 : TX_MXS4_O(0), TX_MXS4_O(1), TX_MXS4_O(2)
+                 : TX_MXS_IN
+                 : "memory");
+  else if constexpr (T == 2)
+    asm volatile(TX_MXS_B(TX_MXS4) TX_MXS4(2, "%[a0]") TX_MXS4(3, "%[a1]") TX_MXS_W
+                 : TX_MXS4_O(0), TX_MXS4_O(1), TX_MXS4_O(2), TX_MXS4_O(3)
+                 : TX_MXS_IN, [a1] "v"(xb)
+                 : "memory");
+  else if constexpr (T == 3)
+    asm volatile(TX_MXS_B(TX_MXS4) TX_MXS4(2, "%[a0]") TX_MXS4(3, "%[a1]") TX_MXS4(4, "%[a2]")
+                 TX_MXS_W
+                 : TX_MXS4_O(0), TX_MXS4_O(1), TX_MXS4_O(2), TX_MXS4_O(3), TX_MXS4_O(4)
+                 : TX_MXS_IN, [a1] "v"(xb), [a2] "v"(xc)
+                 : "memory");
+  else
+    asm volatile(TX_MXS_B(TX_MXS4) TX_MXS4(2, "%[a0]") TX_MXS4(3, "%[a1]") TX_MXS4(4, "%[a2]")
+                 TX_MXS4(5, "%[a3]") TX_MXS_W
+                 : TX_MXS4_O(0), TX_MXS4_O(1), TX_MXS4_O(2), TX_MXS4_O(3), TX_MXS4_O(4),
+                   TX_MXS4_O(5)
+                 : TX_MXS_IN, [a1] "v"(xb), [a2] "v"(xc), [a3] "v"(xd)
+                 : "memory");
+#pragma unroll
+  for (int i = 0; i < 2 + T; ++i)
+    sc[i] = (int)(v[i] | (w[i] << 8));
+}
+#undef TX_MXS
+#undef TX_MXS4
+#undef TX_MXS_B
+#undef TX_MXS_O
+#undef TX_MXS4_O
+#undef TX_MXS_W
+#undef TX_MXS_IN
+
+// FA, FB: the MFMA format codes of A and B (0 e4m3, 1 e5m2; with MX also 4,
+// e2m1 on both sides); SCALED takes e4m3 x e4m3 with block scales.  BT: B
+// K-major; I8: int8 -> int32 (BT only); MX: e8m0 scales per 32 K.
+template <int SR, bool SCALED, int FA = 0, int FB = 0, bool BT = false, bool I8 = false,
+          bool MX = false>
 __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode_f8_kernel(DecodeF8Args p) {
   static_assert(!SCALED || (FA == 0 && FB == 0), "block scales take e4m3 operands");
   static_assert(!I8 || (BT && FA == 0 && FB == 0), "int8: the K-major form");
-  typedef DecodeF8Cfg<SR, SCALED> Cfg;
+  static_assert(!MX || (!SCALED && !BT && (FA == 4) == (FB == 4)), "MX: row-major B");
+  constexpr bool F4 = MX && FA == 4;
+  typedef DecodeF8Cfg<SR, SCALED, MX, F4> Cfg;
   constexpr int S = Cfg::S, SLOT = Cfg::SLOT, T = Cfg::T;
   typedef std::conditional_t<I8, i32x4_t, f32x4_t> Acc;
   __shared__ __attribute__((aligned(1024))) uint8_t ring[S * SLOT];
   __shared__ uint32_t last_flag;
+  __shared__ __attribute__((aligned(256))) uint8_t mxs[MX ? (Cfg::MXS_BYTES + 255) / 256 * 256 : 4];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -311,14 +420,52 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode_f8_kernel(DecodeF
   // +1 KiB per read.  A, tile t: row 16 t + L ((row >> 1) & 7 = L / 2),
   // chunks 2 G and 2 G + 1 (the second at the first ^ 16): +2 KiB per tile.
   // K-major B, block j: storage row 16 j + L, chunks 2 G and 2 G + 1, like A.
+  // MX: B rows 16 G + L / 2 (+8, +64, +72), A chunks G and 4 + G (^ 64).
   uint32_t b_off[2];
 #pragma unroll
   for (int jj = 0; jj < 2; ++jj) {
     const int j = 2 * wave + jj;
     b_off[jj] = BT ? (16 * j + L) * 128 + (((2 * G) ^ (L >> 1)) << 4)
-                   : (32 * G + (L >> 1)) * 128 + ((j ^ (L >> 1)) << 4) + 8 * (L & 1);
+                   : ((MX ? 16 : 32) * G + (L >> 1)) * 128 + ((j ^ (L >> 1)) << 4) + 8 * (L & 1);
   }
-  const uint32_t a_off = Cfg::A_OFF + L * 128 + (((2 * G) ^ (L >> 1)) << 4);
+  const uint32_t a_off = Cfg::A_OFF + L * 128 + (((MX ? G : 2 * G) ^ (L >> 1)) << 4);
+
+  // MX scales.  Row r < 128 is column n0 + r of B, row 128 + r row r of A; a
+  // row holds `pitch` dwords from its first byte of the segment rounded down
+  // (an odd number, enough for the split's groups of the segment and up to 3
+  // bytes of misalignment).
+  const int seg_groups = (nb < Cfg::SEG_B ? nb : Cfg::SEG_B) * Cfg::GPB;
+  const int pitch = MX ? ((seg_groups + 3 + 3) / 4) | 1 : 1; // <= 33
+  auto stage_scales = [&](int i0) { // batches i0 .. i0 + SEG_B - 1 of the split
+    const int64_t g0 = (int64_t)(b_begin + i0) * Cfg::GPB;
+    const int items = Cfg::SROWS * pitch;
+    const int64_t a_bytes = ((int64_t)p.M * p.sa_ld + 3) & ~3ll,
+                  b_bytes = ((int64_t)p.N * p.sa_ld + 3) & ~3ll;
+    for (int q0 = 64 * wave; q0 < items; q0 += 64 * kDecodeWaves) {
+      const int q = q0 + lane, r = q / pitch, dw = q - r * pitch;
+      const bool is_b = r < kDec8StripN;
+      const int64_t row = is_b ? n0 + r : r - kDec8StripN;
+      const int64_t at = ((row * p.sa_ld + g0) & ~3ll) + 4 * dw;
+      const void *src = reinterpret_cast<const uint8_t *>(is_b ? p.sb : p.sa) + at;
+      // (whole dwords: each holds at least one byte of the array)
+      if (q >= items || row >= (is_b ? p.N : p.M) || at >= (is_b ? b_bytes : a_bytes))
+        src = tx_zero_chunk;
+      __builtin_amdgcn_global_load_lds(src, (lds_void *)(mxs + 4 * q0), 4, 0, 0);
+    }
+  };
+  // This lane's scale bytes: the two column blocks and row tile 0 (a tile is
+  // 16 rows further, the same misalignment as 16 K / 32 % 4 == 0).
+  uint32_t xs[3] = {0, 0, 0};
+  if constexpr (MX) {
+    const uint32_t g0 = (uint32_t)b_begin * Cfg::GPB; // a multiple of 4
+#pragma unroll
+    for (int jj = 0; jj < 3; ++jj) {
+      const int r = jj < 2 ? 16 * (2 * wave + jj) + L : L;
+      const uint32_t row = jj < 2 ? (uint32_t)n0 + r : (uint32_t)r;
+      xs[jj] = lds_addr(mxs) + 4u * (uint32_t)((jj < 2 ? r : kDec8StripN + r) * pitch) +
+               ((row * (uint32_t)p.sa_ld + g0) & 3u) + G;
+    }
+  }
 
   // operand formats FB (MFMA A := B columns) and FA; no hardware scales
   auto mma = [&](const i32x8_t &bcol, const i32x8_t &arow, f32x4_t c) -> f32x4_t {
@@ -332,10 +479,27 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode_f8_kernel(DecodeF
     i32x4_t a[T][2];
     if constexpr (BT)
       dec8_read_kmajor<T>(base + b_off[0], base + b_off[1], base + a_off, bk, a);
+    else if constexpr (MX)
+      dec8_read_mx<T>(base + b_off[0], base + b_off[1], base + a_off, (base + a_off) ^ 64u, bq, a);
     else
       dec8_read<T>(base + b_off[0], base + b_off[1], base + a_off, (base + a_off) ^ 16u, bq, a);
     const int b = batch(i);
-    if (b >= p.k_main_batches) { // the K tail: bytes of A (and K-major B) at or past K
+    int sx[2 + T];
+    if constexpr (MX) {
+      const uint32_t at = (uint32_t)(i % Cfg::SEG_B) * Cfg::GPB;
+      dec8_read_scales<T, F4>(xs[0] + at, xs[1] + at, xs[2] + at, 64u * (uint32_t)pitch, sx);
+      if (b >= p.k_main_batches) { // groups at or past K / 32 (whole 16-byte chunks: no byte masks)
+        const int g = b * Cfg::GPB + G;
+#pragma unroll
+        for (int x = 0; x < 2 + T; ++x) {
+          if (g >= p.sa_ld)
+            sx[x] = (sx[x] & ~0xff) | 127;
+          if (F4 && g + 4 >= p.sa_ld)
+            sx[x] = (sx[x] & 0xff) | (127 << 8);
+        }
+      }
+    }
+    if (!MX && b >= p.k_main_batches) { // the K tail: bytes of A (and K-major B) at or past K
       const int64_t k = (int64_t)b * kDec8BatchK + 32 * G;
 #pragma unroll
       for (int t = 0; t < T; ++t) {
@@ -384,7 +548,17 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode_f8_kernel(DecodeF
         for (int t = 0; t < T; ++t) {
           const i32x8_t arow = {a[t][0][0], a[t][0][1], a[t][0][2], a[t][0][3],
                                 a[t][1][0], a[t][1][1], a[t][1][2], a[t][1][3]};
-          if constexpr (SCALED) {
+          if constexpr (F4) {
+            const i32x4_t b0 = {bcol[0], bcol[1], bcol[2], bcol[3]},
+                          b1 = {bcol[4], bcol[5], bcol[6], bcol[7]};
+            acc[t][jj] = txk_mfma_scale_16x16x128_f4(b0, a[t][0], acc[t][jj], 4, 4, 0, sx[jj], 0,
+                                                     sx[2 + t]);
+            acc[t][jj] = txk_mfma_scale_16x16x128_f4(b1, a[t][1], acc[t][jj], 4, 4, 1, sx[jj], 1,
+                                                     sx[2 + t]);
+          } else if constexpr (MX) {
+            acc[t][jj] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                bcol, arow, acc[t][jj], FB, FA, 0, sx[jj], 0, sx[2 + t]);
+          } else if constexpr (SCALED) {
             const f32x4_t part = mma(bcol, arow, f32x4_t{0, 0, 0, 0});
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -397,7 +571,11 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode_f8_kernel(DecodeF
     }
   };
 
-  // Prologue: S - 1 batches in flight; batch i uses slot i % S.
+  // Prologue: S - 1 batches in flight; batch i uses slot i % S.  (MX: the
+  // first segment's scales before them, so that waiting for batch 0 waits for
+  // the scales.)
+  if constexpr (MX)
+    stage_scales(0);
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
     issue(s, ring + s * SLOT);
@@ -409,6 +587,13 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode_f8_kernel(DecodeF
       const int i = i0 + s;
       if (i >= nb)
         goto k_loop_done;
+      if constexpr (MX) {
+        if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
+          asm volatile("s_barrier" ::: "memory");
+          stage_scales(i);
+          wait_vmcnt<0>();
+        }
+      }
       wait_vmcnt<(S - 2) * Cfg::VPB>();
       asm volatile("s_barrier" ::: "memory");
       issue(i + S - 1, ring + ((s + S - 1) % S) * SLOT);

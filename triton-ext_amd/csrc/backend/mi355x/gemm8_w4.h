@@ -70,17 +70,9 @@
 #include <type_traits>
 
 #include "gemm16_w4.h"
+#include "mfma_f4.h"
 
 namespace txk {
-
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
-
-// The fp4 form of the scaled MFMA reads 4-dword operands: the intrinsic's
-// v4i32 overload, called by its LLVM name (the clang builtin is declared for
-// 8-dword operands only).
-extern "C" __device__ f32x4_t txk_mfma_scale_16x16x128_f4(i32x4_t, i32x4_t, f32x4_t, int, int,
-                                                          int, int, int, int)
-    __asm("llvm.amdgcn.mfma.scale.f32.16x16x128.f8f6f4.v4i32.v4i32");
 
 // FA, FB: MFMA format codes of A and B (0 e4m3, 1 e5m2; 4 e2m1 with the MX
 // epilogues only); the unscaled fp8 dot takes e4m3 / e5m2 in any mix.

@@ -233,7 +233,8 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
     // fp32 C, e4m3 x e4m3 with 128-block scales and bf16 / fp32 C, M <= 64;
     // with B K-major also int8 -> int32 and W8A8, M <= 48 (the row kernel's
     // 32 x 32 x 32 products take M = 64: W8A8 22.4 against 26.8 us at
-    // N = K = 8192); N up to its 16384 strips of 128 columns.
+    // N = K = 8192); MX operands (fp8 pairs or e2m1 on both sides) with bf16 /
+    // fp32 C; N up to its 16384 strips of 128 columns.
     const bool fp8a = d->a_type == TX_F8E4M3 || d->a_type == TX_F8E5M2;
     const bool fp8b = d->b_type == TX_F8E4M3 || d->b_type == TX_F8E5M2;
     const bool kmajor = (d->flags & TX_FLAG_B_KMAJOR) != 0;
@@ -245,9 +246,14 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
          (kmajor && d->a_type == TX_I8 && d->b_type == TX_I8 && d->M <= 48 &&
           ((d->scale_mode == TX_SCALE_NONE && d->c_type == TX_I32) ||
            (d->scale_mode == TX_SCALE_ROWCOL && d->c_type == TX_BF16))));
+    const bool decode_mx = d->scale_mode == TX_SCALE_MX32 && !upcast && !kmajor && d->M <= 64 &&
+                           d->N <= (int64_t)16384 * 128 &&
+                           (d->c_type == TX_BF16 || d->c_type == TX_F32);
     const size_t first = spanA < TX_SPAN32_LIMIT && spanB < TX_SPAN32_LIMIT ? 0 : 1;
     if (upcast)
       t = chooseTile(kTiles16, d->M, d->N, d->K, kPeak16 / 2 / kCUs, first); // MX x bf16: bf16 tile
+    else if (decode_mx)
+      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, ba == 4 ? 256 : 128, 1.0};
     else if (d->scale_mode == TX_SCALE_MX32)
       t = ba == 4 ? kTileMx4 : kTileMx8;
     else if (decode_f8)
