@@ -123,7 +123,11 @@ typedef enum tx_kernel {
   TX_KERNEL_DECODE_F8 = 8,    /* 8-bit decode shapes (M <= 64): fp8 unscaled or
                                * with 128-block scales, and int8 (int32 C or
                                * W8A8, M <= 48) with B K-major; B streamed
-                               * once, MFMA 16x16x128 (int8: 16x16x64)       */
+                               * once, MFMA 16x16x128 (int8: 16x16x64); MX
+                               * operands (M <= 64) by the scaled MFMA       */
+  TX_KERNEL_DECODE_MX_BF16 = 9, /* scaled B (MX, or e2m1 with e4m3 scales) x bf16 of
+                                 * decode shape (M <= 96): B streamed once and
+                                 * upcast in registers, MFMA 16x16x32          */
 } tx_kernel;
 
 /* Bit flags for tx_dot_desc.flags */

@@ -1,16 +1,20 @@
 """GPU parity of the MX decode kernels (dot_scaled with a few rows of A) against the oracle.
 
 MX x MX (decode_f8.h's MX form): the scaled MFMA's own bound (test_mx_gpu.check_mx).
-Shapes sit at the edges: slices of 16 .. 64 rows, N and K that fill no strip
+bf16 x MX and e4m3 scales (decode16.h's WQ form): the operand upcast is exact, so the
+result is within fp32 summation error of the oracle, K 2^-24 sum |a b|, plus one bf16 ulp
+for bf16 C.  Shapes sit at the edges: slices of 16 .. 96 rows, N and K that fill no strip
 or batch, scale rows that start at every byte of a dword, split K, and more than one
 segment of staged scales (K past 4096 in one split).
 """
 import numpy as np
 import pytest
 
+import oracle
+import test_mx_gpu
 import triton_ext_amd as tx
-from dotcase import say, to_device
-from test_mx_gpu import check_mx, mx_case, ref_of, run_gpu
+from dotcase import bits_to_f32, from_device, say, to_device
+from test_mx_gpu import FMT, check_mx, mx_bf16_case, mx_case, ref_of, run_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +71,78 @@ def test_mx_decode_acc_and_repeat(gpu):
     torch.cuda.synchronize()
     assert torch.equal(c0.view(torch.int32), c1.view(torch.int32))
     assert torch.equal(got.view(torch.int32), (acc + c0).view(torch.int32))
+
+
+@pytest.mark.parametrize("fmt", ["e2m1", "e4m3", "e5m2"])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 250, 480), (16, 128, 256), (33, 272, 416), (64, 136, 512),
+                                   (80, 300, 288), (96, 256, 992), (97, 128, 256)])
+def test_mx_bf16_decode_small(gpu, fmt, out, M, N, K):
+    """One split on both sides: bit for bit the bf16 dot of the host upcast, and the oracle."""
+    p = _plan(M, N, K, tx.BF16, FMT_TX[fmt])
+    assert p.kernel == (tx.KERNEL_DECODE_MX_BF16 if M <= 96 else tx.KERNEL_GEMM_MX_BF16)
+    test_mx_gpu.test_mx_bf16_vs_oracle(gpu, "b", fmt, out, M, N, K)
+
+
+@pytest.mark.parametrize("fmt", ["e2m1", "e4m3", "e5m2"])
+def test_mx_bf16_decode_scale_range(gpu, fmt):
+    """Scales over [1, 239] (pair conversion and the fp32 path beside it): bit for bit the
+    bf16 dot of the host upcast; NaN scales make exactly their columns NaN."""
+    import torch
+    say(f"bf16 x {fmt} decode scale range")
+    M, N, K = 32, 272, 512
+    cs = mx_bf16_case(M, N, K, "b", fmt, seed=78 + len(fmt))
+    cs["s"] = np.random.default_rng(3).integers(1, 240, size=cs["s"].shape).astype(np.uint8)
+    cs["b16"] = test_mx_gpu.upcast_bf16(cs["codes"], cs["s"], fmt, "b")
+    bf = lambda x: to_device(x.view(np.int16), gpu).view(torch.bfloat16)
+    run = lambda s: from_device(tx.dot_scaled(bf(cs["a16"]), None, "bf16", to_device(cs["b"], gpu),
+                                              to_device(s, gpu), fmt))
+    got = run(cs["s"])
+    want = from_device(tx.dot(bf(cs["a16"]), bf(cs["b16"]), out_dtype=torch.float32))
+    assert np.array_equal(got.view(np.int32), want.view(np.int32))
+    s = cs["s"].copy()
+    s[1::2, 5] = 255
+    nan = np.isnan(run(s))
+    # (e5m2 terms reach 2^127: an even column's sum may itself be inf - inf)
+    assert nan[:, 1::2].all() and np.array_equal(nan[:, 0::2], np.isnan(got[:, 0::2]))
+
+
+@pytest.mark.parametrize("lhs,rhs,fmt", [("bf16", "e2m1", "mx"), ("bf16", "e4m3", "mx"),
+                                         ("bf16", "e2m1", "nv"), ("e2m1", "e2m1", "nv")])
+@pytest.mark.parametrize("M,N,K", [(3, 600, 8256), (40, 16640, 4352)])
+def test_wq_decode_split_and_segments(gpu, lhs, rhs, fmt, M, N, K):
+    """Split K, and one split of several scale segments; sampled columns against the oracle."""
+    import torch
+    nv = fmt == "nv"
+    p = _plan(M, N, K, FMT_TX.get(lhs, tx.BF16), FMT_TX[rhs], tx.SCALE_NV16 if nv else tx.SCALE_MX32)
+    assert p.kernel == tx.KERNEL_DECODE_MX_BF16 and (p.split_k > 1) == (N == 600)
+    say(f"wq decode {lhs}x{rhs} {fmt} {M}x{N}x{K} split={p.split_k}")
+    rng = np.random.default_rng(M + N)
+    grp, lo, hi = (16, 0x20, 0x50) if nv else (32, 117, 138)
+    bc = test_mx_gpu.codes(rng, (K, N), rhs)
+    sb = rng.integers(lo, hi, size=(N, K // grp)).astype(np.uint8)
+    b = test_mx_gpu.pack(bc, 0) if rhs == "e2m1" else bc
+    if lhs == "bf16":
+        a, sa = test_mx_gpu.upcast_bf16(rng.integers(0, 16, size=(M, K)).astype(np.uint8),
+                                        np.full((M, K // 32), 127, np.uint8), "e2m1", "a"), None
+        da = to_device(a.view(np.int16), gpu).view(torch.bfloat16)
+    else:
+        a = test_mx_gpu.pack(rng.integers(0, 16, size=(M, K)).astype(np.uint8), 1)
+        sa = rng.integers(lo, hi, size=(M, K // grp)).astype(np.uint8)
+        da = to_device(a, gpu)
+    e4 = lambda x: None if x is None else (to_device(x, gpu).view(torch.float8_e4m3fn) if nv
+                                           else to_device(x, gpu))
+    got = from_device(tx.dot_scaled(da, e4(sa), lhs, to_device(b, gpu), e4(sb), rhs))
+    cols = np.sort(rng.choice(N, 64, replace=False))
+    ref = oracle.dot_scaled(a, sa, FMT[lhs] if lhs != "bf16" else oracle.BF16,
+                            np.ascontiguousarray(b[:, cols]), np.ascontiguousarray(sb[cols]),
+                            FMT[rhs], K=K, nv16=nv)
+    k = np.arange(K) // grp
+    dec = (lambda s: torch.from_numpy(s).view(torch.float8_e4m3fn).double().numpy()) if nv else \
+        (lambda s: np.exp2(s.astype(np.float64) - 127))
+    bv = np.abs(oracle.mx_decode(bc[:, cols], FMT[rhs]) * dec(np.ascontiguousarray(sb[cols]))[:, k].T)
+    av = np.abs(bits_to_f32(a, "bf16").astype(np.float64)) if lhs == "bf16" else \
+        np.abs(oracle.mx_decode(np.stack([a & 15, a >> 4], 2).reshape(M, K), FMT[lhs]) * dec(sa)[:, k])
+    bound = K * 2.0 ** -24 * (av @ bv) + 1e-30
+    d = np.abs(got[:, cols].astype(np.float64) - ref)
+    assert (d <= bound).all(), f"worst d/bound {(d / bound).max():.3g}"

@@ -256,6 +256,17 @@ const Decode16KernelFn kDecode16WideKernels[2][2][kDec16WideMaxM / 16] = {
     {TX_D16W_SLICES(false, true), TX_D16W_SLICES(true, true)}};
 #undef TX_D16W_SLICES
 
+// The same with B upcast in registers, strips of 128 columns, slices of 16 ..
+// 96 rows: B e2m1 / e4m3 / e5m2 under e8m0 scales, e2m1 under e4m3 scales.
+#define TX_DWQ_SLICES(WQ)                                                                      \
+  {decode16_kernel<16, true, false, 128, WQ>, decode16_kernel<32, true, false, 128, WQ>,       \
+   decode16_kernel<48, true, false, 128, WQ>, decode16_kernel<64, true, false, 128, WQ>,       \
+   decode16_kernel<80, true, false, 128, WQ>, decode16_kernel<96, true, false, 128, WQ>}
+const Decode16KernelFn kDecodeWqKernels[4][kDec16MaxM / 16] = {
+    TX_DWQ_SLICES(WQ_MX_E2M1), TX_DWQ_SLICES(WQ_MX_E4M3), TX_DWQ_SLICES(WQ_MX_E5M2),
+    TX_DWQ_SLICES(WQ_NV_E2M1)};
+#undef TX_DWQ_SLICES
+
 // MFMA format code of an MX operand type (-1 if it has none).
 int mxFormat(int32_t t) {
   return t == TX_F8E4M3 ? 0 : t == TX_F8E5M2 ? 1 : t == TX_F4E2M1 ? 4 : -1;
@@ -493,6 +504,25 @@ int64_t decode16Workspace(const tx_dot_desc &d, int ksplit) {
          ksplit * decode16_split_bytes(decode16Strips(d), decode16Rows(d), (int)d.block_n);
 }
 
+// The 16-bit decode kernel with B upcast in registers (decode16.h, WQ): B in
+// an MX format or e2m1 with e4m3 scales, A bf16 (an e2m1 A under e4m3 scales
+// is upcast into the workspace first, M K elements), M <= 96, C bf16 or fp32.
+bool useDecodeWq(const tx_dot_desc &d) {
+  return (mxUpcastSide(d) == 2 || mxUpcastSide(d) == 3) && d.M <= kDec16MaxM &&
+         d.N <= kDec16MaxStrips * 128 && (d.c_type == TX_BF16 || d.c_type == TX_F32);
+}
+bool decodeWqTile(const tx_dot_desc &d) {
+  return d.block_m == decode16Rows(d) && d.block_n == 128 && d.block_k == kDec16BatchK;
+}
+// Bytes of an A upcast first, kept after the split-K partials.
+int64_t decodeWqUpcastA(const tx_dot_desc &d) {
+  return mxUpcastSide(d) == 3 ? (d.M * d.K * 2 + 255) / 256 * 256 : 0;
+}
+int64_t decodeWqWorkspace(const tx_dot_desc &d, int ksplit) {
+  const int64_t up = decodeWqUpcastA(d), sk = decode16Workspace(d, ksplit);
+  return up + (sk > 0 ? sk : up > 0 ? kDecodeCounterBytes : 0);
+}
+
 // The 8-bit ring decode kernel (decode_f8.h), B row-major or K-major: fp8 x
 // fp8 (e4m3 / e5m2 in any mix) with fp32 C; e4m3 x e4m3 with 128-block scales
 // and bf16 / fp32 C; with B K-major also int8 -> int32 and W8A8 at M <= 48
@@ -657,6 +687,17 @@ int txMi355xDotRun(tx_dot_plan *plan) {
     plan->passes_run += 1;
     return TX_OK;
   }
+  if (useDecodeWq(d) && decodeWqTile(d)) {
+    const int ks = decode16Split(d);
+    plan->kernel = TX_KERNEL_DECODE_MX_BF16;
+    plan->split_k = ks;
+    plan->grid_x = (int32_t)(decode16Strips(d) * ks);
+    plan->grid_y = plan->grid_z = 1;
+    plan->block_threads = kDecodeWaves * 64;
+    plan->workspace_bytes = decodeWqWorkspace(d, ks);
+    plan->passes_run += 1;
+    return TX_OK;
+  }
   if (useDecode(d) && decodeTile(d)) {
     const int ks = decodeSplit(d);
     plan->kernel = TX_KERNEL_DECODE_I8;
@@ -787,6 +828,7 @@ extern "C" TX_API const char *tx_kernel_name(int32_t kernel) {
   case TX_KERNEL_GEMM_MX: return "gemm_mx_mfma_scale16x16x128";
   case TX_KERNEL_GEMM_MX_BF16: return "mx_upcast_bf16+gemm_16bit_mfma32x32x16";
   case TX_KERNEL_DECODE_16BIT: return "decode_16bit_mfma16x16x32";
+  case TX_KERNEL_DECODE_MX_BF16: return "decode_mx_bf16_mfma16x16x32";
   case TX_KERNEL_DECODE_F8: return "decode_8bit_mfma16x16x128_f8f6f4|16x16x64_i8";
   default: return "?";
   }
@@ -946,6 +988,45 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
   return TX_OK;
 }
 
+// The upcast of one scaled operand (1: A, 2: B) to bf16 at `dst`.
+int launchUpcast(const tx_dot_desc &d, int one, const void *src, const void *scale, uint16_t *dst,
+                 hipStream_t stream) {
+  typedef void (*UpFn)(txk::UpcastArgs);
+  const bool nv = d.scale_mode == TX_SCALE_NV16;
+  const int fmt = mxFormat(one == 2 ? d.b_type : d.a_type);
+  txk::UpcastArgs u;
+  u.src = static_cast<const uint8_t *>(src);
+  u.scale = static_cast<const uint8_t *>(scale);
+  u.dst = dst;
+  u.ld_dst = one == 2 ? mxUpcastLdB(d) : d.K;
+  u.ld_scale = d.K / (nv ? 16 : 32);
+  u.fmt = fmt;
+  int64_t threads;
+  UpFn fn;
+  if (one == 2) {
+    u.rows = d.K;
+    u.cols = d.N;
+    u.ld_src = d.ldb; // fp8: bytes per row; e2m1: bytes per packed row
+    threads = (d.K / 8) * cdiv(d.N, 16); // 16 columns x 8 K rows per thread
+    fn = nv ? txk::mx_upcast_b_kernel<4, true>
+            : fmt == 0 ? txk::mx_upcast_b_kernel<0> : fmt == 1 ? txk::mx_upcast_b_kernel<1>
+                                                   : txk::mx_upcast_b_kernel<4>;
+  } else {
+    u.rows = d.M;
+    u.cols = d.K;
+    u.ld_src = fmt == 4 ? d.lda / 2 : d.lda;
+    threads = d.M * (d.K / 16);
+    fn = nv ? txk::mx_upcast_a_kernel<4, true>
+            : fmt == 0 ? txk::mx_upcast_a_kernel<0> : fmt == 1 ? txk::mx_upcast_a_kernel<1>
+                                                   : txk::mx_upcast_a_kernel<4>;
+  }
+  if (threads > 0) {
+    hipLaunchKernelGGL(fn, dim3((unsigned)cdiv(threads, 256)), dim3(256), 0, stream, u);
+    TX_HIP_CHECK(hipGetLastError());
+  }
+  return TX_OK;
+}
+
 // tl.dot_scaled through bf16: upcast the scaled operand(s) -- one side
 // against a bf16 operand (MX), or each e2m1 side under e4m3 scales (NV16) --
 // into the workspace (A's first, then B's), then the bf16 tile on them, all
@@ -955,7 +1036,6 @@ int launchMxUpcast(const tx_dot_plan &plan, const void *A, const void *B, void *
                    hipStream_t stream) {
   const tx_dot_desc &d = plan.desc;
   const int side = mxUpcastSide(d);
-  const bool nv = d.scale_mode == TX_SCALE_NV16;
   const int64_t need = mxUpcastWorkspace(d);
   if (!side)
     return fail(TX_ERR_INVALID, "plan has no operand to upcast");
@@ -969,48 +1049,13 @@ int launchMxUpcast(const tx_dot_plan &plan, const void *A, const void *B, void *
   uint16_t *wa = reinterpret_cast<uint16_t *>(up);
   uint16_t *wb = reinterpret_cast<uint16_t *>(
       up + ((side & 1) ? (d.M * d.K * 2 + 255) / 256 * 256 : 0));
-  typedef void (*UpFn)(txk::UpcastArgs);
-  auto upcast = [&](int one) -> int {
-    const int fmt = mxFormat(one == 2 ? d.b_type : d.a_type);
-    txk::UpcastArgs u;
-    u.src = static_cast<const uint8_t *>(one == 2 ? B : A);
-    u.scale = static_cast<const uint8_t *>(one == 2 ? sb : sa);
-    u.dst = one == 2 ? wb : wa;
-    u.ld_dst = one == 2 ? mxUpcastLdB(d) : d.K;
-    u.ld_scale = d.K / (nv ? 16 : 32);
-    u.fmt = fmt;
-    int64_t threads;
-    UpFn fn;
-    if (one == 2) {
-      u.rows = d.K;
-      u.cols = d.N;
-      u.ld_src = d.ldb; // fp8: bytes per row; e2m1: bytes per packed row
-      threads = (d.K / 8) * cdiv(d.N, 16); // 16 columns x 8 K rows per thread
-      fn = nv ? txk::mx_upcast_b_kernel<4, true>
-              : fmt == 0 ? txk::mx_upcast_b_kernel<0> : fmt == 1 ? txk::mx_upcast_b_kernel<1>
-                                                     : txk::mx_upcast_b_kernel<4>;
-    } else {
-      u.rows = d.M;
-      u.cols = d.K;
-      u.ld_src = fmt == 4 ? d.lda / 2 : d.lda;
-      threads = d.M * (d.K / 16);
-      fn = nv ? txk::mx_upcast_a_kernel<4, true>
-              : fmt == 0 ? txk::mx_upcast_a_kernel<0> : fmt == 1 ? txk::mx_upcast_a_kernel<1>
-                                                     : txk::mx_upcast_a_kernel<4>;
-    }
-    if (threads > 0) {
-      hipLaunchKernelGGL(fn, dim3((unsigned)cdiv(threads, 256)), dim3(256), 0, stream, u);
-      TX_HIP_CHECK(hipGetLastError());
-    }
-    return TX_OK;
-  };
   if (side & 1) {
-    const int rc = upcast(1);
+    const int rc = launchUpcast(d, 1, A, sa, wa, stream);
     if (rc != TX_OK)
       return rc;
   }
   if (side & 2) {
-    const int rc = upcast(2);
+    const int rc = launchUpcast(d, 2, B, sb, wb, stream);
     if (rc != TX_OK)
       return rc;
   }
@@ -1084,14 +1129,27 @@ int launchDecode(const tx_dot_plan &plan, const void *A, const void *B, void *C,
   return TX_OK;
 }
 
-int launchDecode16(const tx_dot_plan &plan, const void *A, const void *B, void *C, void *ws,
-                   size_t ws_bytes, hipStream_t stream) {
+// (and, with B's scales `sb`, the form that upcasts B in registers)
+int launchDecode16(const tx_dot_plan &plan, const void *A, const void *B, void *C, const void *sa,
+                   const void *sb, void *ws, size_t ws_bytes, hipStream_t stream) {
   const tx_dot_desc &d = plan.desc;
   const int ks = plan.split_k;
-  const int64_t need = decode16Workspace(d, ks);
+  const bool wq = plan.kernel == TX_KERNEL_DECODE_MX_BF16;
+  const int64_t need = wq ? decodeWqWorkspace(d, ks) : decode16Workspace(d, ks);
   if (need > 0 && (!ws || (int64_t)ws_bytes < need))
     return fail(TX_ERR_WORKSPACE, "decode needs %lld workspace bytes, got %zu",
                 (long long)need, ws_bytes);
+  const int64_t up_bytes = wq ? decodeWqUpcastA(d) : 0;
+  if (up_bytes > 0) { // A's upcast, after the counters and partials
+    if (reinterpret_cast<uintptr_t>(ws) & 15)
+      return fail(TX_ERR_INVALID, "workspace must be 16-byte aligned");
+    uint16_t *const wa =
+        reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(ws) + (need - up_bytes));
+    const int rc = launchUpcast(d, 1, A, sa, wa, stream);
+    if (rc != TX_OK)
+      return rc;
+    A = wa;
+  }
   Decode16Args a;
   a.A = static_cast<const uint16_t *>(A);
   a.B = static_cast<const uint16_t *>(B);
@@ -1101,9 +1159,11 @@ int launchDecode16(const tx_dot_plan &plan, const void *A, const void *B, void *
   a.M = (int32_t)d.M;
   a.N = (int32_t)d.N;
   a.K = (int32_t)d.K;
-  a.lda = d.lda;
-  a.ldb = d.ldb;
+  a.lda = up_bytes > 0 ? d.K : d.lda;
+  a.ldb = d.ldb; // (WQ: bytes of a code row)
   a.ldc = d.ldc;
+  a.sb = static_cast<const uint8_t *>(sb);
+  a.sb_ld = wq ? (int32_t)(d.K / (d.scale_mode == TX_SCALE_NV16 ? 16 : 32)) : 0;
   a.ksplit = ks;
   a.batches_per_split = (int32_t)cdiv(cdiv(d.K, kDec16BatchK), ks);
   a.k_main_batches = (int32_t)(plan.k_split / kDec16BatchK);
@@ -1113,7 +1173,12 @@ int launchDecode16(const tx_dot_plan &plan, const void *A, const void *B, void *
                         : nullptr;
   const int bt = (d.flags & TX_FLAG_B_KMAJOR) != 0, bf = d.a_type == TX_BF16,
             slice = decode16Rows(d) / 16 - 1;
-  const Decode16KernelFn fn = d.block_n == 128 ? kDecode16WideKernels[bt][bf][slice]
+  const int wqi = d.scale_mode == TX_SCALE_NV16 ? 3
+                  : d.b_type == TX_F4E2M1       ? 0
+                  : d.b_type == TX_F8E4M3       ? 1
+                                                : 2;
+  const Decode16KernelFn fn = wq               ? kDecodeWqKernels[wqi][slice]
+                              : d.block_n == 128 ? kDecode16WideKernels[bt][bf][slice]
                                                : kDecode16Kernels[bt][bf][slice];
   hipLaunchKernelGGL(fn, dim3(plan.grid_x), dim3(plan.block_threads), 0, stream, a);
   TX_HIP_CHECK(hipGetLastError());
@@ -1258,6 +1323,14 @@ int checkPlan(const tx_dot_plan &p) {
       return fail(TX_ERR_INVALID, "the plan's decode launch does not follow from its descriptor");
     return TX_OK;
   }
+  if (p.kernel == TX_KERNEL_DECODE_MX_BF16) {
+    const int sk = p.split_k;
+    if (!useDecodeWq(d) || !decodeWqTile(d) || sk < 1 || sk > (int)kMaxSplit ||
+        (sk & (sk - 1)) || p.grid_x != decode16Strips(d) * sk ||
+        p.block_threads != kDecodeWaves * 64 || p.workspace_bytes != decodeWqWorkspace(d, sk))
+      return fail(TX_ERR_INVALID, "the plan's decode launch does not follow from its descriptor");
+    return TX_OK;
+  }
   if (p.kernel == TX_KERNEL_DECODE_I8) {
     const int sk = p.split_k;
     if (!useDecode(d) || !decodeTile(d) || sk < 1 || sk > (int)kMaxSplit ||
@@ -1348,7 +1421,8 @@ int launchPlanned(const tx_dot_plan *plan, const void *A, const void *B, void *C
     return launchDecode(*plan, A, B, C, scale_a, scale_b, workspace,
                         workspace_bytes, s);
   case TX_KERNEL_DECODE_16BIT:
-    return launchDecode16(*plan, A, B, C, workspace, workspace_bytes, s);
+  case TX_KERNEL_DECODE_MX_BF16:
+    return launchDecode16(*plan, A, B, C, scale_a, scale_b, workspace, workspace_bytes, s);
   case TX_KERNEL_DECODE_F8:
     return launchDecodeF8(*plan, A, B, C, scale_a, scale_b, workspace, workspace_bytes, s);
   case TX_KERNEL_GEMM_MX_BF16:

@@ -63,13 +63,40 @@
 // wave w owns 16-column blocks 2 w and 2 w + 1 (the second block's B
 // fragments read in a block of their own); in K-major B, storage rows
 // 32 w .. 32 w + 31.
+//
+// WQ: B in a microscaled format with bf16 A (tl.dot_scaled's weight-only
+// form): e2m1 (packed rows [K/2][N]), e4m3 or e5m2 ([K][N]) with e8m0 scales
+// per 32 K, or e2m1 with e4m3 scales per 16 K, scales [N][K / 32 or 16].
+// Triton upcasts the scaled operand to bf16 and runs the bf16 dot; here each
+// wave upcasts its B fragments in registers on the way to the MFMA (W = 128
+// strips), so B is read once in its own bytes instead of being written to
+// memory and read back as bf16.  The K order of the MFMAs is the plain
+// kernel's, so the sums are those of the bf16 dot of the upcast operand.
+//  * B's batch is 128 K: 64 packed rows or 128 byte rows of 128 bytes, 16-byte
+//    chunk c of row r at c ^ swz(r).  ds_read_b64_tr_b8 hands a lane 8 rows of
+//    one column, and the 8 rows are the addressing lanes' choice: e2m1 takes
+//    rows 4 G .. +3 of two K steps at once (a step is 16 packed rows, one
+//    dword its 8 elements), fp8 rows 8 G .. +7 of one.
+//  * Upcast: v_cvt_scalef32_pk_bf16_* converts pairs under one scale where
+//    the scale exponent lies in [17, 239], where the product is exact; a batch
+//    with another scale in any of the wave's lanes decodes to fp32 pairs
+//    (exact, as is their ldexp short of overflow) and rounds once.  e4m3
+//    scales (not powers of two) multiply the fp32 pair; the product is exact
+//    in bf16.
+//  * Scales are staged per segment of 128 groups like decode_f8.h's MX form;
+//    columns past N and groups past K take a unit scale (their codes are 0).
 #pragma once
 
 #include <type_traits>
 
 #include "decode_i8.h"
+#include "mx_upcast.h"
 
 namespace txk {
+
+// B's format in the 16-bit decode kernel: A's type, or microscaled (WQ).
+enum { WQ_NONE = 0, WQ_MX_E2M1, WQ_MX_E4M3, WQ_MX_E5M2, WQ_NV_E2M1 };
+__device__ uint32_t tx_unit_scales[2] = {0x7f7f7f7fu, 0x38383838u}; // e8m0 2^0; e4m3 1.0
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 
@@ -92,6 +119,8 @@ struct Decode16Args {
   int32_t k_main_batches; // batches with every K row < K (unmasked)
   float *partials;        // [ksplit][strips][4 waves][SR / 16][64 lanes][4] fp32
   uint32_t *counters;     // [strips] arrival counters
+  const uint8_t *sb;      // WQ: scales [N][sb_ld]
+  int32_t sb_ld;
 };
 
 // Bytes of one split's partials: every strip's SR x W fp32 sums.
@@ -100,18 +129,31 @@ __host__ __device__ constexpr int64_t decode16_split_bytes(int64_t strips, int s
   return strips * sr * w * 4;
 }
 
-template <int SR, int W = kDec16StripN> struct Decode16Cfg {
+template <int SR, int W = kDec16StripN, int WQ = WQ_NONE> struct Decode16Cfg {
   static_assert(W == 64 || W == 128, "strips of 64 or 128 columns");
+  static constexpr bool FP4 = WQ == WQ_MX_E2M1 || WQ == WQ_NV_E2M1;
+  // WQ: scale groups a batch, batches a segment, scale bytes staged
+  static constexpr int GPB = WQ == WQ_NV_E2M1 ? 8 : 4, SEG_B = 128 / GPB;
+  static constexpr int WQS_BYTES = WQ ? W * 35 * 4 : 0;
   static constexpr int T = SR / 16;                         // 16-row tiles
   static constexpr int JB = W / 64;                         // 16-column blocks a wave
-  static constexpr int A_OFF = kDec16BatchK * 2 * W;        // B's batch first
+  static constexpr int A_OFF = FP4 ? kDec16BatchK / 2 * W : WQ ? kDec16BatchK * W
+                                                              : kDec16BatchK * 2 * W; // B's batch first
   static constexpr int SLOT = A_OFF + SR * kDec16BatchK * 2; // then SR rows of 256 bytes
-  static constexpr int S = 158 * 1024 / SLOT > 8 ? 8 : 158 * 1024 / SLOT;
-  static constexpr int B_LOADS = A_OFF / 1024 / kDecodeWaves;                  // 4
+  static constexpr int S_FIT = (158 * 1024 - WQS_BYTES) / SLOT;
+  static constexpr int S = S_FIT > 8 ? 8 : S_FIT;
+  static constexpr int B_LOADS = A_OFF / 1024 / kDecodeWaves;                  // 4 (W = 64)
   static constexpr int A_LOADS = SR * kDec16BatchK * 2 / 1024 / kDecodeWaves; // SR / 16
   static constexpr int VPB = B_LOADS + A_LOADS;
   static_assert(SR % 16 == 0 && SR >= 16 && SR <= kDec16MaxM, "slices of 16 .. 96 rows");
   static_assert(S >= 3 && (S - 2) * VPB <= 63, "ring depth; vmcnt is 6 bits");
+  static_assert(!WQ || (W == 128 && (S - 1) * VPB + (W * 35 + 255) / 256 <= 63),
+                "WQ: strips of 128 columns; vmcnt is 6 bits");
+  // WQ: the chunk swizzle of B's row r: distinct over the 8 rows of a
+  // transposed read (e2m1: rows r and r + 16 of 4 consecutive r)
+  __device__ __forceinline__ static int swz(int r) {
+    return FP4 ? (r & 3) | ((r >> 2) & 4) : r & 7;
+  }
 };
 
 // Operands of two K steps (32 rows each, KS and KS + 1) of a batch: the
@@ -291,12 +333,117 @@ __device__ __forceinline__ void dec16_read_bk_pair(uint32_t b0, uint32_t b1, i32
                : "memory");
 }
 
-template <int SR, bool BF, bool BT = false, int W = kDec16StripN>
+// WQ: the operands of two K steps: NB transposed reads of each of the wave's
+// two column blocks (e2m1: one, both steps' dwords; fp8: one a step, +4 KiB),
+// the blocks' staged scale dwords (three from an aligned address, of which
+// the batch's bytes are cut at the row's misalignment) and T row tiles of A.
+#define TX_DWQ_T(t, off)                                                                   \
+  "ds_read_b128 %[x0" #t "], %[a0] offset:" #off "\n\tds_read_b128 %[x1" #t "], %[a1] offset:" #off \
+  "\n\t"
+#define TX_DWQ_O(t) [x0##t] "=&v"(a[0][t]), [x1##t] "=&v"(a[1][t])
+#define TX_DWQ_H1                                                                          \
+  "ds_read_b64_tr_b8 %[y0], %[b0]\n\tds_read_b64_tr_b8 %[y1], %[b1]\n\t"
+#define TX_DWQ_H2                                                                          \
+  TX_DWQ_H1 "ds_read_b64_tr_b8 %[y2], %[b0] offset:4096\n\tds_read_b64_tr_b8 %[y3], %[b1] offset:4096\n\t"
+#define TX_DWQ_BO1 [y0] "=&v"(bq[0][0]), [y1] "=&v"(bq[1][0])
+#define TX_DWQ_BO2 TX_DWQ_BO1, [y2] "=&v"(bq[0][1]), [y3] "=&v"(bq[1][1])
+#define TX_DWQ_IN [b0] "v"(b0), [b1] "v"(b1), [a0] "v"(a0), [a1] "v"(a1)
+#define TX_DWQ_ASM(H, BO)                                                                  \
+  if constexpr (T == 1)                                                                    \
+    asm volatile(H TX_DWQ_T(0, 0) "s_waitcnt lgkmcnt(0)" : BO, TX_DWQ_O(0) : TX_DWQ_IN : "memory"); \
+  else if constexpr (T == 2)                                                               \
+    asm volatile(H TX_DWQ_T(0, 0) TX_DWQ_T(1, 4096) "s_waitcnt lgkmcnt(0)"                  \
+                 : BO, TX_DWQ_O(0), TX_DWQ_O(1)                                            \
+                 : TX_DWQ_IN                                                               \
+                 : "memory");                                                              \
+  else if constexpr (T == 3)                                                               \
+    asm volatile(H TX_DWQ_T(0, 0) TX_DWQ_T(1, 4096) TX_DWQ_T(2, 8192) "s_waitcnt lgkmcnt(0)" \
+                 : BO, TX_DWQ_O(0), TX_DWQ_O(1), TX_DWQ_O(2)                               \
+                 : TX_DWQ_IN                                                               \
+                 : "memory");                                                              \
+  else                                                                                     \
+    asm volatile(H TX_DWQ_T(0, 0) TX_DWQ_T(1, 4096) TX_DWQ_T(2, 8192) TX_DWQ_T(3, 12288)    \
+                 "s_waitcnt lgkmcnt(0)"                                                    \
+                 : BO, TX_DWQ_O(0), TX_DWQ_O(1), TX_DWQ_O(2), TX_DWQ_O(3)                   \
+                 : TX_DWQ_IN                                                               \
+                 : "memory")
+template <int T, int NB>
+__device__ __forceinline__ void decwq_read_pair(uint32_t b0, uint32_t b1, uint32_t a0, uint32_t a1,
+                                                v2i_t (&bq)[2][NB], i32x4_t (&a)[2][T]) {
+  if constexpr (NB == 1) {
+    TX_DWQ_ASM(TX_DWQ_H1, TX_DWQ_BO1);
+  } else {
+    TX_DWQ_ASM(TX_DWQ_H2, TX_DWQ_BO2);
+  }
+}
+#undef TX_DWQ_ASM
+#undef TX_DWQ_IN
+#undef TX_DWQ_BO2
+#undef TX_DWQ_BO1
+#undef TX_DWQ_H2
+#undef TX_DWQ_H1
+#undef TX_DWQ_O
+#undef TX_DWQ_T
+__device__ __forceinline__ void decwq_read_scales(uint32_t x0, uint32_t x1, uint32_t (&v)[2][3]) {
+  v2i_t p, q;
+  uint32_t r, t;
+  asm volatile("ds_read2_b32 %0, %4 offset0:0 offset1:1\n\tds_read2_b32 %1, %5 offset0:0 offset1:1\n\t"
+               "ds_read_b32 %2, %4 offset:8\n\tds_read_b32 %3, %5 offset:8\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(p), "=&v"(q), "=&v"(r), "=&v"(t)
+               : "v"(x0), "v"(x1)
+               : "memory");
+  v[0][0] = p.x, v[0][1] = p.y, v[0][2] = r;
+  v[1][0] = q.x, v[1][1] = q.y, v[1][2] = t;
+}
+
+// Elements 2 i and 2 i + 1 of 8 codes of a column (e2m1: a dword; fp8: two) in fp32.
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+template <int FMT, int I> __device__ __forceinline__ f32x2_t decwq_pair(uint32_t w0, uint32_t w1) {
+  if constexpr (FMT == 4)
+    return __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w0, 1.0f, I);
+  else if constexpr (FMT == 1)
+    return __builtin_amdgcn_cvt_scalef32_pk_f32_bf8(I < 2 ? w0 : w1, 1.0f, (I & 1) != 0);
+  else
+    return __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(I < 2 ? w0 : w1, 1.0f, (I & 1) != 0);
+}
+
+// One MFMA operand of B: 8 codes under one scale byte, as 8 bf16.  HW: the
+// scale lies in the pair conversion's exact range (MX).
+template <int WQ, bool HW>
+__device__ __forceinline__ i32x4_t decwq_upcast(uint32_t w0, uint32_t w1, uint32_t s) {
+  constexpr int FMT = WQ == WQ_MX_E4M3 ? 0 : WQ == WQ_MX_E5M2 ? 1 : 4;
+  if constexpr (WQ != WQ_NV_E2M1 && HW) {
+    const float f = __builtin_bit_cast(float, s << 23);
+    if constexpr (FMT == 4)
+      return i32x4_t{(int)mx_cvt_pair<4, 0>(w0, f), (int)mx_cvt_pair<4, 1>(w0, f),
+                     (int)mx_cvt_pair<4, 2>(w0, f), (int)mx_cvt_pair<4, 3>(w0, f)};
+    else
+      return i32x4_t{(int)mx_cvt_pair<FMT, 0>(w0, f), (int)mx_cvt_pair<FMT, 1>(w0, f),
+                     (int)mx_cvt_pair<FMT, 0>(w1, f), (int)mx_cvt_pair<FMT, 1>(w1, f)};
+  } else {
+    const float f = __builtin_amdgcn_cvt_f32_fp8((int)s, 0); // NV: the e4m3 scale
+    auto pair = [&](f32x2_t v) {
+      if constexpr (WQ == WQ_NV_E2M1)
+        return (int)pk_bf16_rne(v.x * f, v.y * f);
+      const float x = __builtin_amdgcn_ldexpf(v.x, (int)s - 127);
+      const float y = __builtin_amdgcn_ldexpf(v.y, (int)s - 127);
+      const float nan = __builtin_nanf("");
+      return (int)pk_bf16_rne(s == 255 ? nan : x, s == 255 ? nan : y);
+    };
+    return i32x4_t{pair(decwq_pair<FMT, 0>(w0, w1)), pair(decwq_pair<FMT, 1>(w0, w1)),
+                   pair(decwq_pair<FMT, 2>(w0, w1)), pair(decwq_pair<FMT, 3>(w0, w1))};
+  }
+}
+
+template <int SR, bool BF, bool BT = false, int W = kDec16StripN, int WQ = WQ_NONE>
 __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16Args p) {
-  typedef Decode16Cfg<SR, W> Cfg;
+  static_assert(!WQ || (BF && !BT && W == 128), "WQ: bf16 A, row-major B, strips of 128");
+  typedef Decode16Cfg<SR, W, WQ> Cfg;
   constexpr int S = Cfg::S, SLOT = Cfg::SLOT, T = Cfg::T, JB = Cfg::JB;
   __shared__ __attribute__((aligned(1024))) uint8_t ring[S * SLOT];
   __shared__ uint32_t last_flag;
+  __shared__ __attribute__((aligned(256))) uint8_t wqs[WQ ? (Cfg::WQS_BYTES + 255) / 256 * 256 : 4];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -344,7 +491,14 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
     for (int u = 0; u < Cfg::B_LOADS; ++u) {
       const int q = Cfg::B_LOADS * wave + u;
       const void *src;
-      if constexpr (BT) {
+      if constexpr (WQ != WQ_NONE) { // rows 8 q .. +7 of the batch's 64 or 128
+        const int row = 8 * q + (lane >> 3);
+        const int c = (lane & 7) ^ Cfg::swz(row);
+        const int64_t k = (Cfg::FP4 ? k0 / 2 : k0) + row, n = n0 + 16 * c;
+        src = reinterpret_cast<const uint8_t *>(p.B) + k * p.ldb + n;
+        if (mask && (!live || k >= (Cfg::FP4 ? p.K / 2 : p.K) || n >= p.N))
+          src = tx_zero_chunk;
+      } else if constexpr (BT) {
         const int r = 4 * q + (lane >> 4);
         const int c = (lane & 15) ^ (r & 15);
         const int64_t n = n0 + r, k = k0 + 8 * c;
@@ -409,17 +563,94 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
       bk_k[jj][ks] = (16 * (JB * wave + jj) + L) * 256 + (((4 * ks + G) ^ L) << 4);
   }
 
+  // WQ: a segment's scales of the strip's columns, `pitch` dwords a column from
+  // its first byte rounded down (decode_f8.h's MX form).
+  const int seg_groups = (nb < Cfg::SEG_B ? nb : Cfg::SEG_B) * Cfg::GPB;
+  const int pitch = WQ ? ((seg_groups + 3 + 3) / 4 + 1) | 1 : 1; // <= 35: the last read's third dword
+  auto stage_scales = [&](int i0) {
+    const int64_t g0 = (int64_t)(b_begin + i0) * Cfg::GPB;
+    const int items = W * pitch;
+    const int64_t bytes = ((int64_t)p.N * p.sb_ld + 3) & ~3ll;
+    for (int q0 = 64 * wave; q0 < items; q0 += 64 * kDecodeWaves) {
+      const int q = q0 + lane, r = q / pitch, dw = q - r * pitch;
+      const int64_t at = (((n0 + r) * p.sb_ld + g0) & ~3ll) + 4 * dw;
+      const void *src = p.sb + at;
+      // (whole dwords: each holds at least one byte of the array)
+      if (q >= items || n0 + r >= p.N || at >= bytes)
+        src = &tx_unit_scales[WQ == WQ_NV_E2M1];
+      __builtin_amdgcn_global_load_lds(src, (lds_void *)(wqs + 4 * q0), 4, 0, 0);
+    }
+  };
+  // This lane's column of each block: its staged row and misalignment, and its
+  // first transposed read (a K step pair is +4 KiB, fp8 +8 KiB).
+  uint32_t xs[2] = {0, 0}, mis[2] = {0, 0}, wq_b[2] = {0, 0};
+  if constexpr (WQ != WQ_NONE) {
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      const int J = 2 * wave + jj, r = L >> 1;
+      xs[jj] = lds_addr(wqs) + 4u * (uint32_t)((16 * J + L) * pitch);
+      mis[jj] = ((uint32_t)(n0 + 16 * J + L) * (uint32_t)p.sb_ld) & 3u; // (g0 is a multiple of 4)
+      const int row = Cfg::FP4 ? 4 * G + (r & 3) + 16 * (r >> 2) : 8 * G + r;
+      wq_b[jj] = row * 128 + ((J ^ Cfg::swz(row)) << 4) + 8 * (L & 1);
+    }
+  }
+
   auto consume = [&](const uint8_t *slot, int i) {
     const uint32_t base = lds_addr(slot);
     const int b = batch(i);
     const bool tail = b >= p.k_main_batches;
     const int64_t k0 = (int64_t)b * kDec16BatchK;
+    uint32_t sc[2][4]; // WQ: the scale byte of block jj at K step ks
+    bool soft = false;
+    if constexpr (WQ != WQ_NONE) {
+      uint32_t v[2][3];
+      const uint32_t at = (uint32_t)(i % Cfg::SEG_B) * Cfg::GPB;
+      decwq_read_scales(xs[0] + at, xs[1] + at, v);
+      bool odd = false;
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj) {
+        const uint32_t d0 = __builtin_amdgcn_alignbyte(v[jj][1], v[jj][0], mis[jj]);
+        const uint32_t d1 = __builtin_amdgcn_alignbyte(v[jj][2], v[jj][1], mis[jj]);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+          if constexpr (WQ == WQ_NV_E2M1) { // group 2 ks + G / 2 of the batch's 8
+            sc[jj][ks] = ((ks < 2 ? d0 : d1) >> (16 * (ks & 1) + 8 * (G >> 1))) & 0xff;
+            if (tail && b * Cfg::GPB + 2 * ks + (G >> 1) >= p.sb_ld)
+              sc[jj][ks] = 0x38;
+          } else {
+            sc[jj][ks] = (d0 >> (8 * ks)) & 0xff;
+            if (tail && b * Cfg::GPB + ks >= p.sb_ld)
+              sc[jj][ks] = 127;
+            odd = odd || sc[jj][ks] - kHwScaleLo > kHwScaleHi - kHwScaleLo;
+          }
+        }
+      }
+      if constexpr (WQ != WQ_NV_E2M1)
+        soft = __any(odd);
+    }
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
       constexpr int T4 = T < 4 ? T : 4; // tiles the first read block brings
       i32x4_t bq[JB][2];
       i32x4_t a4[2][T4];
-      if constexpr (BT) {
+      if constexpr (WQ != WQ_NONE) {
+        constexpr int NB = Cfg::FP4 ? 1 : 2;
+        v2i_t w[2][NB];
+        const uint32_t o = base + pr * (Cfg::FP4 ? 4096 : 8192);
+        decwq_read_pair<T4, NB>(o + wq_b[0], o + wq_b[1], base + a_k[2 * pr], base + a_k[2 * pr + 1],
+                                w, a4);
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint32_t w0 = Cfg::FP4 ? (h ? w[jj][0].y : w[jj][0].x) : w[jj][NB - 1 ? h : 0].x;
+            const uint32_t w1 = Cfg::FP4 ? 0 : w[jj][NB - 1 ? h : 0].y;
+            if (soft)
+              bq[jj][h] = decwq_upcast<WQ, false>(w0, w1, sc[jj][2 * pr + h]);
+            else
+              bq[jj][h] = decwq_upcast<WQ, true>(w0, w1, sc[jj][2 * pr + h]);
+          }
+      } else if constexpr (BT) {
         dec16_read_pair_kmajor<T4>(base + bk_k[0][2 * pr], base + bk_k[0][2 * pr + 1],
                                    base + a_k[2 * pr], base + a_k[2 * pr + 1], bq[0], a4);
         if constexpr (JB == 2)
@@ -458,7 +689,7 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj)
           bf[jj] = bq[jj][h];
-        if (tail) {
+        if (!WQ && tail) { // (WQ: K is a multiple of 16, no chunk of A crosses it)
           const int64_t k = k0 + 32 * (2 * pr + h) + 8 * G;
 #pragma unroll
           for (int t = 0; t < T; ++t)
@@ -478,7 +709,10 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
     }
   };
 
-  // Prologue: S - 1 batches in flight; batch i uses slot i % S.
+  // Prologue: S - 1 batches in flight; batch i uses slot i % S.  (WQ: the
+  // first segment's scales before them.)
+  if constexpr (WQ != WQ_NONE)
+    stage_scales(0);
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
     issue(s, ring + s * SLOT);
@@ -493,6 +727,13 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
       const int i = i0 + s;
       if (i >= nb)
         goto k_loop_done;
+      if constexpr (WQ != WQ_NONE) {
+        if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
+          asm volatile("s_barrier" ::: "memory");
+          stage_scales(i);
+          wait_vmcnt<0>();
+        }
+      }
       wait_vmcnt<(S - 2) * Cfg::VPB>();
       asm volatile("s_barrier" ::: "memory");
       issue(i + S - 1, ring + ((s + S - 1) % S) * SLOT);

@@ -249,8 +249,16 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
     const bool decode_mx = d->scale_mode == TX_SCALE_MX32 && !upcast && !kmajor && d->M <= 64 &&
                            d->N <= (int64_t)16384 * 128 &&
                            (d->c_type == TX_BF16 || d->c_type == TX_F32);
+    // The 16-bit decode kernel with B upcast in registers: bf16 A (or e2m1 A
+    // under e4m3 scales), B scaled, M <= 96; K of two batches or more.
+    const bool decode_wq = upcast && d->b_type != TX_BF16 &&
+                           (d->a_type == TX_BF16 || d->scale_mode == TX_SCALE_NV16) &&
+                           d->M <= 96 && d->K >= 256 && d->N <= (int64_t)16384 * 128 &&
+                           (d->c_type == TX_BF16 || d->c_type == TX_F32);
     const size_t first = spanA < TX_SPAN32_LIMIT && spanB < TX_SPAN32_LIMIT ? 0 : 1;
-    if (upcast)
+    if (decode_wq)
+      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 128, 1.0};
+    else if (upcast)
       t = chooseTile(kTiles16, d->M, d->N, d->K, kPeak16 / 2 / kCUs, first); // MX x bf16: bf16 tile
     else if (decode_mx)
       t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, ba == 4 ? 256 : 128, 1.0};
