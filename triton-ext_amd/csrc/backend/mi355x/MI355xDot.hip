@@ -22,20 +22,7 @@
 #include "triton_ext/tx_dot.h"
 #include "triton_ext/tx_passes.h"
 
-#include "attn_fwd.h"
-#include "attn_fwd8.h"
-#include "mx_upcast.h"
-
-#include "decode16.h"
-#include "decode_f8.h"
-#include "decode_i8.h"
-#include "decode_rows_i8.h"
-#include "gemm16_dma.h"
-#include "gemm8_w4.h"
-#include "splitk_reduce.h"
-#include "gemm8_n224.h"
-#include "gemm16_w4.h"
-#include "gemm_tile.h"
+#include "kernels.h"
 
 using namespace txk;
 
@@ -62,210 +49,6 @@ int fail(int code, const char *fmt, ...) {
   } while (0)
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// ---------------------------------------------------------------------------
-// Kernel table: every (operands, tile, epilogue) the backend instantiates.
-// ---------------------------------------------------------------------------
-
-typedef void (*GemmKernelFn)(GemmArgs);
-
-struct GemmConfig {
-  int op, bm, bn, bk, wm, wn, epi;
-  GemmKernelFn fn;
-  int bt;        // B K-major (TX_FLAG_B_KMAJOR)
-  int lds_bytes; // dynamic LDS (0 for kernels with static LDS)
-  int dma;       // 0: register-staged (gemm_tile.h), 1: direct-to-LDS
-                 // staging with 64-bit addresses (gemm16_dma.h), 2: 16-bit
-                 // 256x256 tile (gemm16_w4.h), 5: 8-bit 256x256x128 and
-                 // 256x224x128 tiles (gemm8_w4.h, gemm8_n224.h); 2 and 5
-                 // address A and B through 32-bit buffer offsets
-  int fmt;       // MX operand formats: MFMA code of A | code of B << 4
-};
-
-#define TX_GEMM(OP, BM, BN, BK, WM, WN, EPI)                                   \
-  GemmConfig {                                                                 \
-    OP, BM, BN, BK, WM, WN, EPI, gemm_tile_kernel<OP, BM, BN, BK, WM, WN, EPI>,\
-        0, GemmTile<OP, BM, BN, BK, WM, WN, EPI>::LDS_BYTES, 0                 \
-  }
-#define TX_GEMM_DMA_S(OP, BM, BN, BK, WM, WN, ST, EPI)                         \
-  GemmConfig {                                                                 \
-    OP, BM, BN, BK, WM, WN, EPI,                                               \
-        gemm16_dma_kernel<OP, BM, BN, BK, WM, WN, ST, EPI>, 0, 0, 1            \
-  }
-#define TX_GEMM_DMA(OP, BM, BN, BK, WM, WN, EPI)                               \
-  TX_GEMM_DMA_S(OP, BM, BN, BK, WM, WN, 2, EPI)
-
-#define TX_GEMM_W4(OP, EPI)                                                    \
-  GemmConfig { OP, 256, 256, 64, 2, 2, EPI, gemm16_w4_kernel<OP, EPI, 4>, 0, 0, 2 }
-#define TX_GEMM_W4T(OP, EPI)                                                   \
-  GemmConfig { OP, 256, 256, 64, 2, 2, EPI, gemm16_w4_kernel<OP, EPI, 4, true>, 1, 0, 2 }
-#define TX_GEMM_8(OP, EPI)                                                     \
-  GemmConfig { OP, 256, 256, 128, 2, 4, EPI, gemm8_w4_kernel<OP, EPI>, 0, 0, 5 }
-// MX (tl.dot_scaled) tiles: MFMA format codes FA, FB (0 e4m3, 1 e5m2,
-// 4 e2m1); BK in elements (128 bytes of K per step).
-#define TX_GEMM_MX(FA, FB, BK, EPI)                                            \
-  GemmConfig {                                                                 \
-    OP_F8, 256, 256, BK, 2, 4, EPI, gemm8_w4_kernel<OP_F8, EPI, FA, FB>, 0, 0, \
-        5, (FA) | ((FB) << 4)                                                  \
-  }
-// Unscaled fp8 with e5m2 operands (MFMA format codes FA, FB; fp32 C).
-#define TX_GEMM_8F(FA, FB)                                                     \
-  GemmConfig {                                                                 \
-    OP_F8, 256, 256, 128, 2, 4, EPI_F32, gemm8_w4_kernel<OP_F8, EPI_F32, FA, FB>, \
-        0, 0, 5, (FA) | ((FB) << 4)                                            \
-  }
-// The same with B K-major (TX_FLAG_B_KMAJOR): every 8-bit epilogue but MX's.
-#define TX_GEMM_8T(OP, EPI)                                                    \
-  GemmConfig { OP, 256, 256, 128, 2, 4, EPI, gemm8_w4_kernel<OP, EPI, 0, 0, true>, 1, 0, 5 }
-#define TX_GEMM_8FT(FA, FB)                                                    \
-  GemmConfig {                                                                 \
-    OP_F8, 256, 256, 128, 2, 4, EPI_F32, gemm8_w4_kernel<OP_F8, EPI_F32, FA, FB, true>, \
-        1, 0, 5, (FA) | ((FB) << 4)                                            \
-  }
-#define TX_GEMM_8N(OP, EPI)                                                    \
-  GemmConfig { OP, 256, 224, 128, 4, 2, EPI, gemm8_n224_kernel<OP, EPI>, 0, 0, 5 }
-
-// Every (operands, tile, epilogue) instantiated; findGemmConfig takes the
-// entry that matches a plan exactly.
-const GemmConfig kGemmConfigs[] = {
-    // bf16 / fp16 operands, 256x256x64 tiles of 4 waves
-    TX_GEMM_W4(OP_BF16, EPI_BF16),
-    TX_GEMM_W4(OP_BF16, EPI_F32),
-    TX_GEMM_W4(OP_F16, EPI_F32),
-    TX_GEMM_W4(OP_F16, EPI_F16),
-    // the same with B K-major (TX_FLAG_B_KMAJOR)
-    TX_GEMM_W4T(OP_BF16, EPI_BF16),
-    TX_GEMM_W4T(OP_BF16, EPI_F32),
-    TX_GEMM_W4T(OP_F16, EPI_F32),
-    TX_GEMM_W4T(OP_F16, EPI_F16),
-    // bf16 / fp16 operands, 128x128x64 tiles: direct-to-LDS staging, 64-bit
-    // addresses (operands spanning 2 GiB or more); two stages, two
-    // workgroups per CU (three or four stages leave one: 32.3 -> 25.6% of
-    // peak at bf16 4096^3)
-    TX_GEMM_DMA(OP_BF16, 128, 128, 64, 2, 2, EPI_BF16),
-    TX_GEMM_DMA(OP_BF16, 128, 128, 64, 2, 2, EPI_F32),
-    TX_GEMM_DMA(OP_F16, 128, 128, 64, 2, 2, EPI_F32),
-    TX_GEMM_DMA(OP_F16, 128, 128, 64, 2, 2, EPI_F16),
-    // 64x64x32 tiles (the reference's BLOCK of config 0): direct-to-LDS
-    // staging, three stages (measured at fp16 512^3: 2 / 3 / 4 / 5 stages
-    // 8.35 / 7.40 / 7.83 / 8.71 us; register staging 9.05 us)
-    TX_GEMM_DMA_S(OP_BF16, 64, 64, 32, 2, 2, 3, EPI_BF16),
-    TX_GEMM_DMA_S(OP_BF16, 64, 64, 32, 2, 2, 3, EPI_F32),
-    TX_GEMM_DMA_S(OP_F16, 64, 64, 32, 2, 2, 3, EPI_F32),
-    TX_GEMM_DMA_S(OP_F16, 64, 64, 32, 2, 2, 3, EPI_F16),
-    // int8 / fp8 operands, 256x256x128 tiles of 8 waves (gemm8_w4.h)
-    TX_GEMM_8(OP_I8, EPI_I32),
-    TX_GEMM_8(OP_I8, EPI_ROWCOL_BF16),
-    TX_GEMM_8(OP_F8, EPI_BLOCK128_BF16),
-    TX_GEMM_8(OP_F8, EPI_BLOCK128_F32),
-    TX_GEMM_8(OP_F8, EPI_F32),
-    // fp8 tt.dot with e5m2 on either side (the tutorial's p . v with fp8e5 p)
-    TX_GEMM_8F(1, 1),
-    TX_GEMM_8F(0, 1),
-    TX_GEMM_8F(1, 0),
-    // the same with B K-major (q . k^T, or weights kept [out][in])
-    TX_GEMM_8T(OP_I8, EPI_I32),
-    TX_GEMM_8T(OP_I8, EPI_ROWCOL_BF16),
-    TX_GEMM_8T(OP_F8, EPI_BLOCK128_BF16),
-    TX_GEMM_8T(OP_F8, EPI_BLOCK128_F32),
-    TX_GEMM_8T(OP_F8, EPI_F32),
-    TX_GEMM_8FT(1, 1),
-    TX_GEMM_8FT(0, 1),
-    TX_GEMM_8FT(1, 0),
-    // MX: e8m0-scaled fp8 (e4m3 / e5m2 in any mix) and fp4 (gemm8_w4.h)
-    TX_GEMM_MX(0, 0, 128, EPI_MX_F32),
-    TX_GEMM_MX(0, 0, 128, EPI_MX_BF16),
-    TX_GEMM_MX(0, 1, 128, EPI_MX_F32),
-    TX_GEMM_MX(0, 1, 128, EPI_MX_BF16),
-    TX_GEMM_MX(1, 0, 128, EPI_MX_F32),
-    TX_GEMM_MX(1, 0, 128, EPI_MX_BF16),
-    TX_GEMM_MX(1, 1, 128, EPI_MX_F32),
-    TX_GEMM_MX(1, 1, 128, EPI_MX_BF16),
-    TX_GEMM_MX(4, 4, 256, EPI_MX_F32),
-    TX_GEMM_MX(4, 4, 256, EPI_MX_BF16),
-    // the same with 256x224 tiles (gemm8_n224.h)
-    TX_GEMM_8N(OP_I8, EPI_I32),
-    TX_GEMM_8N(OP_I8, EPI_ROWCOL_BF16),
-    TX_GEMM_8N(OP_F8, EPI_BLOCK128_BF16),
-    TX_GEMM_8N(OP_F8, EPI_BLOCK128_F32),
-    TX_GEMM_8N(OP_F8, EPI_F32),
-    // int8 operands, int32 accumulation, 128x128x128 register-staged tiles
-    TX_GEMM(OP_I8, 128, 128, 128, 2, 2, EPI_I32),
-    TX_GEMM(OP_I8, 128, 128, 128, 2, 2, EPI_ROWCOL_BF16),
-    // fp8 e4m3 operands, fp32 accumulation, 128x128x128 register-staged tiles
-    TX_GEMM(OP_F8, 128, 128, 128, 2, 2, EPI_BLOCK128_BF16),
-    TX_GEMM(OP_F8, 128, 128, 128, 2, 2, EPI_BLOCK128_F32),
-    TX_GEMM(OP_F8, 128, 128, 128, 2, 2, EPI_F32),
-};
-constexpr int kNumGemmConfigs = sizeof(kGemmConfigs) / sizeof(kGemmConfigs[0]);
-
-typedef void (*DecodeKernelFn)(DecodeArgs);
-const DecodeKernelFn kDecodeKernels[4] = {decode_i8_kernel<1>, decode_i8_kernel<2>,
-                                           decode_i8_kernel<3>, decode_i8_kernel<4>};
-// The row-parallel decode kernel by slice height (64, 128, 256 rows): rings
-// of 6, 4 and 3 slots of 24, 32 and 48 KiB (a 128-row batch: B's 16 KiB and
-// the slice's A).
-// [B K-major][slice of 64, 128, 256 rows]
-const DecodeKernelFn kDecodeRowsKernels[2][3] = {
-    {decode_rows_i8_kernel<64, 6>, decode_rows_i8_kernel<128, 4>, decode_rows_i8_kernel<256, 3>},
-    {decode_rows_i8_kernel<64, 6, true>, decode_rows_i8_kernel<128, 4, true>,
-     decode_rows_i8_kernel<256, 3, true>}};
-// The 8-bit ring decode kernel: unscaled fp8 by [B K-major][A e4m3 / e5m2]
-// [B e4m3 / e5m2][slice of 16, 32, 48, 64 rows], block-scaled (e4m3) by
-// [B K-major][slice], int8 with B K-major (int32 C or W8A8) by slice.
-typedef void (*DecodeF8KernelFn)(DecodeF8Args);
-#define TX_DF8_SLICES(SC, FA, FB, BT, I8)                                                  \
-  {decode_f8_kernel<16, SC, FA, FB, BT, I8>, decode_f8_kernel<32, SC, FA, FB, BT, I8>,     \
-   decode_f8_kernel<48, SC, FA, FB, BT, I8>, decode_f8_kernel<64, SC, FA, FB, BT, I8>}
-const DecodeF8KernelFn kDecodeF8Kernels[2][2][2][4] = {
-    {{TX_DF8_SLICES(false, 0, 0, false, false), TX_DF8_SLICES(false, 0, 1, false, false)},
-     {TX_DF8_SLICES(false, 1, 0, false, false), TX_DF8_SLICES(false, 1, 1, false, false)}},
-    {{TX_DF8_SLICES(false, 0, 0, true, false), TX_DF8_SLICES(false, 0, 1, true, false)},
-     {TX_DF8_SLICES(false, 1, 0, true, false), TX_DF8_SLICES(false, 1, 1, true, false)}}};
-const DecodeF8KernelFn kDecodeF8ScaledKernels[2][4] = {TX_DF8_SLICES(true, 0, 0, false, false),
-                                                       TX_DF8_SLICES(true, 0, 0, true, false)};
-const DecodeF8KernelFn kDecodeI8KmajorKernels[4] = TX_DF8_SLICES(false, 0, 0, true, true);
-#undef TX_DF8_SLICES
-// MX operands: fp8 by [A e4m3 / e5m2][B e4m3 / e5m2][slice], and e2m1 by slice.
-#define TX_DMX_SLICES(FA, FB)                                                              \
-  {decode_f8_kernel<16, false, FA, FB, false, false, true>,                                \
-   decode_f8_kernel<32, false, FA, FB, false, false, true>,                                \
-   decode_f8_kernel<48, false, FA, FB, false, false, true>,                                \
-   decode_f8_kernel<64, false, FA, FB, false, false, true>}
-const DecodeF8KernelFn kDecodeMx8Kernels[2][2][4] = {
-    {TX_DMX_SLICES(0, 0), TX_DMX_SLICES(0, 1)}, {TX_DMX_SLICES(1, 0), TX_DMX_SLICES(1, 1)}};
-const DecodeF8KernelFn kDecodeMx4Kernels[4] = TX_DMX_SLICES(4, 4);
-#undef TX_DMX_SLICES
-// The 16-bit decode kernel by [B K-major][bf16][slice rows / 16 - 1], slices
-// of 16 .. 96 rows.
-typedef void (*Decode16KernelFn)(Decode16Args);
-#define TX_D16_SLICES(BF, BT)                                                                  \
-  {decode16_kernel<16, BF, BT>, decode16_kernel<32, BF, BT>, decode16_kernel<48, BF, BT>,      \
-   decode16_kernel<64, BF, BT>, decode16_kernel<80, BF, BT>, decode16_kernel<96, BF, BT>}
-const Decode16KernelFn kDecode16Kernels[2][2][kDec16MaxM / 16] = {
-    {TX_D16_SLICES(false, false), TX_D16_SLICES(true, false)},
-    {TX_D16_SLICES(false, true), TX_D16_SLICES(true, true)}};
-#undef TX_D16_SLICES
-// The same with strips of 128 columns, slices of 16 .. 80 rows.
-#define TX_D16W_SLICES(BF, BT)                                                                 \
-  {decode16_kernel<16, BF, BT, 128>, decode16_kernel<32, BF, BT, 128>,                         \
-   decode16_kernel<48, BF, BT, 128>, decode16_kernel<64, BF, BT, 128>,                         \
-   decode16_kernel<80, BF, BT, 128>}
-const Decode16KernelFn kDecode16WideKernels[2][2][kDec16WideMaxM / 16] = {
-    {TX_D16W_SLICES(false, false), TX_D16W_SLICES(true, false)},
-    {TX_D16W_SLICES(false, true), TX_D16W_SLICES(true, true)}};
-#undef TX_D16W_SLICES
-
-// The same with B upcast in registers, strips of 128 columns, slices of 16 ..
-// 96 rows: B e2m1 / e4m3 / e5m2 under e8m0 scales, e2m1 under e4m3 scales.
-#define TX_DWQ_SLICES(WQ)                                                                      \
-  {decode16_kernel<16, true, false, 128, WQ>, decode16_kernel<32, true, false, 128, WQ>,       \
-   decode16_kernel<48, true, false, 128, WQ>, decode16_kernel<64, true, false, 128, WQ>,       \
-   decode16_kernel<80, true, false, 128, WQ>, decode16_kernel<96, true, false, 128, WQ>}
-const Decode16KernelFn kDecodeWqKernels[4][kDec16MaxM / 16] = {
-    TX_DWQ_SLICES(WQ_MX_E2M1), TX_DWQ_SLICES(WQ_MX_E4M3), TX_DWQ_SLICES(WQ_MX_E5M2),
-    TX_DWQ_SLICES(WQ_NV_E2M1)};
-#undef TX_DWQ_SLICES
 
 // MFMA format code of an MX operand type (-1 if it has none).
 int mxFormat(int32_t t) {
@@ -972,7 +755,6 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
   r.ldp = splitLdp(d);
   r.M = (int32_t)d.M;
   r.N = (int32_t)d.N;
-  r.split_k = split;
   r.kind = d.c_type == TX_F32   ? txk::SPLIT_F32
            : d.c_type == TX_I32 ? txk::SPLIT_I32
            : d.c_type == TX_F16 ? txk::SPLIT_F16
@@ -981,7 +763,8 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
   r.acc = (d.flags & TX_FLAG_ACCUMULATE) != 0;
   const int64_t quads = d.M * cdiv(d.N, 4);
   if (quads > 0) {
-    hipLaunchKernelGGL(txk::splitk_reduce_kernel, dim3((unsigned)cdiv(quads, 256)), dim3(256), 0,
+    const SplitReduceFn fn = kSplitReduceKernels[split >= 16 ? 3 : split >= 8 ? 2 : split >= 4 ? 1 : 0];
+    hipLaunchKernelGGL(fn, dim3((unsigned)cdiv(quads, 256)), dim3(256), 0,
                        stream, r);
     TX_HIP_CHECK(hipGetLastError());
   }
@@ -991,7 +774,6 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
 // The upcast of one scaled operand (1: A, 2: B) to bf16 at `dst`.
 int launchUpcast(const tx_dot_desc &d, int one, const void *src, const void *scale, uint16_t *dst,
                  hipStream_t stream) {
-  typedef void (*UpFn)(txk::UpcastArgs);
   const bool nv = d.scale_mode == TX_SCALE_NV16;
   const int fmt = mxFormat(one == 2 ? d.b_type : d.a_type);
   txk::UpcastArgs u;
@@ -1002,24 +784,18 @@ int launchUpcast(const tx_dot_desc &d, int one, const void *src, const void *sca
   u.ld_scale = d.K / (nv ? 16 : 32);
   u.fmt = fmt;
   int64_t threads;
-  UpFn fn;
   if (one == 2) {
     u.rows = d.K;
     u.cols = d.N;
     u.ld_src = d.ldb; // fp8: bytes per row; e2m1: bytes per packed row
     threads = (d.K / 8) * cdiv(d.N, 16); // 16 columns x 8 K rows per thread
-    fn = nv ? txk::mx_upcast_b_kernel<4, true>
-            : fmt == 0 ? txk::mx_upcast_b_kernel<0> : fmt == 1 ? txk::mx_upcast_b_kernel<1>
-                                                   : txk::mx_upcast_b_kernel<4>;
   } else {
     u.rows = d.M;
     u.cols = d.K;
     u.ld_src = fmt == 4 ? d.lda / 2 : d.lda;
     threads = d.M * (d.K / 16);
-    fn = nv ? txk::mx_upcast_a_kernel<4, true>
-            : fmt == 0 ? txk::mx_upcast_a_kernel<0> : fmt == 1 ? txk::mx_upcast_a_kernel<1>
-                                                   : txk::mx_upcast_a_kernel<4>;
   }
+  const UpcastKernelFn fn = kUpcastKernels[one == 2][nv ? 3 : fmt == 4 ? 2 : fmt];
   if (threads > 0) {
     hipLaunchKernelGGL(fn, dim3((unsigned)cdiv(threads, 256)), dim3(256), 0, stream, u);
     TX_HIP_CHECK(hipGetLastError());
@@ -1581,29 +1357,6 @@ extern "C" TX_API int tx_attn_fwd_launch(const tx_attn_plan *plan, const void *q
   a.N_CTX = (int32_t)d.N_CTX;
   a.qk_scale = plan->qk_scale;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  typedef void (*AttnFn)(txk::AttnArgs);
-#define TX_ATTN_BLOCKS(C, HD, BF)                                                          \
-  {{txk::attn_fwd_kernel<C, HD, BF, 128, 64>, txk::attn_fwd_kernel<C, HD, BF, 128, 32>},    \
-   {txk::attn_fwd_kernel<C, HD, BF, 64, 64>, txk::attn_fwd_kernel<C, HD, BF, 64, 32>}}
-#define TX_ATTN_DTYPES(C, HD) {TX_ATTN_BLOCKS(C, HD, false), TX_ATTN_BLOCKS(C, HD, true)}
-  // [causal][head_dim 16 / 32 / 64 / 128 / 256][bf16][BLOCK_M 64][BLOCK_N 32]
-  static const AttnFn kAttn[2][5][2][2][2] = {
-      {TX_ATTN_DTYPES(false, 16), TX_ATTN_DTYPES(false, 32), TX_ATTN_DTYPES(false, 64),
-       TX_ATTN_DTYPES(false, 128), TX_ATTN_DTYPES(false, 256)},
-      {TX_ATTN_DTYPES(true, 16), TX_ATTN_DTYPES(true, 32), TX_ATTN_DTYPES(true, 64),
-       TX_ATTN_DTYPES(true, 128), TX_ATTN_DTYPES(true, 256)}};
-#undef TX_ATTN_DTYPES
-#undef TX_ATTN_BLOCKS
-  // [causal][head_dim 16 / 32 / 64 / 128 / 256][BLOCK_M 64][BLOCK_N 32]
-#define TX_ATTN8_BLOCKS(C, HD)                                                             \
-  {{txk::attn_fwd8_kernel<C, HD, 128, 64>, txk::attn_fwd8_kernel<C, HD, 128, 32>},          \
-   {txk::attn_fwd8_kernel<C, HD, 64, 64>, txk::attn_fwd8_kernel<C, HD, 64, 32>}}
-  static const AttnFn kAttn8[2][5][2][2] = {
-      {TX_ATTN8_BLOCKS(false, 16), TX_ATTN8_BLOCKS(false, 32), TX_ATTN8_BLOCKS(false, 64),
-       TX_ATTN8_BLOCKS(false, 128), TX_ATTN8_BLOCKS(false, 256)},
-      {TX_ATTN8_BLOCKS(true, 16), TX_ATTN8_BLOCKS(true, 32), TX_ATTN8_BLOCKS(true, 64),
-       TX_ATTN8_BLOCKS(true, 128), TX_ATTN8_BLOCKS(true, 256)}};
-#undef TX_ATTN8_BLOCKS
   const int c = d.causal ? 1 : 0;
   const int hd = d.head_dim == 16    ? 0
                  : d.head_dim == 32  ? 1

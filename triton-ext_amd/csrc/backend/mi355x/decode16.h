@@ -96,6 +96,7 @@ namespace txk {
 
 // B's format in the 16-bit decode kernel: A's type, or microscaled (WQ).
 enum { WQ_NONE = 0, WQ_MX_E2M1, WQ_MX_E4M3, WQ_MX_E5M2, WQ_NV_E2M1 };
+#define tx_unit_scales TX_TU_CAT(tx_unit_scales, TX_TU)
 __device__ uint32_t tx_unit_scales[2] = {0x7f7f7f7fu, 0x38383838u}; // e8m0 2^0; e4m3 1.0
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;

@@ -27,11 +27,14 @@ struct SplitReduceArgs {
   void *C;
   const float *sa, *sb; // SPLIT_ROWCOL: [M], [N]
   int64_t ldc, ldp;     // row strides in elements
-  int32_t M, N, split_k;
+  int32_t M, N;
   int32_t kind; // SplitEpilogue
   int32_t acc;  // SPLIT_F32 / SPLIT_I32: add to C's contents
 };
 
+// S: the number of ranges (2, 4, 8 or 16), so that a thread's loads are all in
+// flight before the first is added.
+template <int S>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(SplitReduceArgs p) {
   const int qn = (p.N + 3) / 4;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -42,9 +45,14 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(SplitReduceArgs p) {
   const bool whole = n + 4 <= p.N;
   if (p.kind == SPLIT_I32 || p.kind == SPLIT_ROWCOL) {
     const i32x4_t *src = reinterpret_cast<const i32x4_t *>(p.part) + off / 4;
-    i32x4_t s = src[0];
-    for (int z = 1; z < p.split_k; ++z)
-      s += src[z * (stride / 4)];
+    i32x4_t v[S];
+#pragma unroll
+    for (int z = 0; z < S; ++z)
+      v[z] = src[z * (stride / 4)];
+    i32x4_t s = v[0];
+#pragma unroll
+    for (int z = 1; z < S; ++z)
+      s += v[z];
     if (p.kind == SPLIT_I32) {
       int32_t *c = static_cast<int32_t *>(p.C) + (int64_t)m * p.ldc + n;
       if (whole) {
@@ -79,9 +87,14 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(SplitReduceArgs p) {
     return;
   }
   const f32x4_t *src = reinterpret_cast<const f32x4_t *>(p.part) + off / 4;
-  f32x4_t s = src[0];
-  for (int z = 1; z < p.split_k; ++z)
-    s += src[z * (stride / 4)];
+  f32x4_t v[S];
+#pragma unroll
+  for (int z = 0; z < S; ++z)
+    v[z] = src[z * (stride / 4)];
+  f32x4_t s = v[0];
+#pragma unroll
+  for (int z = 1; z < S; ++z)
+    s += v[z];
   if (p.kind == SPLIT_F32) {
     float *c = static_cast<float *>(p.C) + (int64_t)m * p.ldc + n;
     if (whole) {
