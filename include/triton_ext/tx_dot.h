@@ -146,6 +146,13 @@ typedef enum tx_kernel {
  * C's contents (int32 exactly; fp32 in one more rounding than an MFMA chain
  * seeded with C).  Not for the W8A8 decode path (bf16 C). */
 #define TX_FLAG_ACCUMULATE 0x4
+/* A 256x256 tile plan runs on 128x128 tiles (a deep LDS ring, one workgroup a
+ * CU), which fill the chip where the 256x256 tiles would leave CUs idle.  The
+ * planner sets it in plan->desc.flags when it chooses the tile (block 0); with
+ * an explicit block it takes the 256x256 tiles only.  The plan's fields stay
+ * those of its 256x256 tiles; split_k is then the most K ranges a launch
+ * makes (fewer when the 128x128 tiles alone fill the CUs). */
+#define TX_FLAG_TILES_128 0x100
 
 typedef struct tx_dot_desc {
   int64_t M, N, K;

@@ -123,6 +123,8 @@ TX_API int tx_dot_operand_spans(const tx_dot_desc *desc, int64_t *a_bytes, int64
  * largest power of two up to 16 with tiles * S <= 256 and at least 8 K steps
  * a range; 1 (no split) otherwise. */
 TX_API int32_t tx_gemm_split_k(int64_t tiles, int64_t ksteps);
+/* The same for the 128x128 tiles of TX_FLAG_TILES_128. */
+TX_API int32_t tx_ring_split_k(int64_t tiles128, int64_t ksteps);
 /* Row stride (elements) of a B operand that tl.dot_scaled with one bf16 side
  * upcasts to bf16 in the workspace: N rounded up to 16 columns, so every row
  * starts 16-byte aligned for the bf16 tile.  (An upcast A is packed: K.) */

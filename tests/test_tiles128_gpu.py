@@ -1,0 +1,142 @@
+"""GPU parity of the 128x128 ring tiles (TX_FLAG_TILES_128, gemm_ring.h): every operand kind
+and layout at tile edges, K tails of one byte to a whole step, split K and a single step,
+against the 256x256 tiles the same plan names without the flag (explicit block).
+
+int8 sums are exact and must be equal.  The others add the same products in fp32, in K order
+within a range (16-bit, fp8: one MFMA chain per range; block-scaled: one fma per 128 K), so
+two results differ by at most the rounding of the sums: (K / 16 + 8) 2^-23 sum |a b| here,
+plus one ulp of a 16-bit C.
+"""
+import numpy as np
+import pytest
+
+import triton_ext_amd as tx
+from dotcase import say
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(97, 128, 512), (129, 257, 2049), (300, 131, 4100), (128, 640, 64), (513, 1000, 1111)]
+
+
+def _padded(torch, x, junk):
+    """x in rows 16 bytes apart, the padding and the row after the last full of `junk`."""
+    es = x.element_size()
+    ld = (x.shape[1] * es + 15) // 16 * 16 // es + 16 // es
+    buf = torch.empty((x.shape[0] + 1, ld), dtype=x.dtype, device=x.device)
+    buf.view(torch.uint8).fill_(junk)
+    buf[:x.shape[0], :x.shape[1]] = x
+    return buf[:x.shape[0], :x.shape[1]]
+
+
+def _both(dot, desc_args, flags=0):
+    """The dot on the plan with TX_FLAG_TILES_128 and on the 256x256 tiles."""
+    out = []
+    for f in (tx.FLAG_TILES_128, 0):
+        p = tx.plan(tx.make_desc(flags=flags | f, **desc_args))
+        assert (p.desc.block_m, p.desc.block_n) == (256, 256)
+        assert bool(p.desc.flags & tx.FLAG_TILES_128) == bool(f)
+        out.append(dot(p))
+    return out
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("kind", ["bf16", "f16_f32", "int8", "w8a8", "fp8", "fp8_mix", "fp8b",
+                                  "fp8b_f32"])
+@pytest.mark.parametrize("kmajor", [False, True])
+def test_tiles128_vs_256(gpu, kind, kmajor, M, N, K):
+    import torch
+    say(f"tiles128 {kind} kmajor={kmajor} {M}x{N}x{K}")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(M + N + K)
+    a, b = (torch.randn(s, generator=g, device=gpu) for s in ((M, K), (N, K) if kmajor else (K, N)))
+    sa = sb = None
+    mode, out, junk = tx.SCALE_NONE, torch.float32, 0x7F
+    if kind in ("bf16", "f16_f32"):
+        t = torch.bfloat16 if kind == "bf16" else torch.float16
+        out = torch.bfloat16 if kind == "bf16" else torch.float32
+        a, b, junk = a.to(t), b.to(t), 0xFF
+    elif kind in ("int8", "w8a8"):
+        a, b = (torch.round(x * 40).clamp(-127, 127).to(torch.int8) for x in (a, b))
+        out = torch.int32 if kind == "int8" else torch.bfloat16
+        if kind == "w8a8":
+            mode, sa, sb = tx.SCALE_ROWCOL, torch.rand(M, device=gpu), torch.rand(N, device=gpu)
+    else:
+        a = a.to(torch.float8_e4m3fn)
+        b = b.to(torch.float8_e5m2 if kind == "fp8_mix" else torch.float8_e4m3fn)
+        if kind in ("fp8b", "fp8b_f32"):
+            mode, out = tx.SCALE_BLOCK128, torch.bfloat16 if kind == "fp8b" else torch.float32
+            kb = -(-K // 128)
+            sa = torch.rand((M, kb), device=gpu) + 0.5
+            sb = torch.rand((kb, -(-N // 128)), device=gpu) + 0.5
+    a, b = _padded(torch, a, junk), _padded(torch, b, junk)
+    c = tx.new_output(M, N, out, gpu)
+    bv = b.t() if kmajor else b
+    desc = dict(M=M, N=N, K=K, a_type=tx.tx_type(a), b_type=tx.tx_type(b), c_type=tx.tx_type(c),
+                scale_mode=mode, block=(256, 256, 64 if a.element_size() == 2 else 128),
+                lda=a.stride(0), ldb=b.stride(0), ldc=c.stride(0))
+
+    def run(p):
+        r = tx.new_output(M, N, out, gpu)
+        tx.dot(a, bv, out=r, scale_a=sa, scale_b=sb, plan=p)
+        return r.clone()
+    got, want = _both(run, desc, tx.FLAG_B_KMAJOR if kmajor else 0)
+    torch.cuda.synchronize()
+    if kind in ("int8", "w8a8"):
+        assert torch.equal(got, want)
+        return
+    f = lambda x: x.to(torch.float32).double().abs()
+    if mode == tx.SCALE_BLOCK128:
+        S = (f(a) * sa.double().repeat_interleave(128, 1)[:, :K]) @ \
+            (f(bv) * sb.double().repeat_interleave(128, 0)[:K].repeat_interleave(128, 1)[:, :N])
+    else:
+        S = f(a) @ f(bv)
+    bound = (K / 16 + 8) * 2.0 ** -23 * S + 1e-30
+    if out == torch.bfloat16:
+        bound = bound + 2.0 ** -7 * f(want)
+    d = (got.double() - want.double()).abs()
+    assert torch.isfinite(got.double()).all() and (d <= bound).all(), float((d / bound).max())
+
+
+@pytest.mark.parametrize("M,N,K", [(97, 128, 512), (129, 257, 2080), (300, 131, 4128), (128, 640, 64)])
+@pytest.mark.parametrize("fa,fb", [("e4m3", "e4m3"), ("e5m2", "e4m3"), ("e2m1", "e2m1")])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+def test_tiles128_mx(gpu, fa, fb, out, M, N, K):
+    """The planner's choice at these sizes is the ring tile; against the oracle."""
+    from test_decode_mx_gpu import FMT_TX
+    from test_mx_gpu import check_mx, mx_case, ref_of, run_gpu
+    r = lambda x, q: -(-x // q) * q
+    p = tx.plan(tx.make_desc(M, N, K, FMT_TX[fa], tx.F32, b_type=FMT_TX[fb], lda=r(K, 32),
+                             ldb=r(N, 16), ldc=r(N, 4), scale_mode=tx.SCALE_MX32))
+    assert p.kernel == tx.KERNEL_GEMM_MX and p.desc.flags & tx.FLAG_TILES_128
+    assert (p.split_k > 1) == (K >= 4096 or (K > 2048 and fa != "e2m1"))
+    say(f"tiles128 mx {fa}x{fb} {out} {M}x{N}x{K} split={p.split_k}")
+    cs = mx_case(M, N, K, fa, fb, seed=M + N + K)
+    check_mx(run_gpu(gpu, cs, out), ref_of(cs, out), cs, out, f"tiles128 mx {out}")
+
+
+def test_tiles128_acc_noalloc_and_repeat(gpu):
+    """acc + dot is the dot plus acc in one fp32 addition, split and whole; launches repeat
+    bit for bit; the no-allocation launch gives the same bits."""
+    import ctypes
+
+    import torch
+    say("tiles128 acc / noalloc")
+    for M, N, K in ((200, 300, 4096), (700, 900, 512)):
+        a = torch.randn((M, K), device=gpu).bfloat16()
+        b = torch.randn((K, N), device=gpu).bfloat16()
+        b = tx.aligned_rows(b)
+        p = tx.plan_for(a, b, tx.F32, ldc=-(-N // 4) * 4)
+        assert p.desc.flags & tx.FLAG_TILES_128 and (p.split_k > 1) == (K == 4096)
+        c0, c1 = (tx.dot(a, b, out_dtype=torch.float32) for _ in range(2))
+        acc = torch.randn((M, N), device=gpu)
+        got = tx.dot(a, b, acc=acc)
+        c2 = tx.new_output(M, N, torch.float32, gpu)
+        tx.check(tx.load().tx_dot_launch_noalloc(ctypes.byref(p), a.data_ptr(), b.data_ptr(),
+                                                 c2.data_ptr(), None, None,
+                                                 torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert torch.equal(c0.view(torch.int32), c1.view(torch.int32))
+        assert torch.equal(c0, c2) and torch.equal(got, acc + c0)
+        want = a.double() @ b.double()
+        assert ((c0.double() - want).abs() <= 1e-5 * (a.double().abs() @ b.double().abs())).all()
+        assert np.isfinite(c0.sum().item())

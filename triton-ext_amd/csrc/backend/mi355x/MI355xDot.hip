@@ -173,6 +173,16 @@ int findGemmConfig(int op, int epi, int bm, int bn, int bk, bool bt, int fmt) {
   return -1;
 }
 
+// The 128x128 ring tile of a dot planned with TX_FLAG_TILES_128 (NULL: none).
+const GemmConfig *findRing(int op, int epi, bool bt, int fmt) {
+  for (int i = 0; i < kNumRingConfigs; ++i) {
+    const GemmConfig &c = kRingConfigs[i];
+    if (c.op == op && c.epi == epi && c.bt == (int)bt && c.fmt == fmt)
+      return &c;
+  }
+  return nullptr;
+}
+
 // Decode row tiling: slices of 16 * MT rows (MT = ceil(M / 16) up to 4), one
 // slice up to M = 64 and slices of 64 beyond.  Slices multiply the B bytes a
 // workgroup streams (fewer splits), so they are used only once M outgrows one
@@ -371,10 +381,22 @@ int partialEpi(const tx_dot_desc &d, int op) {
     return EPI_I32;
   if (op == OP_F8 && d.scale_mode == TX_SCALE_BLOCK128)
     return EPI_BLOCK128_F32;
+  if (d.scale_mode == TX_SCALE_MX32)
+    return EPI_MX_F32;
   return EPI_F32;
+}
+// K ranges of a dot on the 128x128 ring tiles (TX_FLAG_TILES_128): at most the
+// plan's split_k, whose partials the workspace holds.
+bool ringPlan(const tx_dot_desc &d) { return (d.flags & TX_FLAG_TILES_128) != 0; }
+int ringSplit(const tx_dot_desc &d) {
+  return (d.flags & TX_FLAG_NO_LOOP_SPLIT)
+             ? 1
+             : tx_ring_split_k(cdiv(d.M, 128) * cdiv(d.N, 128), cdiv(d.K, d.block_k));
 }
 // d: the dot the tile runs (for the MX x bf16 upcast, its bf16 dot: bfDot).
 int gemmSplit(const tx_dot_desc &d, int op, int64_t tiles) {
+  if (ringPlan(d) && d.scale_mode == TX_SCALE_MX32)
+    return ringSplit(d); // (the 256x256 MX tiles themselves run unsplit)
   if (d.block_m != 256 || d.block_n != 256 || d.scale_mode == TX_SCALE_MX32 ||
       d.scale_mode == TX_SCALE_NV16 || (d.flags & TX_FLAG_NO_LOOP_SPLIT) ||
       findGemmConfig(op, partialEpi(d, op), d.block_m, d.block_n, d.block_k,
@@ -409,7 +431,8 @@ int64_t gemmWorkspace(const tx_dot_desc &d, int split) {
 // 2^31 bytes (out-of-range chunks, at offset 2^31, read zeros).
 int checkSpans32(const tx_dot_desc &d, const GemmConfig &c) {
   if (c.dma != 2 && c.dma != 5)
-    return TX_OK;
+    return ringPlan(d) ? fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128 takes the 256x256 tiles")
+                       : TX_OK;
   tx_dot_desc e = d; // the operands as the tile reads them
   if (mxUpcastSide(d) & 1)
     e.a_type = TX_BF16, e.lda = d.K;
@@ -425,6 +448,14 @@ int checkSpans32(const tx_dot_desc &d, const GemmConfig &c) {
                 "the %dx%d tile addresses operands through 32-bit offsets: A spans %lld "
                 "bytes, B %lld (limit 2^31); a 128x128 tile takes larger operands",
                 c.bm, c.bn, (long long)sa, (long long)sb);
+  if (ringPlan(d) && (c.bm != 256 || c.bn != 256))
+    return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128 takes the 256x256 tiles");
+  if (ringPlan(d) && cdiv(d.M, 128) * cdiv(d.N, 128) > INT32_MAX)
+    return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128: a grid above 2^31 tiles");
+  // (the ring tile also forms the offsets of up to 127 rows of B past K)
+  if (ringPlan(d) && !(d.flags & TX_FLAG_B_KMAJOR) &&
+      (e.K + 128) * e.ldb * (tx_dtype_bits(e.b_type) == 16 ? 2 : 1) >= ((int64_t)1 << 32))
+    return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128: 128 rows of B past K end beyond 2^32 bytes");
   return TX_OK;
 }
 
@@ -564,7 +595,8 @@ int validate(const tx_dot_desc *in, tx_dot_desc *d) {
   if (d->ldc == 0) d->ldc = d->N;
   if (d->lda < d->K || d->ldb < (bt ? d->K : d->N) || d->ldc < d->N)
     return fail(TX_ERR_INVALID, "row stride shorter than the row");
-  if (d->flags & ~(TX_FLAG_NO_LOOP_SPLIT | TX_FLAG_B_KMAJOR | TX_FLAG_ACCUMULATE))
+  if (d->flags & ~(TX_FLAG_NO_LOOP_SPLIT | TX_FLAG_B_KMAJOR | TX_FLAG_ACCUMULATE |
+                   TX_FLAG_TILES_128))
     return fail(TX_ERR_INVALID, "unknown flags 0x%x", d->flags);
   if ((d->flags & TX_FLAG_ACCUMULATE) && d->c_type != TX_F32 && d->c_type != TX_I32)
     return fail(TX_ERR_UNSUPPORTED, "accumulating into C needs an fp32 or int32 C");
@@ -662,12 +694,18 @@ extern "C" TX_API int tx_dot_plan_create(const tx_dot_desc *desc,
 
 namespace {
 
+struct KernelShape {
+  GemmKernelFn fn;
+  unsigned grid, threads;
+};
+
 int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
                const void *sa, const void *sb, void *ws, size_t ws_bytes, hipStream_t stream) {
   const tx_dot_desc &d = plan.desc;
   int op, epi;
   classify(d, &op, &epi);
-  const int split = plan.split_k > 1 ? plan.split_k : 1;
+  const bool ring = ringPlan(d);
+  int split = plan.split_k > 1 ? plan.split_k : 1;
   // split-K: the tile kernel with the 32-bit partial epilogue, then the reduction
   const int ci = findGemmConfig(op, split > 1 ? partialEpi(d, op) : epi, d.block_m, d.block_n,
                                 d.block_k, (d.flags & TX_FLAG_B_KMAJOR) != 0, fmtOf(d));
@@ -678,6 +716,15 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
       plan.n_tiles <= 0 || plan.block_threads != c.wm * c.wn * 64 ||
       plan.grid_y != split)
     return fail(TX_ERR_INVALID, "plan launch shape does not match its tile");
+  if (ring && split > ringSplit(d))
+    split = ringSplit(d);
+  const GemmConfig *rc = nullptr;
+  if (ring) {
+    rc = findRing(op, split > 1 ? partialEpi(d, op) : epi, (d.flags & TX_FLAG_B_KMAJOR) != 0,
+                  fmtOf(d));
+    if (!rc)
+      return fail(TX_ERR_UNSUPPORTED, "plan names a tile that is not instantiated");
+  }
   const int64_t need = gemmSplitWorkspace(d, split);
   if (need > 0 && (!ws || (int64_t)ws_bytes < need))
     return fail(TX_ERR_WORKSPACE, "split-K needs %lld workspace bytes, got %zu", (long long)need,
@@ -724,12 +771,20 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
     a.last_ks = d.block_k / km;
   const int gm = plan.group_m > 0 ? plan.group_m : 1;
   a.group_m = plan.m_tiles < gm ? plan.m_tiles : gm;
+  const KernelShape k = ring ? KernelShape{rc->fn, (unsigned)(cdiv(d.M, 128) * cdiv(d.N, 128)),
+                                           (unsigned)(rc->wm * rc->wn * 64)}
+                             : KernelShape{c.fn, (unsigned)plan.grid_x,
+                                           (unsigned)plan.block_threads};
+  if (ring) {
+    a.tiles_m = (int32_t)cdiv(d.M, 128);
+    a.tiles_n = (int32_t)cdiv(d.N, 128);
+    a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
+  }
   a.sa_ld = (int32_t)(mx ? d.K / 32 : cdiv(d.K, 128));
   a.sb_ld = (int32_t)cdiv(d.N, 128);
   a.accumulate = (d.flags & TX_FLAG_ACCUMULATE) != 0;
   if (split == 1) {
-    hipLaunchKernelGGL(c.fn, dim3(plan.grid_x), dim3(plan.block_threads),
-                       c.lds_bytes, stream, a);
+    hipLaunchKernelGGL(k.fn, dim3(k.grid), dim3(k.threads), c.lds_bytes, stream, a);
     TX_HIP_CHECK(hipGetLastError());
     return TX_OK;
   }
@@ -739,12 +794,12 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
   const int ksteps = (int)cdiv(d.K, d.block_k);
   a.split_k = split;
   a.split_steps = ksteps / split;
-  a.k_main_steps -= (split - 1) * a.split_steps;
+  if (!ring) // (the ring tile takes its range by absolute steps)
+    a.k_main_steps -= (split - 1) * a.split_steps;
   a.C = part;
   a.ldc = splitLdp(d);
   a.accumulate = 0;
-  hipLaunchKernelGGL(c.fn, dim3(plan.grid_x, split), dim3(plan.block_threads), c.lds_bytes,
-                     stream, a);
+  hipLaunchKernelGGL(k.fn, dim3(k.grid, split), dim3(k.threads), c.lds_bytes, stream, a);
   TX_HIP_CHECK(hipGetLastError());
   txk::SplitReduceArgs r;
   r.part = part;
@@ -1075,7 +1130,8 @@ int checkPlan(const tx_dot_plan &p) {
       p.m_tiles != cdiv(d.M, d.block_m) || p.n_tiles != cdiv(d.N, d.block_n) ||
       p.m_edge != d.M % d.block_m || p.n_edge != d.N % d.block_n || p.grid_z != 1 ||
       (p.grid_y != 1 && p.kernel != TX_KERNEL_GEMM_16BIT && p.kernel != TX_KERNEL_GEMM_I8 &&
-       p.kernel != TX_KERNEL_GEMM_F8 && p.kernel != TX_KERNEL_GEMM_MX_BF16))
+       p.kernel != TX_KERNEL_GEMM_F8 && p.kernel != TX_KERNEL_GEMM_MX_BF16 &&
+       p.kernel != TX_KERNEL_GEMM_MX))
     // (the tiles' split-K ranges, checked below)
     return fail(TX_ERR_INVALID, "the plan's loop split or tile grid does not follow from its "
                 "descriptor");
@@ -1164,7 +1220,8 @@ int launchPlanned(const tx_dot_plan *plan, const void *A, const void *B, void *C
   if (noalloc && plan->split_k > 1 && plan->grid_y == plan->split_k &&
       plan->workspace_bytes > (int64_t)TX_NOALLOC_SCRATCH_BYTES &&
       (plan->kernel == TX_KERNEL_GEMM_16BIT || plan->kernel == TX_KERNEL_GEMM_I8 ||
-       plan->kernel == TX_KERNEL_GEMM_F8 || plan->kernel == TX_KERNEL_GEMM_MX_BF16)) {
+       plan->kernel == TX_KERNEL_GEMM_F8 || plan->kernel == TX_KERNEL_GEMM_MX_BF16 ||
+       plan->kernel == TX_KERNEL_GEMM_MX)) {
     unsplit = *plan;
     unsplit.split_k = 1;
     unsplit.grid_y = 1;

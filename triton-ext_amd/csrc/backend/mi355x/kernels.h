@@ -15,6 +15,7 @@
 #include "gemm16_w4.h"
 #include "gemm8_n224.h"
 #include "gemm8_w4.h"
+#include "gemm_ring.h"
 #include "gemm_tile.h"
 #include "mx_upcast.h"
 #include "splitk_reduce.h"
@@ -31,14 +32,17 @@ struct GemmConfig {
   int dma;       // 0: register-staged (gemm_tile.h), 1: direct-to-LDS
                  // staging with 64-bit addresses (gemm16_dma.h), 2: 16-bit
                  // 256x256 tile (gemm16_w4.h), 5: 8-bit 256x256x128 and
-                 // 256x224x128 tiles (gemm8_w4.h, gemm8_n224.h); 2 and 5
-                 // address A and B through 32-bit buffer offsets
+                 // 256x224x128 tiles (gemm8_w4.h, gemm8_n224.h), 6: 128x128
+                 // tiles on a deep ring (gemm_ring.h, kRingConfigs); 2, 5 and
+                 // 6 address A and B through 32-bit buffer offsets
   int fmt;       // MX operand formats: MFMA code of A | code of B << 4
 };
 
-// Every (operands, tile, epilogue) instantiated.
-constexpr int kNumGemmConfigs = 52;
+// Every (operands, tile, epilogue) instantiated, and the 128x128 ring tiles
+// that serve 256x256 tile plans with TX_FLAG_TILES_128.
+constexpr int kNumGemmConfigs = 52, kNumRingConfigs = 34;
 extern const GemmConfig kGemmConfigs[kNumGemmConfigs];
+extern const GemmConfig kRingConfigs[kNumRingConfigs];
 
 // The kernels launched right before and after a tile, in the tiles' own unit
 // (code object): the upcast of an MX operand by [B side][format e4m3, e5m2,

@@ -31,60 +31,63 @@ int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 struct Tile {
   int32_t bm, bn, bk;
-  double eff;  // fraction of MFMA peak a tile of this size sustains
-  int occ = 1; // workgroups per CU that eff needs (latency hidden by each other)
+  bool tiles128 = false; // TX_FLAG_TILES_128: the 256x256 plan on 128x128 tiles
 };
 
-// Tiles the backend instantiates, largest first.  `eff` is the fraction of
-// the dense MFMA peak each tile sustained at 4096^3 on one MI355X (bench.py
-// --only tiles: bf16 -> bf16 and int8 -> int32, back-to-back launches):
-// 16-bit 256x256x64 0.509, 128x128x64 0.341, 64x64x32 0.187; 8-bit
-// 256x256x128 0.463, 128x128x128 0.173.  tileCost weighs them against the
-// waves of tiles a shape needs.
-// With fewer workgroups than occ per CU a tile runs at the rate of occ per
-// CU all the same (measured at M = 128 / 512, N = K = 8192: 64x64x32 190 us,
-// 128x128x64 154 us, where eff alone predicts 36 and 80).
-const Tile kTiles16[] = {{256, 256, 64, 0.509, 1}, {128, 128, 64, 0.341, 2},
-                         {64, 64, 32, 0.187, 4}};
-// 8-bit tiles.  (A 256x224 tile also exists for explicit requests: it fills
-// all CUs at N = 7168, but its A-resident wave layout needs 28 transposed B
-// reads per step against 16; it measured 0.273 at int8 4096^3 and no faster
-// than 256x256 at N = 7168.)
-const Tile kTiles8[] = {{256, 256, 128, 0.463, 1}, {128, 128, 128, 0.173, 2}};
-// MX (tl.dot_scaled) tiles: one 256x256 tile of 128 bytes of K per step,
-// i.e. 128 fp8 or 256 fp4 elements.
-const Tile kTileMx8 = {256, 256, 128, 0.45}, kTileMx4 = {256, 256, 256, 0.33};
+// Estimated time of a tiled dot, in us.  A round of n workgroups (at most one,
+// or `occ`, a CU) takes `per + steps * (s0 + s1 * n / CUs)`: a K step is
+// slower the more CUs load and draw power at once.  Fitted to back-to-back
+// launches on one MI355X, measured / estimated in us:
+//   bf16 256x256x64:  4096^3 104 / 106, 3072^3 61 / 70, M = 512 N = K = 8192 (split 4) 82 / 82;
+//   bf16 128x128:     M = 1000 N = K = 4000 39.4 / 39.6, 3072^3 78 / 79, 2048^3 22 / 23;
+//   bf16 64x64x32:    512^3 7.4 / 9, 1024^3 18 / 19;
+//   W8A8 256x256x128: 3072^3 39 / 43, M = 512 N = K = 8192 (split 4) 54 / 61;
+//   W8A8 128x128:     M = 512 N = K = 8192 40 / 41, 3072^3 50 / 46;
+//   fp8 block-scaled  256: M = 1024 N = K = 7168 73 / 77, 128: 79 / 80, M = 512 40 / 43;
+//   mxfp8             256: M = 1024 N = 8192 K = 4096 53 / 54, 128: 53 / 52;
+//   mxfp4             256: the same shape 33 / 34, 128: 36 / 36.
+struct Rate {
+  double launch, per, s0, s1;
+  int occ; // workgroups a CU
+};
+constexpr Rate k256x16{4.5, 2.5, 1.00, 0.55, 1}, k128x16{4.0, 2.2, 0.33, 0.20, 1};
+constexpr Rate k64x16{2.0, 0.5, 0.33, 0.20, 4}, k128dma{3.0, 0.5, 0.90, 0.40, 2};
+constexpr Rate k256x8{5.0, 3.0, 1.05, 0.70, 1}, k128x8{4.0, 2.2, 0.33, 0.22, 1};
+constexpr Rate k128f8b{4.0, 2.2, 0.40, 0.27, 1};
+constexpr Rate k256mx8{5.0, 3.0, 1.15, 0.55, 1}, k128mx8{4.0, 2.2, 0.40, 0.28, 1};
+constexpr Rate k256mx4{5.0, 3.0, 1.20, 0.90, 1}, k128mx4{4.0, 2.2, 0.48, 0.37, 1};
 
-// Estimated time of a tiled dot in MAC-units of one CU: whole waves of
-// occ workgroups a CU, each a tile over its K range costing BM*BN*K / eff.  The 256x256 tiles split K when they leave most CUs idle
-// (tx_gemm_split_k): the ranges run as more workgroups, and their fp32
-// partials, written and read back (8 S M N bytes), add their HBM time and a
-// second launch at `cu_macs` (a CU's peak MAC rate).
-double tileCost(const Tile &t, int64_t M, int64_t N, int64_t K, double cu_macs) {
-  const int64_t tiles = cdiv(M, t.bm) * cdiv(N, t.bn);
-  const int64_t ksteps = cdiv(K, t.bk);
-  const int32_t s = t.bm == 256 && t.bn == 256 ? tx_gemm_split_k(tiles, ksteps) : 1;
-  const int64_t waves = cdiv(tiles * s, (int64_t)kCUs * t.occ) * t.occ;
-  double c = (double)waves * t.bm * t.bn * (double)cdiv(ksteps, s) * t.bk / t.eff;
-  if (s > 1)
-    c += (8.0 * s * (double)M * (double)N / kHbm + 4e-6) * cu_macs;
-  return c;
+double estimate(const Rate &r, int64_t bm, int64_t bn, int64_t bk, int64_t split, int64_t M,
+                int64_t N, int64_t K) {
+  const int64_t n = cdiv(M, bm) * cdiv(N, bn) * split;
+  const double steps = (double)cdiv(cdiv(K, bk), split);
+  const int64_t cap = (int64_t)kCUs * r.occ, full = n / cap, rem = n % cap;
+  auto round = [&](int64_t wgs) {
+    return r.per + steps * (r.s0 + r.s1 * (wgs < kCUs ? (double)wgs / kCUs : 1.0));
+  };
+  double us = r.launch + (double)full * round(cap) + (rem ? round(rem) : 0.0);
+  if (split > 1) // the reduction, its partials written and read at about 6 TB/s
+    us += 3.0 + 8.0 * (double)split * (double)M * (double)N / 6e6;
+  return us;
 }
 
-// Cheapest candidate from index `first` on (the 256-wide tile is index 0).
-template <size_t N>
-Tile chooseTile(const Tile (&cands)[N], int64_t M, int64_t Nn, int64_t K, double cu_macs,
-                size_t first = 0) {
-  Tile best = cands[first];
-  double bestCost = tileCost(best, M, Nn, K, cu_macs);
-  for (size_t i = first + 1; i < N; ++i) {
-    double c = tileCost(cands[i], M, Nn, K, cu_macs);
-    if (c < bestCost) {
-      best = cands[i];
-      bestCost = c;
-    }
+// The 256x256 tile of a dot: on 256x256 or on 128x128 tiles (TX_FLAG_TILES_128).
+// bk: elements of 128 bytes of K; split256: the 256x256 tiles may split K.
+Tile choose256(const Rate &r256, const Rate &r128, int32_t bk, bool split256, int64_t M, int64_t N,
+               int64_t K, bool can128, double *us) {
+  Tile t{256, 256, bk};
+  const int64_t steps = cdiv(K, bk);
+  const int64_t s256 = split256 ? tx_gemm_split_k(cdiv(M, 256) * cdiv(N, 256), steps) : 1;
+  *us = estimate(r256, 256, 256, bk, s256, M, N, K);
+  if (!can128)
+    return t;
+  const double u128 = estimate(r128, 128, 128, bk,
+                               tx_ring_split_k(cdiv(M, 128) * cdiv(N, 128), steps), M, N, K);
+  if (u128 < *us) {
+    t.tiles128 = true;
+    *us = u128;
   }
-  return best;
+  return t;
 }
 
 } // namespace
@@ -94,6 +97,10 @@ extern "C" int32_t tx_gemm_split_k(int64_t tiles, int64_t ksteps) {
   while (s < 16 && tiles * s * 2 <= kCUs && ksteps / (s * 2) >= 8)
     s *= 2;
   return s;
+}
+
+extern "C" int32_t tx_ring_split_k(int64_t tiles128, int64_t ksteps) {
+  return tx_gemm_split_k(tiles128, ksteps); // the same rule on its own tiles
 }
 
 extern "C" int32_t tx_dtype_bits(int32_t dtype) {
@@ -157,7 +164,10 @@ extern "C" int tx_dot_operand_spans(const tx_dot_desc *d, int64_t *a_bytes, int6
   return TX_OK;
 }
 
-extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
+namespace {
+
+// tx_arith_intensity; *tiles128: the chosen tile runs on 128x128 tiles.
+int analyse(const tx_dot_desc *d, tx_ai_report *out, bool *tiles128) {
   if (!d || !out)
     return TX_ERR_INVALID;
   *out = tx_ai_report{};
@@ -194,7 +204,7 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
   double tm = out->bytes / out->peak_bw;
   out->roofline_us = 1e6 * (tc > tm ? tc : tm);
 
-  Tile t{d->block_m, d->block_n, d->block_k, 1.0};
+  Tile t{d->block_m, d->block_n, d->block_k};
   if (t.bm <= 0 || t.bn <= 0 || t.bk <= 0) {
     // Operands as the tile reads them (an upcast MX side: packed bf16), and
     // whether the 256-wide tiles (32-bit buffer offsets) can address them.
@@ -255,17 +265,39 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
                            (d->a_type == TX_BF16 || d->scale_mode == TX_SCALE_NV16) &&
                            d->M <= 96 && d->K >= 256 && d->N <= (int64_t)16384 * 128 &&
                            (d->c_type == TX_BF16 || d->c_type == TX_F32);
-    const size_t first = spanA < TX_SPAN32_LIMIT && spanB < TX_SPAN32_LIMIT ? 0 : 1;
+    // Operands the 32-bit-offset tiles reach; the 128x128 ring tiles also form
+    // the offsets of up to 127 rows of a row-major B past K.
+    const bool span32 = spanA < TX_SPAN32_LIMIT && spanB < TX_SPAN32_LIMIT;
+    const int64_t ldbBytes = (e.ldb ? e.ldb : kmajor ? e.K : e.N) * tx_dtype_bits(e.b_type) / 8;
+    const bool can128 = span32 && ldbBytes < TX_SPAN32_LIMIT / 128 &&
+                        cdiv(d->M, 128) * cdiv(d->N, 128) < (1 << 24);
+    const bool mx = d->scale_mode == TX_SCALE_MX32;
+    double us = 0.0;
+    // The 16-bit tiles: 256x256 (or 128x128) against 64x64, which only
+    // launch-bound sizes still take; operands past 2 GiB the tiles with 64-bit
+    // addresses.
+    auto tile16 = [&]() -> Tile {
+      if (!span32) {
+        const double u128 = estimate(k128dma, 128, 128, 64, 1, d->M, d->N, d->K);
+        return u128 <= estimate(k64x16, 64, 64, 32, 1, d->M, d->N, d->K) ? Tile{128, 128, 64}
+                                                                        : Tile{64, 64, 32};
+      }
+      const Tile t256 = choose256(k256x16, k128x16, 64, true, d->M, d->N, d->K, can128, &us);
+      if (!kmajor && estimate(k64x16, 64, 64, 32, 1, d->M, d->N, d->K) < us)
+        return Tile{64, 64, 32};
+      return t256;
+    };
     if (decode_wq)
-      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 128, 1.0};
+      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 128};
     else if (upcast)
-      t = chooseTile(kTiles16, d->M, d->N, d->K, kPeak16 / 2 / kCUs, first); // MX x bf16: bf16 tile
+      t = tile16(); // MX x bf16: the bf16 dot's tile
     else if (decode_mx)
-      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, ba == 4 ? 256 : 128, 1.0};
-    else if (d->scale_mode == TX_SCALE_MX32)
-      t = ba == 4 ? kTileMx4 : kTileMx8;
+      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, ba == 4 ? 256 : 128};
+    else if (mx) // (its 256x256 tiles do not split K)
+      t = ba == 4 ? choose256(k256mx4, k128mx4, 256, false, d->M, d->N, d->K, can128, &us)
+                  : choose256(k256mx8, k128mx8, 128, false, d->M, d->N, d->K, can128, &us);
     else if (decode_f8)
-      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 128, 1.0};
+      t = Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 128};
     else if (decode16) {
       // Every strip reads all of A, so A's re-reads are M / W of B's bytes.
       // Strips of W = 128 columns halve them: at N = K = 8192 bf16 M = 48 / 64
@@ -283,12 +315,10 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
       const int64_t nk = d->N * d->K;
       const bool wide = (rows >= 32 && rows <= 80 && nk >= ((int64_t)1 << 25)) ||
                         (rows == 16 && d->N >= 16384 && nk >= ((int64_t)1 << 26));
-      t = Tile{rows, wide ? 128 : 64, 128, 1.0};
+      t = Tile{rows, wide ? 128 : 64, 128};
     }
-    else if (sa == 2 && (d->flags & TX_FLAG_B_KMAJOR))
-      t = kTiles16[0]; // the K-major B kernel exists for this tile only
     else if (sa == 2)
-      t = chooseTile(kTiles16, d->M, d->N, d->K, kPeak16 / 2 / kCUs, first);
+      t = tile16();
     else if (decode && d->M <= 256)
       // W8A8 decode (M <= 256, N up to its 4096 column strips; past it the
       // 8-bit tiles with split-K: at N = K = 8192 M = 384 57.5 us, 512 63.9,
@@ -299,16 +329,17 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
       // N = K = 8192, in us: M = 32 20.1 / 22.1-22.7 (slices of 64), 48 22.0 /
       // 22.2-22.5, 64 25.2 / 22.3-22.9, 96 29.4 (64) / 31.2-32.0 (128), 128
       // 29.6 / 30.5, 192 53.5 / 43.7-44.8, 256 44.8 / 42.6.
-      t = d->M > 128 ? Tile{128, 128, 128, 1.0}
-          : d->M > 48 ? Tile{64, 128, 128, 1.0}
-                      : Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 64, 1.0};
-    else if (d->flags & TX_FLAG_B_KMAJOR)
-      t = kTiles8[0]; // of the 8-bit tiles only this one has a K-major B form
-    else if (d->a_type == TX_F8E4M3 || d->a_type == TX_F8E5M2)
-      t = kTiles8[first]; // the register-staged 128x128 tile is slower everywhere
+      t = d->M > 128 ? Tile{128, 128, 128}
+          : d->M > 48 ? Tile{64, 128, 128}
+                      : Tile{(int32_t)(16 * cdiv(d->M > 0 ? d->M : 1, 16)), 128, 64};
+    else if (!span32) // the register-staged tile: 64-bit addresses
+      t = Tile{128, 128, 128};
     else
-      t = chooseTile(kTiles8, d->M, d->N, d->K, kPeak8 / 2 / kCUs, first);
+      t = choose256(k256x8, d->scale_mode == TX_SCALE_BLOCK128 ? k128f8b : k128x8, 128, true, d->M,
+                    d->N, d->K, can128, &us);
   }
+  if (tiles128)
+    *tiles128 = t.tiles128;
   out->block_m = t.bm;
   out->block_n = t.bn;
   out->block_k = t.bk;
@@ -316,14 +347,23 @@ extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
   return TX_OK;
 }
 
+} // namespace
+
+extern "C" int tx_arith_intensity(const tx_dot_desc *d, tx_ai_report *out) {
+  return analyse(d, out, nullptr);
+}
+
 namespace {
 
 // Pass body: classification and tile choice for one dot.
 int txArithIntensityRun(tx_dot_plan *plan) {
   tx_ai_report r;
-  int rc = tx_arith_intensity(&plan->desc, &r);
+  bool tiles128 = false;
+  int rc = analyse(&plan->desc, &r, &tiles128);
   if (rc != TX_OK)
     return rc;
+  if (tiles128)
+    plan->desc.flags |= TX_FLAG_TILES_128;
   plan->flops = r.flops;
   plan->bytes = r.bytes;
   plan->intensity = r.intensity;

@@ -26,6 +26,7 @@ NOALLOC_SCRATCH_BYTES = 64 << 20
 FLAG_NO_LOOP_SPLIT = 0x1
 FLAG_B_KMAJOR = 0x2  # B stored [N][K] row-major (a transposed view in torch)
 FLAG_ACCUMULATE = 0x4  # C = C + A . B (fp32 / int32 C)
+FLAG_TILES_128 = 0x100  # a 256x256 tile plan on 128x128 tiles (set by the planner)
 # TritonPluginResult
 TP_SUCCESS, TP_GENERIC_FAILURE = 0, 1
 # tx_cmp_pred (arith::CmpIPredicate order)
