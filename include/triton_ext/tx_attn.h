@@ -64,7 +64,11 @@ typedef struct tx_attn_desc {
    * for fp8 e5m2); 0 = default (128, 64).  The
    * blocks fix the on-band split (causal_start = start_m * BLOCK_M) and the
    * online softmax's key blocks, so they select the rounding of the result
-   * exactly as the tutorial's config does. */
+   * exactly as the tutorial's config does -- but for fp16 / bf16 at 128 x 64
+   * where the programs leave CUs idle: groups of waves then run parts of a
+   * row's key blocks, each with its own running maximum, and their sums are
+   * merged in fp32 (the same precision; p is rounded against a group's
+   * maximum). */
   int32_t block_m, block_n;
 } tx_attn_desc;
 

@@ -1310,6 +1310,37 @@ int attnStrides(const tx_attn_desc &d, int64_t &sz, int64_t &sh, int64_t &sm,
 
 } // namespace
 
+namespace {
+
+// How a plan's keys are split among groups of waves (attn_fwd.h, KS): 0 not
+// at all, 1 in 128 rows x 2 groups, 2 64 x 2, 3 32 x 4.  programs: row blocks of
+// 128 over all heads.  bf16, us without / with the split, causal, one MI355X:
+//   64 programs or fewer, 4 key blocks or more, head dim <= 64 (32 x 4): N = 1024 12.2 / 6.9
+//     (head dim 32), 15.2 / 9.5 (64); 8192 keys of one head 73.8 / 27.4, 87.9 / 41.0
+//   128 programs or fewer (64 x 2): N = 1024 12.1 / 9.1 (32), 15.1 / 11.7 (64),
+//     22.0 / 18.2 (128); N = 128 4.6 / 4.1, 5.9 / 5.2, 8.2 / 7.2; at 192 they lose
+//   256 or fewer, 16 key blocks or more (128 x 2): N = 4096 39.2 / 30.6, 47.1 / 39.7,
+//     68.1 / 59.1; N = 1024 12.3 / 10.7, 15.6 / 14.4, 22.4 / 21.3
+//   head dim <= 32 past that (its softmax leaves the matrix cores idle): 512 programs
+//     31.9 / 28.9, 1024 causal 55.1 / 46.1 (without the mask 58.0 / 57.3: left alone)
+// e5m2 keeps one group: p is rounded to two bits against the running maximum, and a
+// group's own maximum rounds it differently (o changes by 4-7%).
+int attnKs(const tx_attn_plan &p) {
+  const tx_attn_desc &d = p.desc;
+  if (d.block_m != 128 || d.block_n != 64 || d.dtype == TX_F8E5M2 || d.head_dim > 128)
+    return 0;
+  const int64_t programs = p.grid_x, blocks = d.N_CTX / 64;
+  if (programs <= 64 && d.head_dim <= 64 && blocks >= 4)
+    return 3;
+  if (programs <= 128)
+    return 2;
+  if (blocks >= 16 && (programs <= 256 || (d.head_dim <= 32 && (d.causal || programs <= 512))))
+    return 1;
+  return 0;
+}
+
+} // namespace
+
 extern "C" TX_API int tx_attn_fwd_plan(const tx_attn_desc *desc, tx_attn_plan *plan) {
   g_last_error.clear();
   if (!desc || !plan)
@@ -1422,7 +1453,13 @@ extern "C" TX_API int tx_attn_fwd_launch(const tx_attn_plan *plan, const void *q
                                      : 4;
   const AttnFn fn = d.dtype == TX_F8E5M2 ? kAttn8[c][hd][bm64][bn32]
                                          : kAttn[c][hd][d.dtype == TX_BF16][bm64][bn32];
-  hipLaunchKernelGGL(fn, dim3(plan->grid_x), dim3(plan->block_threads), 0, s, a);
+  if (const int ks = attnKs(*plan)) {
+    const int bm = ks == 1 ? 128 : ks == 2 ? 64 : 32, groups = ks == 3 ? 4 : 2;
+    hipLaunchKernelGGL(kAttnKs[ks - 1][c][hd][d.dtype == TX_BF16],
+                       dim3(plan->grid_x * (128 / bm)), dim3(bm * 2 * groups), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(fn, dim3(plan->grid_x), dim3(plan->block_threads), 0, s, a);
+  }
   TX_HIP_CHECK(hipGetLastError());
   return TX_OK;
 }

@@ -70,7 +70,8 @@ template <int HD, bool BF, int BM_ = 128, int BN_ = 64> struct AttnFwd {
   static constexpr uint32_t kOOB = 0x80000000u;
   static_assert(D == 32 || D == 64 || D == 128 || D == 256, "head dims 16 .. 256");
   static_assert(DR == D || (DR == 16 && D == 32), "head dim 16 in the layout of 32");
-  static_assert((BM == 64 || BM == 128) && (BN == 32 || BN == 64), "the tutorial's blocks");
+  static_assert((BM == 64 || BM == 128) && (BN == 32 || BN == 64) || (BM == 32 && BN == 64),
+                "the tutorial's blocks, or one wave's rows");
   static_assert(LW >= 1 && DMA >= 1 && DMA * LW * 1024 == TILE, "whole 1 KiB loads per wave");
   // Fragment reads issued together in qk / pv: every one at head dims up to
   // 128, in groups of 8 at 256 (all 32 would take 128 VGPRs).
@@ -363,10 +364,27 @@ template <int HD, bool BF, int BM_ = 128, int BN_ = 64> struct AttnFwd {
 // odd block and last when it ends at one.
 // A: the element type's fragments (AttnFwd<HD, BF> here, AttnFwd8<HD> for
 // e5m2).
-template <bool CAUSAL, class A> __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[4 * A::TILE];
+//
+// KS > 1: KS groups of waves share the workgroup's query rows, each running
+// 1 / KS of the key blocks through LDS slots of its own; at the end the other
+// groups' (m, l, acc) go through LDS and the first one merges them in order,
+// acc = acc_0 2^(m_0 - m) + acc_1 2^(m_1 - m) and l alike, in fp32.  A launch of
+// few workgroups is the serial chain of its longest row block, whose waves
+// spend most of a block in the softmax: fewer rows a workgroup with more groups
+// use the idle CUs and cut the chain (the times stand at the launch's choice).
+// What bounds it then: the softmax's VALU work at head dims up to 64, the LDS
+// reads of K and V (every wave reads all of its group's blocks) at 128.
+// The groups after the first start from m = -FLT_MAX, l = 0 rather than -inf, 1:
+// a first block of scores that are all -inf then adds nothing, as it would
+// after the first group's blocks.
+template <bool CAUSAL, class A, int KS = 1>
+__device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[KS * 4 * A::TILE];
+  __shared__ float ml[KS > 1 ? (KS - 1) * A::NW * 128 : 1];
+  static_assert((KS - 1) * A::NW * 64 * (A::D / 2) * 4 <= KS * 4 * A::TILE, "acc fits the slots");
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_wg % A::NW, kg = KS > 1 ? wave_wg / A::NW : 0;
   const int g = lane >> 5;
   // Program order: the 8 XCDs take contiguous runs of programs (a head's
   // K/V stays in one L2), and within a head the longest causal rows first.
@@ -386,7 +404,7 @@ template <bool CAUSAL, class A> __device__ __forceinline__ void attn_fwd_body(co
   const i32x4_t rv = make_rsrc(Vh, A::v_bytes(p.N_CTX, p.v_sm));
   uint32_t ko[A::DMA], vo[A::DMA];
   A::kv_offsets(wave, p.k_sm, p.v_sm, ko, vo);
-  const uint32_t k_lds = lds_addr(smem), v_lds = k_lds + 2 * A::TILE;
+  const uint32_t k_lds = lds_addr(smem) + kg * 4 * A::TILE, v_lds = k_lds + 2 * A::TILE;
   typename A::Bases bs;
   A::bases(k_lds, v_lds, bs);
 
@@ -394,40 +412,50 @@ template <bool CAUSAL, class A> __device__ __forceinline__ void attn_fwd_body(co
   // causal_start): unmasked blocks [0, n_main), masked [n_main, n_end).
   // N_CTX and causal_start are multiples of BM, itself a multiple of BN.
   const int causal_start = CAUSAL ? start_m * A::BM : p.N_CTX;
-  const int n_main = causal_start / A::BN;
-  const int n_end = CAUSAL ? (causal_start + A::BM) / A::BN : n_main;
+  const int all_main = causal_start / A::BN;
+  const int all_end = CAUSAL ? (causal_start + A::BM + A::BN - 1) / A::BN : all_main;
+  // This group's blocks: j0 + [0, n_main) unmasked, j0 + [n_main, n_end) masked;
+  // every group runs n_it iterations (its barriers are the workgroup's).
+  const int n_it = KS > 1 ? (all_end + KS - 1) / KS : all_end;
+  const int j0 = kg * n_it;
+  const int rest = all_end - j0; // (below 0: a group with no blocks at all)
+  const int n_end = KS > 1 ? (rest < 0 ? 0 : rest < n_it ? rest : n_it) : all_end;
+  const int n_main = KS > 1 ? (all_main - j0 < 0 ? 0 : all_main - j0 < n_end ? all_main - j0 : n_end)
+                            : all_main;
 
-  float m_i = -INFINITY, l_i = 1.0f;
+  float m_i = kg == 0 ? -INFINITY : -3.402823466e38f, l_i = kg == 0 ? 1.0f : 0.0f;
   typename A::f16v acc[A::D / 32], s[A::BN / 32];
 #pragma unroll
   for (int bd = 0; bd < A::D / 32; ++bd)
     acc[bd] = typename A::f16v{};
 
-  A::issue_k(rk, ko, p.k_sm, 0, k_lds, wave);
-  A::issue_v(rv, vo, p.v_sm, 0, v_lds, wave);
-  if (n_end > 1)
-    A::issue_k(rk, ko, p.k_sm, 1, k_lds + A::TILE, wave);
+  if (KS == 1 || n_end > 0) {
+    A::issue_k(rk, ko, p.k_sm, j0, k_lds, wave);
+    A::issue_v(rv, vo, p.v_sm, j0, v_lds, wave);
+    if (n_end > 1)
+      A::issue_k(rk, ko, p.k_sm, j0 + 1, k_lds + A::TILE, wave);
+  }
   __builtin_amdgcn_s_waitcnt(0x7 << 4); // vmcnt(0)
   __syncthreads();
-  A::template qk<0>(bs, qf, s);
+  A::template qk<0>(bs, qf, s); // (an empty group: stale values, not used)
   __syncthreads(); // K slot 0 is refilled by iteration 0
 
   auto iter = [&](int j, auto mask, auto slot) {
     constexpr bool MASK = decltype(mask)::value;
     constexpr int SL = decltype(slot)::value;
     if (j + 2 < n_end)
-      A::issue_k(rk, ko, p.k_sm, j + 2, k_lds + SL * A::TILE, wave);
+      A::issue_k(rk, ko, p.k_sm, j0 + j + 2, k_lds + SL * A::TILE, wave);
     if (j + 1 < n_end)
-      A::issue_v(rv, vo, p.v_sm, j + 1, v_lds + (1 - SL) * A::TILE, wave);
+      A::issue_v(rv, vo, p.v_sm, j0 + j + 1, v_lds + (1 - SL) * A::TILE, wave);
     typename A::f16v sn[A::BN / 32];
     A::template qk<1 - SL>(bs, qf, sn); // S_{j+1} (a stale slot after the last block: unused)
     // On-band blocks whose keys all lie past this wave's 32 rows add exactly
     // nothing (p = 0, alpha = 1, as for the blocks past the diagonal): the
     // wave skips their softmax and P V.
-    const bool live = !MASK || j * A::BN <= start_m * A::BM + 32 * wave + 31;
+    const bool live = !MASK || (j0 + j) * A::BN <= start_m * A::BM + 32 * wave + 31;
     if (live) {
       typename A::PF pf;
-      A::template softmax<MASK>(s, j * A::BN, m, p.qk_scale, acc, m_i, l_i, pf);
+      A::template softmax<MASK>(s, (j0 + j) * A::BN, m, p.qk_scale, acc, m_i, l_i, pf);
       A::template pv<SL>(bs, pf, acc);
     }
 #pragma unroll
@@ -450,6 +478,44 @@ template <bool CAUSAL, class A> __device__ __forceinline__ void attn_fwd_body(co
   };
   segment(0, n_main, std::false_type());
   segment(n_main, n_end, std::true_type());
+  if constexpr (KS > 1) {
+    for (int j = n_end; j < n_it; ++j)
+      __syncthreads(); // an iteration this group does not have
+    // Merge: per wave and lane, D / 2 accumulators as 16-byte quads in lane
+    // order (the loop's closing barrier has freed the slots).
+    typedef float f4_t __attribute__((ext_vector_type(4)));
+    f4_t *const xch = reinterpret_cast<f4_t *>(smem);
+    constexpr int Q = A::D / 8; // quads a lane
+    if (kg > 0) {
+      const int w = (kg - 1) * A::NW + wave;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        xch[(w * Q + q) * 64 + lane] =
+            f4_t{acc[q / 4][4 * (q % 4)], acc[q / 4][4 * (q % 4) + 1], acc[q / 4][4 * (q % 4) + 2],
+                 acc[q / 4][4 * (q % 4) + 3]};
+      ml[w * 128 + lane] = m_i;
+      ml[w * 128 + 64 + lane] = l_i;
+    }
+    __syncthreads();
+    if (kg > 0)
+      return;
+#pragma unroll
+    for (int k = 0; k < KS - 1; ++k) {
+      const int w = k * A::NW + wave;
+      const float m1 = ml[w * 128 + lane], l1 = ml[w * 128 + 64 + lane];
+      const float mm = fmaxf(m_i, m1);
+      const float a0 = __builtin_amdgcn_exp2f(m_i - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
+      l_i = l_i * a0 + l1 * a1;
+      m_i = mm;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const f4_t o = xch[(w * Q + q) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[q / 4][4 * (q % 4) + e] = acc[q / 4][4 * (q % 4) + e] * a0 + o[e] * a1;
+      }
+    }
+  }
 
   // Epilogue: M = m_i + log2(l_i); O = acc / l_i.
   A::store_o(acc, l_i,
@@ -462,6 +528,12 @@ template <bool CAUSAL, class A> __device__ __forceinline__ void attn_fwd_body(co
 template <bool CAUSAL, int HD, bool BF, int BM = 128, int BN = 64>
 __global__ void __launch_bounds__(BM * 2, HD >= 256 ? 1 : 2) attn_fwd_kernel(AttnArgs p) {
   attn_fwd_body<CAUSAL, AttnFwd<HD, BF, BM, BN>>(p);
+}
+
+// KS groups of waves a workgroup of BM rows, 1 / KS of the keys each.
+template <bool CAUSAL, int HD, bool BF, int BM, int KS>
+__global__ void __launch_bounds__(BM * 2 * KS, BM * KS / 128) attn_fwd_ks_kernel(AttnArgs p) {
+  attn_fwd_body<CAUSAL, AttnFwd<HD, BF, BM, 64>, KS>(p);
 }
 
 } // namespace txk
