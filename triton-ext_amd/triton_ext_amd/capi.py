@@ -65,6 +65,9 @@ class AttnDesc(ctypes.Structure):
                 [("block_m", ctypes.c_int32), ("block_n", ctypes.c_int32)])
 
 
+_ATTN_STRIDES = {t: (f"{t}_sz", f"{t}_sh", f"{t}_sm") for t in "qkvo"}
+
+
 class AttnPlan(ctypes.Structure):
     _fields_ = [("desc", AttnDesc), ("flops", ctypes.c_double), ("bytes", ctypes.c_double),
                 ("qk_scale", ctypes.c_float), ("m_blocks", ctypes.c_int32), ("grid_x", ctypes.c_int32),
@@ -226,12 +229,10 @@ def attn_plan(Z, H, N_CTX, head_dim, causal, sm_scale, dtype=F16, strides=None, 
     """Plan the fused attention forward.  strides: {"q": (sz, sh, sm), ...}
     in elements (missing tensors: packed); for dtype F8E5M2, v's are (batch,
     head, head-dim row) of its key-contiguous storage."""
-    d = AttnDesc()
-    d.Z, d.H, d.N_CTX, d.head_dim, d.dtype = Z, H, N_CTX, head_dim, dtype
-    d.causal, d.sm_scale = int(bool(causal)), sm_scale
+    d = AttnDesc(Z, H, N_CTX, head_dim, dtype, int(bool(causal)), sm_scale)
     for t, st in (strides or {}).items():
-        for f, x in zip(("sz", "sh", "sm"), st):
-            setattr(d, f"{t}_{f}", x)
+        for f, x in zip(_ATTN_STRIDES.get(t, ()), st):
+            setattr(d, f, x)
     d.block_m, d.block_n = block
     p = AttnPlan()
     check(load().tx_attn_fwd_plan(ctypes.byref(d), ctypes.byref(p)))
