@@ -39,6 +39,12 @@
 // for 16 bits K steps 0 and 1 of 32 elements).  MFMA roles are swapped as on
 // the other tiles: lane l ends with C row l % 16 at 4 consecutive columns.
 //
+// Sums: with fp32 C the accumulators are emptied into a second set every 8
+// steps, so no chain of additions is longer than 8 steps or their number.  A
+// range here is up to 8 times the one the 256x256 tile's own split would take,
+// and one chain over it doubled the error (bf16 860x1856x4928 against 64 bits:
+// 3.0e-7, that tile 1.5e-7, this 1.3e-7).
+//
 // The plan is the 256x256 tile's (TX_FLAG_TILES_128): its block_k is one ring
 // step.  Split-K ranges are whole steps; a range's partial C is 32-bit, summed
 // by splitk_reduce.h.
@@ -61,6 +67,7 @@ template <int OP, int EPI, int FA = 0, int FB = 0, bool BT = false> struct GemmR
   static constexpr bool F4 = MX && FA == 4;
   static constexpr bool W32 = EPI == EPI_F32 || EPI == EPI_I32 || EPI == EPI_BLOCK128_F32 ||
                               EPI == EPI_MX_F32; // 32-bit C
+  static constexpr bool CHAINS = W32 && !INT; // sums in two levels
   static constexpr int SG = F4 ? 8 : 4, NSD = F4 ? 4 : 2, RS = 4 * NSD; // MX (gemm8_w4.h)
   static constexpr int A_BYTES = 16384, SA_OFF = 32768;
   static constexpr int SB_OFF = SA_OFF + (MX ? BM * RS : SCALED ? BM * 4 : 0);
@@ -470,6 +477,14 @@ template <int OP, int EPI, int FA = 0, int FB = 0, bool BT = false> struct GemmR
 #pragma unroll
       for (int j = 0; j < FN; ++j)
         acc[i][j] = Acc{0, 0, 0, 0};
+    Acc sum[CHAINS ? FM : 1][FN];
+    if constexpr (CHAINS) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          sum[i][j] = Acc{0, 0, 0, 0};
+    }
     auto slot = [&](int i) { return lds0 + (uint32_t)((unsigned)i % S) * SLOT; };
     auto issue_step = [&](int i) { // ring step i of the range into slot i % S
       const int kt = k_begin + i;
@@ -504,6 +519,17 @@ template <int OP, int EPI, int FA = 0, int FB = 0, bool BT = false> struct GemmR
       for (; i + 1 < nu; i += 2) {
         step(i, f[0], f[1], std::false_type());
         step(i + 1, f[1], f[0], std::false_type());
+        if constexpr (CHAINS) {
+          if ((i & 6) == 6) {
+#pragma unroll
+            for (int x = 0; x < FM; ++x)
+#pragma unroll
+              for (int y = 0; y < FN; ++y) {
+                sum[x][y] += acc[x][y];
+                acc[x][y] = Acc{0, 0, 0, 0};
+              }
+          }
+        }
       }
       for (; i < n; i += 2) {
         step(i, f[0], f[1], std::true_type());
@@ -511,6 +537,13 @@ template <int OP, int EPI, int FA = 0, int FB = 0, bool BT = false> struct GemmR
           step(i + 1, f[1], f[0], std::true_type());
       }
       __builtin_amdgcn_s_waitcnt(0); // the zero loads past the range have landed
+    }
+    if constexpr (CHAINS) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] += sum[i][j];
     }
     epilogue(p, C, m0, n0, wm, wn, acc, lds0);
   }
