@@ -384,7 +384,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   static_assert((KS - 1) * A::NW * 64 * (A::D / 2) * 4 <= KS * 4 * A::TILE, "acc fits the slots");
   const int lane = threadIdx.x & 63;
   const int wave_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wave = wave_wg % A::NW, kg = KS > 1 ? wave_wg / A::NW : 0;
+  const int wave = KS > 1 ? wave_wg % A::NW : wave_wg, kg = KS > 1 ? wave_wg / A::NW : 0;
   const int g = lane >> 5;
   // Program order: the 8 XCDs take contiguous runs of programs (a head's
   // K/V stays in one L2), and within a head the longest causal rows first.
@@ -413,17 +413,24 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   // N_CTX and causal_start are multiples of BM, itself a multiple of BN.
   const int causal_start = CAUSAL ? start_m * A::BM : p.N_CTX;
   const int all_main = causal_start / A::BN;
-  const int all_end = CAUSAL ? (causal_start + A::BM + A::BN - 1) / A::BN : all_main;
+  const int all_end =
+      CAUSAL ? (causal_start + A::BM + (A::BM < A::BN ? A::BN - 1 : 0)) / A::BN : all_main;
   // This group's blocks: j0 + [0, n_main) unmasked, j0 + [n_main, n_end) masked;
   // every group runs n_it iterations (its barriers are the workgroup's).
-  const int n_it = KS > 1 ? (all_end + KS - 1) / KS : all_end;
-  const int j0 = kg * n_it;
-  const int rest = all_end - j0; // (below 0: a group with no blocks at all)
-  const int n_end = KS > 1 ? (rest < 0 ? 0 : rest < n_it ? rest : n_it) : all_end;
-  const int n_main = KS > 1 ? (all_main - j0 < 0 ? 0 : all_main - j0 < n_end ? all_main - j0 : n_end)
-                            : all_main;
+  [[maybe_unused]] int n_it = all_end, j0 = 0;
+  int n_end = all_end, n_main = all_main;
+  if constexpr (KS > 1) {
+    n_it = (all_end + KS - 1) / KS;
+    j0 = kg * n_it;
+    n_end = all_end - j0 < 0 ? 0 : all_end - j0 < n_it ? all_end - j0 : n_it;
+    n_main = all_main - j0 < 0 ? 0 : all_main - j0 < n_end ? all_main - j0 : n_end;
+  }
 
-  float m_i = kg == 0 ? -INFINITY : -3.402823466e38f, l_i = kg == 0 ? 1.0f : 0.0f;
+  float m_i = -INFINITY, l_i = 1.0f;
+  if (KS > 1 && kg > 0) {
+    m_i = -3.402823466e38f;
+    l_i = 0.0f;
+  }
   typename A::f16v acc[A::D / 32], s[A::BN / 32];
 #pragma unroll
   for (int bd = 0; bd < A::D / 32; ++bd)
@@ -440,22 +447,29 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   A::template qk<0>(bs, qf, s); // (an empty group: stale values, not used)
   __syncthreads(); // K slot 0 is refilled by iteration 0
 
+  // Block j of the group, among all of the row's.
+  auto at = [&](int j) {
+    if constexpr (KS > 1)
+      return j0 + j;
+    else
+      return j;
+  };
   auto iter = [&](int j, auto mask, auto slot) {
     constexpr bool MASK = decltype(mask)::value;
     constexpr int SL = decltype(slot)::value;
     if (j + 2 < n_end)
-      A::issue_k(rk, ko, p.k_sm, j0 + j + 2, k_lds + SL * A::TILE, wave);
+      A::issue_k(rk, ko, p.k_sm, at(j + 2), k_lds + SL * A::TILE, wave);
     if (j + 1 < n_end)
-      A::issue_v(rv, vo, p.v_sm, j0 + j + 1, v_lds + (1 - SL) * A::TILE, wave);
+      A::issue_v(rv, vo, p.v_sm, at(j + 1), v_lds + (1 - SL) * A::TILE, wave);
     typename A::f16v sn[A::BN / 32];
     A::template qk<1 - SL>(bs, qf, sn); // S_{j+1} (a stale slot after the last block: unused)
     // On-band blocks whose keys all lie past this wave's 32 rows add exactly
     // nothing (p = 0, alpha = 1, as for the blocks past the diagonal): the
     // wave skips their softmax and P V.
-    const bool live = !MASK || (j0 + j) * A::BN <= start_m * A::BM + 32 * wave + 31;
+    const bool live = !MASK || at(j) * A::BN <= start_m * A::BM + 32 * wave + 31;
     if (live) {
       typename A::PF pf;
-      A::template softmax<MASK>(s, (j0 + j) * A::BN, m, p.qk_scale, acc, m_i, l_i, pf);
+      A::template softmax<MASK>(s, at(j) * A::BN, m, p.qk_scale, acc, m_i, l_i, pf);
       A::template pv<SL>(bs, pf, acc);
     }
 #pragma unroll
