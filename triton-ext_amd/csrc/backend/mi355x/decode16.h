@@ -83,6 +83,13 @@
 //    (exact, as is their ldexp short of overflow) and rounds once.  e4m3
 //    scales (not powers of two) multiply the fp32 pair; the product is exact
 //    in bf16.
+//  * One wave a SIMD and little to load, so a batch's own serial chain bounds it
+//    (bf16 x e2m1, 16 x 8192 x 16384: 0.87 us a batch of 128 K, of which its
+//    loads are 0.15).  Hence one block of LDS reads and one wait a batch rather
+//    than three, one branch for the upcast rather than one a fragment, load
+//    addresses kept and advanced rather than worked out, and a loop that is not
+//    unrolled by the ring (its code holds both upcasts): 0.55 us a batch.  M =
+//    32, N = K = 8192: 23.9 -> 19.3 us (e2m1), 25.2 -> 19.9 (e4m3).
 //  * Scales are staged per segment of 128 groups like decode_f8.h's MX form;
 //    columns past N and groups past K take a unit scale (their codes are 0).
 #pragma once
@@ -334,69 +341,72 @@ __device__ __forceinline__ void dec16_read_bk_pair(uint32_t b0, uint32_t b1, i32
                : "memory");
 }
 
-// WQ: the operands of two K steps: NB transposed reads of each of the wave's
-// two column blocks (e2m1: one, both steps' dwords; fp8: one a step, +4 KiB),
-// the blocks' staged scale dwords (three from an aligned address, of which
-// the batch's bytes are cut at the row's misalignment) and T row tiles of A.
-#define TX_DWQ_T(t, off)                                                                   \
+// WQ: a batch's operands of up to 4 row tiles in one block of LDS reads: both
+// column blocks' staged scale dwords (three from an aligned address, of which
+// the batch's bytes are cut at the row's misalignment), their NB transposed
+// reads of B (e2m1: 2, both steps' dwords in one; fp8: 4, one a step; 4 KiB
+// apart) and the T row tiles of A of the 4 K steps.
+#define TX_DWQ_S                                                                           \
+  "ds_read2_b32 %[p0], %[s0] offset0:0 offset1:1\n\tds_read2_b32 %[p1], %[s1] offset0:0 offset1:1\n\t" \
+  "ds_read_b32 %[r0], %[s0] offset:8\n\tds_read_b32 %[r1], %[s1] offset:8\n\t"
+#define TX_DWQ_B(h, off)                                                                   \
+  "ds_read_b64_tr_b8 %[y0" #h "], %[b0] offset:" #off "\n\tds_read_b64_tr_b8 %[y1" #h            \
+  "], %[b1] offset:" #off "\n\t"
+#define TX_DWQ_A(t, off)                                                                   \
   "ds_read_b128 %[x0" #t "], %[a0] offset:" #off "\n\tds_read_b128 %[x1" #t "], %[a1] offset:" #off \
-  "\n\t"
-#define TX_DWQ_O(t) [x0##t] "=&v"(a[0][t]), [x1##t] "=&v"(a[1][t])
-#define TX_DWQ_H1                                                                          \
-  "ds_read_b64_tr_b8 %[y0], %[b0]\n\tds_read_b64_tr_b8 %[y1], %[b1]\n\t"
-#define TX_DWQ_H2                                                                          \
-  TX_DWQ_H1 "ds_read_b64_tr_b8 %[y2], %[b0] offset:4096\n\tds_read_b64_tr_b8 %[y3], %[b1] offset:4096\n\t"
-#define TX_DWQ_BO1 [y0] "=&v"(bq[0][0]), [y1] "=&v"(bq[1][0])
-#define TX_DWQ_BO2 TX_DWQ_BO1, [y2] "=&v"(bq[0][1]), [y3] "=&v"(bq[1][1])
-#define TX_DWQ_IN [b0] "v"(b0), [b1] "v"(b1), [a0] "v"(a0), [a1] "v"(a1)
-#define TX_DWQ_ASM(H, BO)                                                                  \
+  "\n\tds_read_b128 %[x2" #t "], %[a2] offset:" #off "\n\tds_read_b128 %[x3" #t                \
+  "], %[a3] offset:" #off "\n\t"
+#define TX_DWQ_BO(h) [y0##h] "=&v"(bq[0][h]), [y1##h] "=&v"(bq[1][h])
+#define TX_DWQ_AO(t)                                                                       \
+  [x0##t] "=&v"(a[0][t]), [x1##t] "=&v"(a[1][t]), [x2##t] "=&v"(a[2][t]), [x3##t] "=&v"(a[3][t])
+#define TX_DWQ_ASM(B, BO, A, ...)                                                          \
+  asm volatile(TX_DWQ_S B A "s_waitcnt lgkmcnt(0)"                                          \
+               : [p0] "=&v"(p0), [p1] "=&v"(p1), [r0] "=&v"(v[0][2]), [r1] "=&v"(v[1][2]), BO, \
+                 __VA_ARGS__                                                               \
+               : [s0] "v"(s0), [s1] "v"(s1), [b0] "v"(b0), [b1] "v"(b1), [a0] "v"(a0),       \
+                 [a1] "v"(a1), [a2] "v"(a2), [a3] "v"(a3)                                   \
+               : "memory")
+#define TX_DWQ_T(B, BO)                                                                    \
   if constexpr (T == 1)                                                                    \
-    asm volatile(H TX_DWQ_T(0, 0) "s_waitcnt lgkmcnt(0)" : BO, TX_DWQ_O(0) : TX_DWQ_IN : "memory"); \
+    TX_DWQ_ASM(B, TX_DWQ_C(BO), TX_DWQ_A(0, 0), TX_DWQ_AO(0));                              \
   else if constexpr (T == 2)                                                               \
-    asm volatile(H TX_DWQ_T(0, 0) TX_DWQ_T(1, 4096) "s_waitcnt lgkmcnt(0)"                  \
-                 : BO, TX_DWQ_O(0), TX_DWQ_O(1)                                            \
-                 : TX_DWQ_IN                                                               \
-                 : "memory");                                                              \
+    TX_DWQ_ASM(B, TX_DWQ_C(BO), TX_DWQ_A(0, 0) TX_DWQ_A(1, 4096), TX_DWQ_AO(0), TX_DWQ_AO(1)); \
   else if constexpr (T == 3)                                                               \
-    asm volatile(H TX_DWQ_T(0, 0) TX_DWQ_T(1, 4096) TX_DWQ_T(2, 8192) "s_waitcnt lgkmcnt(0)" \
-                 : BO, TX_DWQ_O(0), TX_DWQ_O(1), TX_DWQ_O(2)                               \
-                 : TX_DWQ_IN                                                               \
-                 : "memory");                                                              \
+    TX_DWQ_ASM(B, TX_DWQ_C(BO), TX_DWQ_A(0, 0) TX_DWQ_A(1, 4096) TX_DWQ_A(2, 8192),         \
+               TX_DWQ_AO(0), TX_DWQ_AO(1), TX_DWQ_AO(2));                                   \
   else                                                                                     \
-    asm volatile(H TX_DWQ_T(0, 0) TX_DWQ_T(1, 4096) TX_DWQ_T(2, 8192) TX_DWQ_T(3, 12288)    \
-                 "s_waitcnt lgkmcnt(0)"                                                    \
-                 : BO, TX_DWQ_O(0), TX_DWQ_O(1), TX_DWQ_O(2), TX_DWQ_O(3)                   \
-                 : TX_DWQ_IN                                                               \
-                 : "memory")
+    TX_DWQ_ASM(B, TX_DWQ_C(BO),                                                             \
+               TX_DWQ_A(0, 0) TX_DWQ_A(1, 4096) TX_DWQ_A(2, 8192) TX_DWQ_A(3, 12288),       \
+               TX_DWQ_AO(0), TX_DWQ_AO(1), TX_DWQ_AO(2), TX_DWQ_AO(3))
+#define TX_DWQ_BO2 TX_DWQ_BO(0), TX_DWQ_BO(1)
+#define TX_DWQ_BO4 TX_DWQ_BO2, TX_DWQ_BO(2), TX_DWQ_BO(3)
 template <int T, int NB>
-__device__ __forceinline__ void decwq_read_pair(uint32_t b0, uint32_t b1, uint32_t a0, uint32_t a1,
-                                                v2i_t (&bq)[2][NB], i32x4_t (&a)[2][T]) {
-  if constexpr (NB == 1) {
-    TX_DWQ_ASM(TX_DWQ_H1, TX_DWQ_BO1);
+__device__ __forceinline__ void decwq_read(uint32_t s0, uint32_t s1, uint32_t b0, uint32_t b1,
+                                           uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3,
+                                           uint32_t (&v)[2][3], v2i_t (&bq)[2][NB],
+                                           i32x4_t (&a)[4][T]) {
+  v2i_t p0, p1;
+  if constexpr (NB == 2) {
+#define TX_DWQ_C(x) TX_DWQ_BO2
+    TX_DWQ_T(TX_DWQ_B(0, 0) TX_DWQ_B(1, 4096), 0);
+#undef TX_DWQ_C
   } else {
-    TX_DWQ_ASM(TX_DWQ_H2, TX_DWQ_BO2);
+#define TX_DWQ_C(x) TX_DWQ_BO4
+    TX_DWQ_T(TX_DWQ_B(0, 0) TX_DWQ_B(1, 4096) TX_DWQ_B(2, 8192) TX_DWQ_B(3, 12288), 0);
+#undef TX_DWQ_C
   }
+  v[0][0] = p0.x, v[0][1] = p0.y;
+  v[1][0] = p1.x, v[1][1] = p1.y;
 }
+#undef TX_DWQ_S
+#undef TX_DWQ_B
+#undef TX_DWQ_A
+#undef TX_DWQ_BO
+#undef TX_DWQ_AO
 #undef TX_DWQ_ASM
-#undef TX_DWQ_IN
-#undef TX_DWQ_BO2
-#undef TX_DWQ_BO1
-#undef TX_DWQ_H2
-#undef TX_DWQ_H1
-#undef TX_DWQ_O
 #undef TX_DWQ_T
-__device__ __forceinline__ void decwq_read_scales(uint32_t x0, uint32_t x1, uint32_t (&v)[2][3]) {
-  v2i_t p, q;
-  uint32_t r, t;
-  asm volatile("ds_read2_b32 %0, %4 offset0:0 offset1:1\n\tds_read2_b32 %1, %5 offset0:0 offset1:1\n\t"
-               "ds_read_b32 %2, %4 offset:8\n\tds_read_b32 %3, %5 offset:8\n\t"
-               "s_waitcnt lgkmcnt(0)"
-               : "=&v"(p), "=&v"(q), "=&v"(r), "=&v"(t)
-               : "v"(x0), "v"(x1)
-               : "memory");
-  v[0][0] = p.x, v[0][1] = p.y, v[0][2] = r;
-  v[1][0] = q.x, v[1][1] = q.y, v[1][2] = t;
-}
+#undef TX_DWQ_BO2
+#undef TX_DWQ_BO4
 
 // Elements 2 i and 2 i + 1 of 8 codes of a column (e2m1: a dword; fp8: two) in fp32.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
@@ -492,14 +502,7 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
     for (int u = 0; u < Cfg::B_LOADS; ++u) {
       const int q = Cfg::B_LOADS * wave + u;
       const void *src;
-      if constexpr (WQ != WQ_NONE) { // rows 8 q .. +7 of the batch's 64 or 128
-        const int row = 8 * q + (lane >> 3);
-        const int c = (lane & 7) ^ Cfg::swz(row);
-        const int64_t k = (Cfg::FP4 ? k0 / 2 : k0) + row, n = n0 + 16 * c;
-        src = reinterpret_cast<const uint8_t *>(p.B) + k * p.ldb + n;
-        if (mask && (!live || k >= (Cfg::FP4 ? p.K / 2 : p.K) || n >= p.N))
-          src = tx_zero_chunk;
-      } else if constexpr (BT) {
+      if constexpr (BT) {
         const int r = 4 * q + (lane >> 4);
         const int c = (lane & 15) ^ (r & 15);
         const int64_t n = n0 + r, k = k0 + 8 * c;
@@ -601,57 +604,12 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
     const int b = batch(i);
     const bool tail = b >= p.k_main_batches;
     const int64_t k0 = (int64_t)b * kDec16BatchK;
-    uint32_t sc[2][4]; // WQ: the scale byte of block jj at K step ks
-    bool soft = false;
-    if constexpr (WQ != WQ_NONE) {
-      uint32_t v[2][3];
-      const uint32_t at = (uint32_t)(i % Cfg::SEG_B) * Cfg::GPB;
-      decwq_read_scales(xs[0] + at, xs[1] + at, v);
-      bool odd = false;
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const uint32_t d0 = __builtin_amdgcn_alignbyte(v[jj][1], v[jj][0], mis[jj]);
-        const uint32_t d1 = __builtin_amdgcn_alignbyte(v[jj][2], v[jj][1], mis[jj]);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          if constexpr (WQ == WQ_NV_E2M1) { // group 2 ks + G / 2 of the batch's 8
-            sc[jj][ks] = ((ks < 2 ? d0 : d1) >> (16 * (ks & 1) + 8 * (G >> 1))) & 0xff;
-            if (tail && b * Cfg::GPB + 2 * ks + (G >> 1) >= p.sb_ld)
-              sc[jj][ks] = 0x38;
-          } else {
-            sc[jj][ks] = (d0 >> (8 * ks)) & 0xff;
-            if (tail && b * Cfg::GPB + ks >= p.sb_ld)
-              sc[jj][ks] = 127;
-            odd = odd || sc[jj][ks] - kHwScaleLo > kHwScaleHi - kHwScaleLo;
-          }
-        }
-      }
-      if constexpr (WQ != WQ_NV_E2M1)
-        soft = __any(odd);
-    }
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
       constexpr int T4 = T < 4 ? T : 4; // tiles the first read block brings
       i32x4_t bq[JB][2];
       i32x4_t a4[2][T4];
-      if constexpr (WQ != WQ_NONE) {
-        constexpr int NB = Cfg::FP4 ? 1 : 2;
-        v2i_t w[2][NB];
-        const uint32_t o = base + pr * (Cfg::FP4 ? 4096 : 8192);
-        decwq_read_pair<T4, NB>(o + wq_b[0], o + wq_b[1], base + a_k[2 * pr], base + a_k[2 * pr + 1],
-                                w, a4);
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const uint32_t w0 = Cfg::FP4 ? (h ? w[jj][0].y : w[jj][0].x) : w[jj][NB - 1 ? h : 0].x;
-            const uint32_t w1 = Cfg::FP4 ? 0 : w[jj][NB - 1 ? h : 0].y;
-            if (soft)
-              bq[jj][h] = decwq_upcast<WQ, false>(w0, w1, sc[jj][2 * pr + h]);
-            else
-              bq[jj][h] = decwq_upcast<WQ, true>(w0, w1, sc[jj][2 * pr + h]);
-          }
-      } else if constexpr (BT) {
+      if constexpr (BT) {
         dec16_read_pair_kmajor<T4>(base + bk_k[0][2 * pr], base + bk_k[0][2 * pr + 1],
                                    base + a_k[2 * pr], base + a_k[2 * pr + 1], bq[0], a4);
         if constexpr (JB == 2)
@@ -690,7 +648,7 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj)
           bf[jj] = bq[jj][h];
-        if (!WQ && tail) { // (WQ: K is a multiple of 16, no chunk of A crosses it)
+        if (tail) {
           const int64_t k = k0 + 32 * (2 * pr + h) + 8 * G;
 #pragma unroll
           for (int t = 0; t < T; ++t)
@@ -710,10 +668,168 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
     }
   };
 
+  // WQ loads: as above, but each lane keeps the addresses of its loads of the
+  // next batch and adds a step to them (0 where it reads the zero chunk: rows of
+  // A >= M, columns of B >= N); batches are issued in order.
+  const uint8_t *wq_src[Cfg::VPB];
+  int64_t wq_step[Cfg::VPB];
+  auto wq_row = [&](int u) { // load u's row of B's batch
+    return 8 * (Cfg::B_LOADS * wave + u) + (lane >> 3);
+  };
+  auto wq_chunk = [&](int u) { // load u's 16-byte chunk of A's batch
+    const int r = 4 * (Cfg::A_LOADS * wave + u) + (lane >> 4);
+    return (lane & 15) ^ (r & 15);
+  };
+  if constexpr (WQ != WQ_NONE) {
+    constexpr int ROWS = Cfg::FP4 ? 64 : 128;
+#pragma unroll
+    for (int u = 0; u < Cfg::B_LOADS; ++u) { // rows 8 q .. +7 of the batch's 64 or 128
+      const int row = wq_row(u), c = (lane & 7) ^ Cfg::swz(row);
+      const int64_t k = (int64_t)b_begin * ROWS + row, n = n0 + 16 * c;
+      const bool in = n < p.N;
+      wq_src[u] = in ? reinterpret_cast<const uint8_t *>(p.B) + k * p.ldb + n
+                     : (const uint8_t *)tx_zero_chunk;
+      wq_step[u] = in ? ROWS * p.ldb : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < Cfg::A_LOADS; ++u) {
+      const int r = 4 * (Cfg::A_LOADS * wave + u) + (lane >> 4);
+      const int64_t k = (int64_t)b_begin * kDec16BatchK + 8 * wq_chunk(u);
+      const bool in = r < p.M;
+      wq_src[Cfg::B_LOADS + u] =
+          in ? reinterpret_cast<const uint8_t *>(p.A + (int64_t)r * p.lda + k)
+             : (const uint8_t *)tx_zero_chunk;
+      wq_step[Cfg::B_LOADS + u] = in ? kDec16BatchK * 2 : 0;
+    }
+  }
+  auto wq_issue = [&](int i, uint8_t *slot) {
+    const int b = b_begin + i;
+    auto load = [&](int u, const void *src) {
+      if (u < Cfg::B_LOADS) // B is read once
+        dma16_stream(src, (lds_void *)(slot + (Cfg::B_LOADS * wave + u) * 1024));
+      else // A: re-read by every strip
+        dma16(src, (lds_void *)(slot + Cfg::A_OFF +
+                                (Cfg::A_LOADS * wave + u - Cfg::B_LOADS) * 1024));
+    };
+    if (i < nb && b < p.k_main_batches) {
+#pragma unroll
+      for (int u = 0; u < Cfg::VPB; ++u)
+        load(u, wq_src[u]);
+    } else { // past the split: zeros; K's end: rows or chunks past K too
+#pragma unroll
+      for (int u = 0; u < Cfg::VPB; ++u) {
+        const int64_t k = (int64_t)b * kDec16BatchK +
+                          (u < Cfg::B_LOADS ? (Cfg::FP4 ? 2 : 1) * wq_row(u)
+                                            : 8 * wq_chunk(u - Cfg::B_LOADS));
+        load(u, i < nb && k < p.K ? wq_src[u] : (const uint8_t *)tx_zero_chunk);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < Cfg::VPB; ++u)
+      wq_src[u] += wq_step[u];
+  };
+  auto wq_consume = [&](const uint8_t *slot, int i) {
+    constexpr int T4 = T < 4 ? T : 4, NB = Cfg::FP4 ? 2 : 4;
+    const uint32_t base = lds_addr(slot);
+    const int b = b_begin + i;
+    const bool tail = b >= p.k_main_batches;
+    const uint32_t at = (uint32_t)(i % Cfg::SEG_B) * Cfg::GPB;
+    uint32_t v[2][3];
+    v2i_t w[2][NB];
+    i32x4_t a[4][T4];
+    decwq_read<T4, NB>(xs[0] + at, xs[1] + at, base + wq_b[0], base + wq_b[1], base + a_k[0],
+                       base + a_k[1], base + a_k[2], base + a_k[3], v, w, a);
+    uint32_t sc[2][4]; // the scale byte of block jj at K step ks
+    bool odd = false;
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      uint32_t d0 = __builtin_amdgcn_alignbyte(v[jj][1], v[jj][0], mis[jj]);
+      uint32_t d1 = __builtin_amdgcn_alignbyte(v[jj][2], v[jj][1], mis[jj]);
+      if (tail) { // groups at or past the row's last
+        const int left = p.sb_ld - b * Cfg::GPB; // > 0
+        const uint32_t unit = WQ == WQ_NV_E2M1 ? 0x38383838u : 0x7f7f7f7fu;
+        const uint32_t k0m = left >= 4 ? ~0u : (1u << (8 * left)) - 1;
+        const uint32_t k1m = left >= 8 ? ~0u : left <= 4 ? 0u : (1u << (8 * (left - 4))) - 1;
+        d0 = (d0 & k0m) | (unit & ~k0m);
+        d1 = (d1 & k1m) | (unit & ~k1m);
+      }
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        if constexpr (WQ == WQ_NV_E2M1) { // group 2 ks + G / 2 of the batch's 8
+          sc[jj][ks] = ((ks < 2 ? d0 : d1) >> (16 * (ks & 1) + 8 * (G >> 1))) & 0xff;
+        } else {
+          sc[jj][ks] = (d0 >> (8 * ks)) & 0xff;
+          odd = odd || sc[jj][ks] - kHwScaleLo > kHwScaleHi - kHwScaleLo;
+        }
+      }
+    }
+    auto products = [&](auto hw) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        i32x4_t bf[2];
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj) {
+          const uint32_t w0 = Cfg::FP4 ? (ks & 1 ? w[jj][ks / 2].y : w[jj][ks / 2].x)
+                                       : w[jj][NB == 4 ? ks : 0].x;
+          const uint32_t w1 = Cfg::FP4 ? 0 : w[jj][NB == 4 ? ks : 0].y;
+          bf[jj] = decwq_upcast<WQ, decltype(hw)::value>(w0, w1, sc[jj][ks]);
+        }
+#pragma unroll
+        for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+          for (int t = 0; t < T4; ++t)
+            acc[jj][t] = mfma16x16x32<BF>(bf[jj], a[ks][t], acc[jj][t]);
+        if constexpr (T > 4) { // slices past 64 rows: tiles 4 .. T - 1, two steps a read
+          if (ks & 1)
+            continue;
+          i32x4_t am[2][T - 4], bn[2];
+          dec16_read_more<T - 4>(base + a_k[ks], base + a_k[ks + 1], am);
+#pragma unroll
+          for (int jj = 0; jj < 2; ++jj) {
+            const uint32_t w0 = Cfg::FP4 ? w[jj][ks / 2].y : w[jj][NB == 4 ? ks + 1 : 0].x;
+            const uint32_t w1 = Cfg::FP4 ? 0 : w[jj][NB == 4 ? ks + 1 : 0].y;
+            bn[jj] = decwq_upcast<WQ, decltype(hw)::value>(w0, w1, sc[jj][ks + 1]);
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+              for (int t = 4; t < T; ++t)
+                acc[jj][t] = mfma16x16x32<BF>(h ? bn[jj] : bf[jj], am[h][t - 4], acc[jj][t]);
+        }
+      }
+    };
+    if (WQ != WQ_NV_E2M1 && __any(odd)) // one branch a batch
+      products(std::false_type());
+    else
+      products(std::true_type());
+  };
+
   // Prologue: S - 1 batches in flight; batch i uses slot i % S.  (WQ: the
   // first segment's scales before them.)
-  if constexpr (WQ != WQ_NONE)
+  if constexpr (WQ != WQ_NONE) {
     stage_scales(0);
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s)
+      wq_issue(s, ring + s * SLOT);
+    // The loop below, not unrolled: a batch's code holds both upcasts.
+    int s = 0, sl = S - 1;
+    for (int i = 0; i < nb; ++i) {
+      if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
+        asm volatile("s_barrier" ::: "memory");
+        stage_scales(i);
+        wait_vmcnt<0>();
+      }
+      wait_vmcnt<(S - 2) * Cfg::VPB>();
+      asm volatile("s_barrier" ::: "memory");
+      wq_issue(i + S - 1, ring + sl * SLOT);
+      wq_consume(ring + s * SLOT, i);
+      s = s + 1 == S ? 0 : s + 1;
+      sl = sl + 1 == S ? 0 : sl + 1;
+    }
+    goto k_loop_done;
+  }
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
     issue(s, ring + s * SLOT);
@@ -728,13 +844,6 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
       const int i = i0 + s;
       if (i >= nb)
         goto k_loop_done;
-      if constexpr (WQ != WQ_NONE) {
-        if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
-          asm volatile("s_barrier" ::: "memory");
-          stage_scales(i);
-          wait_vmcnt<0>();
-        }
-      }
       wait_vmcnt<(S - 2) * Cfg::VPB>();
       asm volatile("s_barrier" ::: "memory");
       issue(i + S - 1, ring + ((s + S - 1) % S) * SLOT);
