@@ -39,11 +39,13 @@
 // for 16 bits K steps 0 and 1 of 32 elements).  MFMA roles are swapped as on
 // the other tiles: lane l ends with C row l % 16 at 4 consecutive columns.
 //
-// Sums: with fp32 C the accumulators are emptied into a second set every 8
-// steps, so no chain of additions is longer than 8 steps or their number.  A
-// range here is up to 8 times the one the 256x256 tile's own split would take,
-// and one chain over it doubled the error (bf16 860x1856x4928 against 64 bits:
-// 3.0e-7, that tile 1.5e-7, this 1.3e-7).
+// Sums: with fp32 C from 16-bit or e2m1 operands the accumulators are emptied
+// into a second set every 8 steps, so no chain of additions is longer than 8
+// steps or their number.  A range here is up to 8 times the one the 256x256
+// tile's own split would take, and one chain over it doubled the error (bf16
+// 860x1856x4928 against 64 bits: 3.0e-7, that tile 1.5e-7, this 1.3e-7).  fp8
+// operands' error is the MFMA's own sum of 32 products (1.29e-5 either way,
+// K = 2048 to 8192), and there the second set costs 6 % of the time.
 //
 // The plan is the 256x256 tile's (TX_FLAG_TILES_128): its block_k is one ring
 // step.  Split-K ranges are whole steps; a range's partial C is 32-bit, summed
@@ -67,7 +69,7 @@ template <int OP, int EPI, int FA = 0, int FB = 0, bool BT = false> struct GemmR
   static constexpr bool F4 = MX && FA == 4;
   static constexpr bool W32 = EPI == EPI_F32 || EPI == EPI_I32 || EPI == EPI_BLOCK128_F32 ||
                               EPI == EPI_MX_F32; // 32-bit C
-  static constexpr bool CHAINS = W32 && !INT; // sums in two levels
+  static constexpr bool CHAINS = W32 && (B16 || F4); // sums in two levels
   static constexpr int SG = F4 ? 8 : 4, NSD = F4 ? 4 : 2, RS = 4 * NSD; // MX (gemm8_w4.h)
   static constexpr int A_BYTES = 16384, SA_OFF = 32768;
   static constexpr int SB_OFF = SA_OFF + (MX ? BM * RS : SCALED ? BM * 4 : 0);

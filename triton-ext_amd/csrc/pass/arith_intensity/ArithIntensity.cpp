@@ -45,7 +45,7 @@ struct Tile {
 //   W8A8 128x128:     M = 512 N = K = 8192 40 / 41, 3072^3 50 / 46;
 //   fp8 block-scaled  256: M = 1024 N = K = 7168 73 / 77, 128: 79 / 80, M = 512 40 / 43;
 //   mxfp8             256: M = 1024 N = 8192 K = 4096 53 / 54, 128: 53 / 52;
-//   mxfp4             256: the same shape 33 / 34, 128: 36 / 36.
+//   mxfp4             256: the same shape 33 / 34, 128: 36 / 39; 2048x2800x8192 61 / 56, 66 / 61.
 struct Rate {
   double launch, per, s0, s1;
   int occ; // workgroups a CU
@@ -55,7 +55,7 @@ constexpr Rate k64x16{2.0, 0.5, 0.33, 0.20, 4}, k128dma{3.0, 0.5, 0.90, 0.40, 2}
 constexpr Rate k256x8{5.0, 3.0, 1.05, 0.70, 1}, k128x8{4.0, 2.2, 0.33, 0.22, 1};
 constexpr Rate k128f8b{4.0, 2.2, 0.40, 0.27, 1};
 constexpr Rate k256mx8{5.0, 3.0, 1.15, 0.55, 1}, k128mx8{4.0, 2.2, 0.40, 0.28, 1};
-constexpr Rate k256mx4{5.0, 3.0, 1.20, 0.90, 1}, k128mx4{4.0, 2.2, 0.48, 0.37, 1};
+constexpr Rate k256mx4{5.0, 3.0, 1.20, 0.90, 1}, k128mx4{4.0, 2.2, 0.53, 0.43, 1};
 
 double estimate(const Rate &r, int64_t bm, int64_t bn, int64_t bk, int64_t split, int64_t M,
                 int64_t N, int64_t K) {
@@ -66,8 +66,14 @@ double estimate(const Rate &r, int64_t bm, int64_t bn, int64_t bk, int64_t split
     return r.per + steps * (r.s0 + r.s1 * (wgs < kCUs ? (double)wgs / kCUs : 1.0));
   };
   double us = r.launch + (double)full * round(cap) + (rem ? round(rem) : 0.0);
-  if (split > 1) // the reduction, its partials written and read at about 6 TB/s
-    us += 3.0 + 8.0 * (double)split * (double)M * (double)N / 6e6;
+  // The reduction: its partials written and read at about 6 TB/s from a whole
+  // round of workgroups; those of a part of one are mostly hidden (fp8
+  // 2048x2800x8192, 176 workgroups: 63 us in all, of which the ranges take 57;
+  // bf16 1000x8192x4096, 256: 78 of which 57).
+  if (split > 1) {
+    const double f = n < kCUs ? (double)n / kCUs : 1.0;
+    us += 3.0 + f * f * 8.0 * (double)split * (double)M * (double)N / 6e6;
+  }
   return us;
 }
 
