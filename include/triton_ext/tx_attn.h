@@ -64,11 +64,10 @@ typedef struct tx_attn_desc {
    * for fp8 e5m2); 0 = default (128, 64).  The
    * blocks fix the on-band split (causal_start = start_m * BLOCK_M) and the
    * online softmax's key blocks, so they select the rounding of the result
-   * exactly as the tutorial's config does -- but for fp16 / bf16 at 128 x 64
-   * where the programs leave CUs idle: groups of waves then run parts of a
-   * row's key blocks, each with its own running maximum, and their sums are
-   * merged in fp32 (the same precision; p is rounded against a group's
-   * maximum). */
+   * exactly as the tutorial's config does.  With both left 0, at fp16 / bf16,
+   * head_dim <= 64 and few programs (tx_attn_plan.key_groups), 4 groups of waves
+   * run parts of a row's key blocks and their fp32 sums are merged: p is
+   * rounded as in one group, only the order of the fp32 sums differs. */
   int32_t block_m, block_n;
 } tx_attn_desc;
 
@@ -79,7 +78,10 @@ typedef struct tx_attn_plan {
   float qk_scale;    /* sm_scale * 1.44269504, in fp32 as the kernel has it */
   int32_t m_blocks;  /* N_CTX / block_m programs per (z, h) */
   int32_t grid_x, block_threads;
-  int32_t reserved;
+  int32_t key_groups; /* groups of waves that split a row's keys: 4, or 0, one group (and a
+                       * plan may be set to 0).  4 with the blocks left 0, fp16 / bf16,
+                       * head_dim <= 64, N_CTX >= 256 and grid_x <= 64 (head_dim <= 32 and
+                       * N_CTX >= 1024: grid_x <= 128) */
 } tx_attn_plan;
 
 /* Validate `desc` and fill `plan`.  TX_ERR_UNSUPPORTED unless dtype is

@@ -17,6 +17,7 @@ against torch's float8_e5m2 cast, and the interpreter's own converter, pinned
 bit for bit against the interpreter's cast (tests/golden/e5m2_cast_interp.npz);
 the attention fixtures attn_fwd_fp8_* pin the forward with the latter.
 """
+import ctypes
 import glob
 import os
 
@@ -219,6 +220,27 @@ def test_kernel_split_is_the_loop_split_plan():
         s = tx.loop_split_plan(0, N, 64, tx.CMP_SGE, start_m * 128)
         assert s.midp == start_m * 128
         assert s.first_trips == start_m * 2 and s.second_trips == (N - start_m * 128) // 64
+
+
+def test_attn_plan_key_groups():
+    """The plan says when groups of waves split a row's keys (few programs, blocks left to the
+    planner); a block asked for has one group, and a launch takes the plan's own number or 0."""
+    def groups(Z, H, N, D, **kw):
+        return tx.attn_plan(Z, H, N, D, True, 0.5, **kw).key_groups
+    assert groups(1, 8, 1024, 64) == 4 and groups(1, 1, 8192, 16, dtype=tx.BF16) == 4
+    assert groups(1, 8, 1024, 64, block=(128, 64)) == groups(1, 8, 1024, 64, block=(64, 64)) == 0
+    assert groups(1, 16, 1024, 128) == 0 and groups(1, 8, 1024, 64, dtype=tx.F8E5M2) == 0
+    assert groups(1, 64, 128, 64) == 0 and groups(1, 32, 256, 64) == 4 and groups(1, 33, 256, 64) == 0
+    assert groups(1, 16, 1024, 32) == 4 and groups(1, 17, 1024, 32) == 0
+    assert groups(1, 32, 512, 32) == 0 and groups(1, 16, 1024, 64) == 0
+    if not tx.load().tx_device_available():  # (dummy pointers: never on a GPU)
+        a = ctypes.c_void_p(1 << 20)
+        for made, edited, want in ((4, 0, tx.ERR_NO_DEVICE), (4, 4, tx.ERR_NO_DEVICE),
+                                   (4, 2, tx.ERR_INVALID), (0, 4, tx.ERR_INVALID)):
+            p = tx.attn_plan(1, 8 if made else 65, 1024, 64, True, 0.5)
+            assert p.key_groups == made
+            p.key_groups = edited
+            assert tx.load().tx_attn_fwd_launch(ctypes.byref(p), a, a, a, a, a, None) == want
 
 
 def test_attn_plan():

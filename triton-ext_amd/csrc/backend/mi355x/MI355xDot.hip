@@ -1308,35 +1308,27 @@ int attnStrides(const tx_attn_desc &d, int64_t &sz, int64_t &sh, int64_t &sm,
   return TX_OK;
 }
 
-} // namespace
-
-namespace {
-
-// How a plan's keys are split among groups of waves (attn_fwd.h, KS): 0 not
-// at all, 1 in 128 rows x 2 groups, 2 64 x 2, 3 32 x 4.  programs: row blocks of
-// 128 over all heads.  bf16, us without / with the split, causal, one MI355X:
-//   64 programs or fewer, 4 key blocks or more, head dim <= 64 (32 x 4): N = 1024 12.2 / 6.9
-//     (head dim 32), 15.2 / 9.5 (64); 8192 keys of one head 73.8 / 27.4, 87.9 / 41.0
-//   128 programs or fewer (64 x 2): N = 1024 12.1 / 9.1 (32), 15.1 / 11.7 (64),
-//     22.0 / 18.2 (128); N = 128 4.6 / 4.1, 5.9 / 5.2, 8.2 / 7.2; at 192 they lose
-//   256 or fewer, 16 key blocks or more (128 x 2): N = 4096 39.2 / 30.6, 47.1 / 39.7,
-//     68.1 / 59.1; N = 1024 12.3 / 10.7, 15.6 / 14.4, 22.4 / 21.3
-//   head dim <= 32 past that (its softmax leaves the matrix cores idle): 512 programs
-//     31.9 / 28.9, 1024 causal 55.1 / 46.1 (without the mask 58.0 / 57.3: left alone)
-// e5m2 keeps one group: p is rounded to two bits against the running maximum, and a
-// group's own maximum rounds it differently (o changes by 4-7%).
-int attnKs(const tx_attn_plan &p) {
+// The number of groups of waves a row's keys are split among (attn_fwd.h, KS)
+// where the caller left the blocks to the planner: 4 groups over 32 rows, or 0,
+// not at all.  programs: row blocks of 128 over all heads.  bf16, us without /
+// with the split, causal and then not, one MI355X:
+//   64 programs or fewer: 256 keys 5.6 / 5.2, 5.2 / 4.9 (head dim 16), 7.6 / 7.1, 6.7 / 6.6 (64);
+//     1024 12.3 / 9.1, 11.8 / 8.9 (32), 15.5 / 12.1, 14.4 / 11.6 (64); 8192 73.8 / 38.8,
+//     74.9 / 39.0 (32), 89.3 / 56.2, 86.9 / 56.6 (64); 128 keys lose (5.3 / 6.1, 64)
+//   65 to 128: 1024 keys 12.3 / 11.9, 12.0 / 11.8, 4096 39.6 / 26.7, 38.8 / 31.3 (32);
+//     head dim 64 loses (1024 15.5 / 17.9, 8192 90.0 / 97.6)
+//   256: 1024 keys 12.6 / 17.3, 8192 74.6 / 79.5 (32)
+// Head dim 128 has no such form (its slots would take 256 KiB), and e5m2 keeps one
+// group: p of two bits moves with the last bits of the maximum.
+int attnKeyGroups(const tx_attn_plan &p) {
   const tx_attn_desc &d = p.desc;
-  if (d.block_m != 128 || d.block_n != 64 || d.dtype == TX_F8E5M2 || d.head_dim > 128)
+  if (d.block_m != 128 || d.block_n != 64 || d.dtype == TX_F8E5M2 || d.head_dim > 64)
     return 0;
   const int64_t programs = p.grid_x, blocks = d.N_CTX / 64;
-  if (programs <= 64 && d.head_dim <= 64 && blocks >= 4)
-    return 3;
-  if (programs <= 128)
-    return 2;
-  if (blocks >= 16 && (programs <= 256 || (d.head_dim <= 32 && (d.causal || programs <= 512))))
-    return 1;
-  return 0;
+  return (programs <= 64 && blocks >= 4) ||
+                 (programs <= 128 && blocks >= 16 && d.head_dim <= 32)
+             ? 4
+             : 0;
 }
 
 } // namespace
@@ -1360,6 +1352,7 @@ extern "C" TX_API int tx_attn_fwd_plan(const tx_attn_desc *desc, tx_attn_plan *p
       d.head_dim != 256)
     return fail(TX_ERR_UNSUPPORTED, "head_dim %d: 16, 32, 64, 128 and 256 are implemented",
                 d.head_dim);
+  const bool own_blocks = d.block_m == 0 && d.block_n == 0;
   if (d.block_m == 0) d.block_m = 128;
   if (d.block_n == 0) d.block_n = 64;
   if ((d.block_m != 64 && d.block_m != 128) || (d.block_n != 32 && d.block_n != 64))
@@ -1387,6 +1380,7 @@ extern "C" TX_API int tx_attn_fwd_plan(const tx_attn_desc *desc, tx_attn_plan *p
   plan->m_blocks = (int32_t)(d.N_CTX / d.block_m);
   plan->grid_x = (int32_t)programs;
   plan->block_threads = d.block_m / 32 * 64; // one wave per 32 query rows
+  plan->key_groups = own_blocks ? attnKeyGroups(*plan) : 0;
   return TX_OK;
 }
 
@@ -1414,7 +1408,8 @@ extern "C" TX_API int tx_attn_fwd_launch(const tx_attn_plan *plan, const void *q
     if (std::memcmp(&again.desc, &plan->desc, sizeof again.desc) != 0 ||
         again.flops != plan->flops || again.bytes != plan->bytes ||
         again.qk_scale != plan->qk_scale || again.m_blocks != plan->m_blocks ||
-        again.grid_x != plan->grid_x || again.block_threads != plan->block_threads)
+        again.grid_x != plan->grid_x || again.block_threads != plan->block_threads ||
+        (plan->key_groups != 0 && plan->key_groups != attnKeyGroups(*plan)))
       return fail(TX_ERR_INVALID, "the plan does not follow from its descriptor");
   }
   if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
@@ -1453,10 +1448,9 @@ extern "C" TX_API int tx_attn_fwd_launch(const tx_attn_plan *plan, const void *q
                                      : 4;
   const AttnFn fn = d.dtype == TX_F8E5M2 ? kAttn8[c][hd][bm64][bn32]
                                          : kAttn[c][hd][d.dtype == TX_BF16][bm64][bn32];
-  if (const int ks = attnKs(*plan)) {
-    const int bm = ks == 1 ? 128 : ks == 2 ? 64 : 32, groups = ks == 3 ? 4 : 2;
-    hipLaunchKernelGGL(kAttnKs[ks - 1][c][hd][d.dtype == TX_BF16],
-                       dim3(plan->grid_x * (128 / bm)), dim3(bm * 2 * groups), 0, s, a);
+  if (plan->key_groups) {
+    hipLaunchKernelGGL(kAttnKs[c][hd][d.dtype == TX_BF16], dim3(plan->grid_x * 4),
+                       dim3(64 * plan->key_groups), 0, s, a);
   } else {
     hipLaunchKernelGGL(fn, dim3(plan->grid_x), dim3(plan->block_threads), 0, s, a);
   }

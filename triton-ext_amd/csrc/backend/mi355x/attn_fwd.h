@@ -208,19 +208,16 @@ template <int HD, bool BF, int BM_ = 128, int BN_ = 64> struct AttnFwd {
     }
   }
 
-  // Softmax of one block (the tutorial's arithmetic) for the lane's query
-  // row m, keys n0 + 8 (r/4) + 4 g + r%4 of each 32-key block: updates m_i and
-  // l_i, rescales acc by alpha and returns P as MFMA B operands (key chunk c
-  // = registers 8 (c%2) .. +7 of key block c/2).  MASK: on-band form.
+  // Running maximum of the lane's query row m after one block, keys n0 + 8
+  // (r/4) + 4 g + r%4 of each 32-key block.  MASK: on-band form, which scales
+  // and masks s in place.
   template <bool MASK>
-  __device__ __forceinline__ static void softmax(f16v (&s)[BN / 32], int n0, int m,
-                                                 float qk_scale, f16v (&acc)[D / 32],
-                                                 float &m_i, float &l_i, h8 (&pf)[BN / 16]) {
+  __device__ __forceinline__ static float row_max(f16v (&s)[BN / 32], int n0, int m,
+                                                  float qk_scale, float m_i) {
     const int g = (threadIdx.x & 63) >> 5;
-    float m_ij;
+    float mx = -INFINITY;
     if constexpr (MASK) {
       // qk = qk * qk_scale + where(m >= n, 0, -1e6); m_ij = max(m_i, rowmax(qk))
-      float mx = -INFINITY;
 #pragma unroll
       for (int b = 0; b < BN / 32; ++b)
 #pragma unroll
@@ -232,27 +229,35 @@ template <int HD, bool BF, int BM_ = 128, int BN_ = 64> struct AttnFwd {
           s[b][r] = t;
           mx = fmaxf(mx, t);
         }
-      m_ij = fmaxf(m_i, xmax(mx));
-#pragma unroll
-      for (int b = 0; b < BN / 32; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s[b][r] = __builtin_amdgcn_exp2f(s[b][r] - m_ij);
+      return fmaxf(m_i, xmax(mx));
     } else {
-      // m_ij = max(m_i, rowmax(qk) * qk_scale); qk = qk * qk_scale - m_ij
-      float mx = -INFINITY;
+      // m_ij = max(m_i, rowmax(qk) * qk_scale)
 #pragma unroll
       for (int b = 0; b < BN / 32; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           mx = fmaxf(mx, s[b][r]);
-      m_ij = fmaxf(m_i, xmax(mx) * qk_scale);
-#pragma unroll
-      for (int b = 0; b < BN / 32; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          s[b][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r], qk_scale, -m_ij));
+      return fmaxf(m_i, xmax(mx) * qk_scale);
     }
+  }
+
+  // Softmax of one block (the tutorial's arithmetic): updates m_i and
+  // l_i, rescales acc by alpha and returns P as MFMA B operands (key chunk c
+  // = registers 8 (c%2) .. +7 of key block c/2).
+  template <bool MASK>
+  __device__ __forceinline__ static void softmax(f16v (&s)[BN / 32], int n0, int m,
+                                                 float qk_scale, f16v (&acc)[D / 32],
+                                                 float &m_i, float &l_i, h8 (&pf)[BN / 16]) {
+    const float m_ij = row_max<MASK>(s, n0, m, qk_scale, m_i);
+#pragma unroll
+    for (int b = 0; b < BN / 32; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if constexpr (MASK)
+          s[b][r] = __builtin_amdgcn_exp2f(s[b][r] - m_ij);
+        else // qk = qk * qk_scale - m_ij
+          s[b][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r], qk_scale, -m_ij));
+      }
     float l_ij = 0.f;
 #pragma unroll
     for (int b = 0; b < BN / 32; ++b)
@@ -368,15 +373,22 @@ template <int HD, bool BF, int BM_ = 128, int BN_ = 64> struct AttnFwd {
 // KS > 1: KS groups of waves share the workgroup's query rows, each running
 // 1 / KS of the key blocks through LDS slots of its own; at the end the other
 // groups' (m, l, acc) go through LDS and the first one merges them in order,
-// acc = acc_0 2^(m_0 - m) + acc_1 2^(m_1 - m) and l alike, in fp32.  A launch of
-// few workgroups is the serial chain of its longest row block, whose waves
-// spend most of a block in the softmax: fewer rows a workgroup with more groups
-// use the idle CUs and cut the chain (the times stand at the launch's choice).
-// What bounds it then: the softmax's VALU work at head dims up to 64, the LDS
-// reads of K and V (every wave reads all of its group's blocks) at 128.
-// The groups after the first start from m = -FLT_MAX, l = 0 rather than -inf, 1:
-// a first block of scores that are all -inf then adds nothing, as it would
-// after the first group's blocks.
+// acc = acc_0 2^(m_0 - m) + acc_1 2^(m_1 - m) and l alike, in fp32.  p must be
+// rounded against the row's running maximum as in one group (a maximum of the
+// group's own keys rounds every p differently, and sums values of V that the
+// row's earlier keys would have weighted 0, past fp32's range if they are
+// large), so a first pass takes the maximum of every group's keys (Q K^T and
+// the maximum alone, about 0.4 of a block's time), and a group starts from
+// that of the groups before it with l = 0.  Then only the order of the fp32
+// sums differs from one group's: o agrees to 7e-5 (bf16, 2-norm), M to 2e-6.
+// A launch of few workgroups is the serial chain of its longest row block,
+// whose waves spend most of a block in the softmax: 32 rows a workgroup with 4
+// groups use the idle CUs and cut that chain (bf16 causal, 8192 keys of one head
+// of 64: 89.3 -> 56.2 us, of 32: 73.8 -> 38.8; (1, 8, 1024, 64) 15.5 -> 12.1).
+// Two groups of 64 or 128 rows gain too little for the first pass (128
+// programs of (1, 16, 1024, D): head dim 64 15.5 -> 15.6, 128 22.3 -> 23.4, where
+// the LDS reads of K and V bound the block), so there is no such form.  What
+// bounds it: the softmax's VALU work.
 template <bool CAUSAL, class A, int KS = 1>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[KS * 4 * A::TILE];
@@ -411,10 +423,15 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   // LoopSplit form of the K/V loop (keys [0, N_CTX), predicate start_n >=
   // causal_start): unmasked blocks [0, n_main), masked [n_main, n_end).
   // N_CTX and causal_start are multiples of BM, itself a multiple of BN.
-  const int causal_start = CAUSAL ? start_m * A::BM : p.N_CTX;
+  // (KS > 1: causal_start is that of the 128 rows the block lies in, and the
+  // last block the one that holds the workgroup's own last row.)
+  const int causal_start = !CAUSAL  ? p.N_CTX
+                           : KS > 1 ? start_m * A::BM / 128 * 128
+                                    : start_m * A::BM;
   const int all_main = causal_start / A::BN;
-  const int all_end =
-      CAUSAL ? (causal_start + A::BM + (A::BM < A::BN ? A::BN - 1 : 0)) / A::BN : all_main;
+  const int all_end = !CAUSAL  ? all_main
+                      : KS > 1 ? (start_m * A::BM + A::BM + A::BN - 1) / A::BN
+                               : (causal_start + A::BM) / A::BN;
   // This group's blocks: j0 + [0, n_main) unmasked, j0 + [n_main, n_end) masked;
   // every group runs n_it iterations (its barriers are the workgroup's).
   [[maybe_unused]] int n_it = all_end, j0 = 0;
@@ -427,14 +444,54 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   }
 
   float m_i = -INFINITY, l_i = 1.0f;
-  if (KS > 1 && kg > 0) {
-    m_i = -3.402823466e38f;
-    l_i = 0.0f;
-  }
   typename A::f16v acc[A::D / 32], s[A::BN / 32];
 #pragma unroll
   for (int bd = 0; bd < A::D / 32; ++bd)
     acc[bd] = typename A::f16v{};
+
+  // Whether this wave computes block j of the row at all.  On-band blocks whose
+  // keys all lie past its 32 rows add exactly nothing (p = 0, alpha = 1, as for
+  // the blocks past the diagonal): it skips their softmax and P V.
+  auto live = [&](int j) { return j * A::BN <= start_m * A::BM + 32 * wave + 31; };
+
+  // First pass of KS > 1: the running maximum at the end of each group but the
+  // last, pairs of K blocks in slots 0, 1 and 2, 3 (V's).
+  if constexpr (KS > 1) {
+    const bool need = kg + 1 < KS;
+    auto issue_pair = [&](int j, int slot) {
+      for (int i = 0; i < 2; ++i)
+        if (need && j + i < n_end)
+          A::issue_k(rk, ko, p.k_sm, j0 + j + i, k_lds + (slot + i) * A::TILE, wave);
+    };
+    float mx = -INFINITY;
+    auto pair_max = [&](int j, auto slot) {
+      constexpr int SL = decltype(slot)::value;
+      issue_pair(j + 2, 2 - SL);
+      auto one = [&](int jj, auto sl) {
+        if (!need || jj >= n_end)
+          return;
+        A::template qk<decltype(sl)::value>(bs, qf, s);
+        if (jj < n_main)
+          mx = A::template row_max<false>(s, (j0 + jj) * A::BN, m, p.qk_scale, mx);
+        else if (live(j0 + jj))
+          mx = A::template row_max<true>(s, (j0 + jj) * A::BN, m, p.qk_scale, mx);
+      };
+      one(j, slot);
+      one(j + 1, std::integral_constant<int, SL + 1>());
+      __builtin_amdgcn_s_waitcnt(0x7 << 4); // vmcnt(0)
+      __syncthreads();
+    };
+    issue_pair(0, 0);
+    __builtin_amdgcn_s_waitcnt(0x7 << 4);
+    __syncthreads();
+    for (int j = 0; j < n_it; j += 4) {
+      pair_max(j, std::integral_constant<int, 0>());
+      if (j + 2 < n_it)
+        pair_max(j + 2, std::integral_constant<int, 2>());
+    }
+    if (need)
+      ml[(kg * A::NW + wave) * 128 + lane] = mx;
+  }
 
   if (KS == 1 || n_end > 0) {
     A::issue_k(rk, ko, p.k_sm, j0, k_lds, wave);
@@ -444,6 +501,15 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
   }
   __builtin_amdgcn_s_waitcnt(0x7 << 4); // vmcnt(0)
   __syncthreads();
+  if constexpr (KS > 1) {
+    if (kg > 0) {
+      l_i = 0.0f;
+#pragma unroll
+      for (int k = 0; k < KS - 1; ++k)
+        if (k < kg)
+          m_i = fmaxf(m_i, ml[(k * A::NW + wave) * 128 + lane]);
+    }
+  }
   A::template qk<0>(bs, qf, s); // (an empty group: stale values, not used)
   __syncthreads(); // K slot 0 is refilled by iteration 0
 
@@ -463,11 +529,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs &p) {
       A::issue_v(rv, vo, p.v_sm, at(j + 1), v_lds + (1 - SL) * A::TILE, wave);
     typename A::f16v sn[A::BN / 32];
     A::template qk<1 - SL>(bs, qf, sn); // S_{j+1} (a stale slot after the last block: unused)
-    // On-band blocks whose keys all lie past this wave's 32 rows add exactly
-    // nothing (p = 0, alpha = 1, as for the blocks past the diagonal): the
-    // wave skips their softmax and P V.
-    const bool live = !MASK || at(j) * A::BN <= start_m * A::BM + 32 * wave + 31;
-    if (live) {
+    if (!MASK || live(at(j))) {
       typename A::PF pf;
       A::template softmax<MASK>(s, at(j) * A::BN, m, p.qk_scale, acc, m_i, l_i, pf);
       A::template pv<SL>(bs, pf, acc);

@@ -68,8 +68,8 @@ extern const Decode16KernelFn kDecode16WideKernels[2][2][kDec16WideMaxM / 16];
 extern const Decode16KernelFn kDecodeWqKernels[4][kDec16MaxM / 16];
 extern const AttnFn kAttn[2][5][2][2][2];
 extern const AttnFn kAttn8[2][5][2][2];
-// The same with groups of waves that share the rows and split the keys:
-// [128 rows x 2 groups, 64 x 2, 32 x 4][causal][head_dim 16 / 32 / 64 / 128][bf16].
-extern const AttnFn kAttnKs[3][2][4][2];
+// The same with 4 groups of waves that share 32 rows and split the keys:
+// [causal][head_dim 16 / 32 / 64][bf16].
+extern const AttnFn kAttnKs[2][3][2];
 
 } // namespace txk

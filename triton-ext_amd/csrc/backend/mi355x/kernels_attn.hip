@@ -19,20 +19,11 @@ const AttnFn kAttn[2][5][2][2][2] = {
 #undef TX_ATTN_DTYPES
 #undef TX_ATTN_BLOCKS
 
-// (head dim 128 has no 32 x 4: its slots would take 256 KiB)
-#define TX_ATTN_KS(C, HD, BM, KS)                                                           \
-  {attn_fwd_ks_kernel<C, HD, false, BM, KS>, attn_fwd_ks_kernel<C, HD, true, BM, KS>}
-#define TX_ATTN_KSD(C, BM, KS)                                                              \
-  {TX_ATTN_KS(C, 16, BM, KS), TX_ATTN_KS(C, 32, BM, KS), TX_ATTN_KS(C, 64, BM, KS),         \
-   TX_ATTN_KS(C, 128, BM, KS)}
-const AttnFn kAttnKs[3][2][4][2] = {
-    {TX_ATTN_KSD(false, 128, 2), TX_ATTN_KSD(true, 128, 2)},
-    {TX_ATTN_KSD(false, 64, 2), TX_ATTN_KSD(true, 64, 2)},
-    {{TX_ATTN_KS(false, 16, 32, 4), TX_ATTN_KS(false, 32, 32, 4), TX_ATTN_KS(false, 64, 32, 4),
-      {nullptr, nullptr}},
-     {TX_ATTN_KS(true, 16, 32, 4), TX_ATTN_KS(true, 32, 32, 4), TX_ATTN_KS(true, 64, 32, 4),
-      {nullptr, nullptr}}}};
-#undef TX_ATTN_KSD
+#define TX_ATTN_KS(C, HD)                                                                   \
+  {attn_fwd_ks_kernel<C, HD, false, 32, 4>, attn_fwd_ks_kernel<C, HD, true, 32, 4>}
+const AttnFn kAttnKs[2][3][2] = {
+    {TX_ATTN_KS(false, 16), TX_ATTN_KS(false, 32), TX_ATTN_KS(false, 64)},
+    {TX_ATTN_KS(true, 16), TX_ATTN_KS(true, 32), TX_ATTN_KS(true, 64)}};
 #undef TX_ATTN_KS
 
 } // namespace txk

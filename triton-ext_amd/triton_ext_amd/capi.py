@@ -71,7 +71,7 @@ _ATTN_STRIDES = {t: (f"{t}_sz", f"{t}_sh", f"{t}_sm") for t in "qkvo"}
 class AttnPlan(ctypes.Structure):
     _fields_ = [("desc", AttnDesc), ("flops", ctypes.c_double), ("bytes", ctypes.c_double),
                 ("qk_scale", ctypes.c_float), ("m_blocks", ctypes.c_int32), ("grid_x", ctypes.c_int32),
-                ("block_threads", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+                ("block_threads", ctypes.c_int32), ("key_groups", ctypes.c_int32)]
 
 
 class LoopSplit(ctypes.Structure):
