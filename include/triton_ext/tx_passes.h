@@ -125,6 +125,12 @@ TX_API int tx_dot_operand_spans(const tx_dot_desc *desc, int64_t *a_bytes, int64
 TX_API int32_t tx_gemm_split_k(int64_t tiles, int64_t ksteps);
 /* The same for the 128x128 tiles of TX_FLAG_TILES_128. */
 TX_API int32_t tx_ring_split_k(int64_t tiles128, int64_t ksteps);
+/* Whether the 128x128 tiles can address a dot whose operands the 256x256 tiles
+ * can (desc as the tile reads it: an upcast operand is bf16): a row-major B's
+ * offsets are formed up to 128 rows past K (e2m1: packed rows, of ldb bytes)
+ * and must stay below 2^32 bytes; fewer than 2^23 tiles of 512 threads.  The
+ * planner and the launch both ask here. */
+TX_API int32_t tx_ring_reaches(const tx_dot_desc *desc);
 /* Row stride (elements) of a B operand that tl.dot_scaled with one bf16 side
  * upcasts to bf16 in the workspace: N rounded up to 16 columns, so every row
  * starts 16-byte aligned for the bf16 tile.  (An upcast A is packed: K.) */

@@ -4,6 +4,8 @@ The flag changes neither the plan's block nor its workspace; it is set where
 the 256x256 tiles leave CUs idle and the split that fills them costs more than
 the smaller tile, and never on a block asked for.
 """
+import ctypes
+
 import pytest
 
 import triton_ext_amd as tx
@@ -27,3 +29,37 @@ def test_choice(M, N, K, t, mode, c, ring):
     q = tx.plan(tx.make_desc(M, N, K, t, c, scale_mode=mode, block=(256, 256, k)))
     assert not q.desc.flags & capi.FLAG_TILES_128
     assert q.grid_x == p.grid_x and q.block_threads == p.block_threads
+
+
+@pytest.mark.parametrize("M,N,K,t", [
+    (128, 16384, 262112, tx.F4E2M1), (128, 1048576, 4064, tx.F4E2M1),  # 131056 / 2032 packed rows
+    (128, 2097152, 2016, tx.F4E2M1), (65, 2097152, 1952, tx.F4E2M1),
+    (128, 1048576, 2016, tx.F8E4M3), (128, 2097152, 992, tx.F8E5M2),
+])
+def test_wide_mx_plans(M, N, K, t):
+    """The planner and the launch layer hold the ring tiles to one bound, 128 rows of B past K
+    within 2^32 bytes (e2m1: packed rows, K / 2 of them): what the planner chooses is planned."""
+    k = 256 if t == tx.F4E2M1 else 128
+    p = tx.plan(tx.make_desc(M, N, K, t, tx.F32, scale_mode=tx.SCALE_MX32))
+    assert (p.desc.block_m, p.desc.block_n, p.desc.block_k) == (256, 256, k)
+    if not tx.load().tx_device_available():  # the launch's own checks accept it (dummy pointers)
+        a = ctypes.c_void_p(1 << 20)
+        assert tx.load().tx_dot_launch(ctypes.byref(p), a, a, a, a, a, a, p.workspace_bytes,
+                                       None) == tx.ERR_NO_DEVICE
+
+
+@pytest.mark.parametrize("K,ld,ok", [
+    (128, (1 << 24) - 16, True),   # 255 rows of B, of 2^24 - 16 bytes: below 2^32
+    (127, 1 << 24, True),          # 255 rows of 2^24
+    (128, 1 << 24, False),         # 256 of them
+])
+def test_ring_bound(K, ld, ok):
+    d = tx.make_desc(300, 512, K, tx.F8E4M3, tx.F32, block=(256, 256, 128), ldb=ld, ldc=512,
+                     lda=128, flags=capi.FLAG_TILES_128)
+    p = capi.DotPlan()
+    rc = tx.load().tx_dot_plan_create(ctypes.byref(d), ctypes.byref(p))
+    assert rc == (tx.OK if ok else tx.ERR_UNSUPPORTED)
+    # left to itself the planner takes the 256x256 tile past the bound
+    d = tx.make_desc(300, 512, K, tx.F8E4M3, tx.F32, ldb=ld, ldc=512, lda=128)
+    p = tx.plan(d)
+    assert ok or not p.desc.flags & capi.FLAG_TILES_128

@@ -140,3 +140,36 @@ def test_tiles128_acc_noalloc_and_repeat(gpu):
         want = a.double() @ b.double()
         assert ((c0.double() - want).abs() <= 1e-5 * (a.double().abs() @ b.double().abs())).all()
         assert np.isfinite(c0.sum().item())
+
+
+def test_tiles128_wide_mxfp4(gpu):
+    """e2m1 B of nearly 2^31 bytes, whose offsets past K lie above 2^31: the same sums as the
+    256x256 tile's, whose K order is the same within 8 steps (the module's bound; |a b| summed
+    over slices of columns)."""
+    import torch
+    M, N, K = 128, 1048576, 4064
+    say(f"tiles128 mxfp4 {M}x{N}x{K}")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(11)
+    a = torch.randint(0, 256, (M, K // 2), generator=g, device=gpu, dtype=torch.uint8)
+    b = torch.randint(0, 256, (K // 2, N), generator=g, device=gpu, dtype=torch.uint8)
+    sa = torch.randint(124, 131, (M, K // 32), generator=g, device=gpu, dtype=torch.uint8)
+    sb = torch.randint(124, 131, (N, K // 32), generator=g, device=gpu, dtype=torch.uint8)
+    a = tx.aligned_rows(a, col_ok=False)
+    p = tx.plan(tx.make_desc(M, N, K, tx.F4E2M1, tx.F32, scale_mode=tx.SCALE_MX32,
+                             lda=2 * a.stride(0), ldb=N, ldc=N))
+    assert p.desc.flags & tx.FLAG_TILES_128
+    got = tx.dot_scaled(a, sa, "e2m1", b, sb, "e2m1", plan=p)
+    want = tx.dot_scaled(a, sa, "e2m1", b, sb, "e2m1", block=(256, 256, 256))
+    torch.cuda.synchronize()
+    mag = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6] * 2, device=gpu, dtype=torch.float64)
+
+    def values(codes, s):  # |rows of codes times their scales| [R, K]
+        x = mag[torch.stack([codes & 15, codes >> 4], 2).long()].view(codes.shape[0], -1)
+        return x * torch.exp2(s.double() - 127).repeat_interleave(32, 1)
+    fa = values(a, sa)
+    for n in (0, N // 2 - 512, N - 1024):
+        S = fa @ values(b[:, n:n + 1024].t().contiguous(), sb[n:n + 1024]).t().contiguous()
+        d = (got[:, n:n + 1024].double() - want[:, n:n + 1024].double()).abs()
+        assert (d <= (K / 16 + 8) * 2.0 ** -23 * S).all()
+    assert torch.isfinite(got).all() and float((got - want).abs().max()) < 1e-2 * float(want.abs().max())

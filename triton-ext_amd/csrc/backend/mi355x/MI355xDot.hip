@@ -450,12 +450,9 @@ int checkSpans32(const tx_dot_desc &d, const GemmConfig &c) {
                 c.bm, c.bn, (long long)sa, (long long)sb);
   if (ringPlan(d) && (c.bm != 256 || c.bn != 256))
     return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128 takes the 256x256 tiles");
-  if (ringPlan(d) && cdiv(d.M, 128) * cdiv(d.N, 128) > INT32_MAX)
-    return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128: a grid above 2^31 tiles");
-  // (the ring tile also forms the offsets of up to 127 rows of B past K)
-  if (ringPlan(d) && !(d.flags & TX_FLAG_B_KMAJOR) &&
-      (e.K + 128) * e.ldb * (tx_dtype_bits(e.b_type) == 16 ? 2 : 1) >= ((int64_t)1 << 32))
-    return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128: 128 rows of B past K end beyond 2^32 bytes");
+  if (ringPlan(d) && !tx_ring_reaches(&e))
+    return fail(TX_ERR_UNSUPPORTED, "TX_FLAG_TILES_128: 128 rows of B past K end beyond 2^32 "
+                                    "bytes, or 2^23 tiles or more");
   return TX_OK;
 }
 

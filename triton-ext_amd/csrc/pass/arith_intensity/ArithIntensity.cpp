@@ -170,6 +170,18 @@ extern "C" int tx_dot_operand_spans(const tx_dot_desc *d, int64_t *a_bytes, int6
   return TX_OK;
 }
 
+extern "C" int32_t tx_ring_reaches(const tx_dot_desc *d) {
+  if (!d || cdiv(d->M, 128) * cdiv(d->N, 128) >= ((int64_t)1 << 23))
+    return 0;
+  if (d->flags & TX_FLAG_B_KMAJOR)
+    return 1;
+  const bool packed = tx_dtype_bits(d->b_type) == 4; // ldb: bytes of a row of two K values
+  const int64_t rows = packed ? (d->K + 1) / 2 : d->K, ldb = d->ldb ? d->ldb : d->N;
+  const __int128 bytes =
+      (__int128)(rows + 128) * ldb * (packed ? 1 : tx_dtype_bits(d->b_type) / 8);
+  return bytes < (__int128)1 << 32;
+}
+
 namespace {
 
 // tx_arith_intensity; *tiles128: the chosen tile runs on 128x128 tiles.
@@ -271,12 +283,9 @@ int analyse(const tx_dot_desc *d, tx_ai_report *out, bool *tiles128) {
                            (d->a_type == TX_BF16 || d->scale_mode == TX_SCALE_NV16) &&
                            d->M <= 96 && d->K >= 256 && d->N <= (int64_t)16384 * 128 &&
                            (d->c_type == TX_BF16 || d->c_type == TX_F32);
-    // Operands the 32-bit-offset tiles reach; the 128x128 ring tiles also form
-    // the offsets of up to 127 rows of a row-major B past K.
+    // Operands the 32-bit-offset tiles reach, and the 128x128 ring tiles too.
     const bool span32 = spanA < TX_SPAN32_LIMIT && spanB < TX_SPAN32_LIMIT;
-    const int64_t ldbBytes = (e.ldb ? e.ldb : kmajor ? e.K : e.N) * tx_dtype_bits(e.b_type) / 8;
-    const bool can128 = span32 && ldbBytes < TX_SPAN32_LIMIT / 128 &&
-                        cdiv(d->M, 128) * cdiv(d->N, 128) < (1 << 24);
+    const bool can128 = span32 && tx_ring_reaches(&e);
     const bool mx = d->scale_mode == TX_SCALE_MX32;
     double us = 0.0;
     // The 16-bit tiles: 256x256 (or 128x128) against 64x64, which only

@@ -99,7 +99,8 @@ EXPORTS = {
         "txReadExtConf"],
     "libloop_split.so": ["tx_loop_split_plan", "tx_loop_split_k"],
     "libarith_intensity.so": ["tx_dtype_size", "tx_dtype_bits", "tx_mi355x_peak_flops",
-                              "tx_mi355x_peak_bw", "tx_arith_intensity", "tx_dot_operand_spans"],
+                              "tx_mi355x_peak_bw", "tx_arith_intensity", "tx_dot_operand_spans",
+                              "tx_ring_reaches"],
     "libmi355x_dot.so": ["tx_dot_plan_create", "tx_dot_launch", "tx_dot_launch_noalloc",
                          "tx_get_last_error", "tx_kernel_name", "tx_device_available"],
 }
