@@ -590,3 +590,36 @@ def test_e4m3_max_codes_are_nan(gpu):
     assert np.array_equal(got[~poisoned], f["c"][~poisoned])
     # the interpreter itself (and the oracle) read +-480: finite everywhere
     assert np.isfinite(f["c"]).all()
+
+
+@pytest.mark.parametrize("M", [16, 200])
+def test_broadcast_operands(gpu, M):
+    """Views of one row or column shown to all (a stride of 0), as operands and as scales, and
+    k / v of one head: the results of their copies, bit for bit."""
+    import torch
+    say(f"broadcast operands M={M}")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(M)
+    K, N = 320, 256
+    a, b = (torch.randn(s, generator=g, device=gpu).bfloat16() for s in ((M, K), (K, N)))
+    rows, cols = a[:1].expand(M, K), b[:, :1].expand(K, N)
+    same = lambda x, y: torch.equal(x.view(torch.int16), y.view(torch.int16))
+    for x, y in ((rows, b), (a, b[:1].expand(K, N)), (a, cols), (a, cols.t().t()),
+                 (a, a[:1].expand(N, K).t())):
+        assert same(tx.dot(x, y), tx.dot(x.clone(memory_format=torch.contiguous_format),
+                                         y.clone(memory_format=torch.contiguous_format)))
+    a8, b8 = (torch.round(x.float() * 30).clamp(-127, 127).to(torch.int8) for x in (a, b))
+    sa, sb = torch.tensor([0.5], device=gpu).expand(M), torch.tensor([0.25], device=gpu).expand(N)
+    assert same(tx.dot(a8, b8, scale_a=sa, scale_b=sb),
+                tx.dot(a8, b8, scale_a=sa.contiguous(), scale_b=sb.contiguous()))
+    sc = torch.full((M, K // 32), 127, device=gpu, dtype=torch.uint8)
+    sbm = torch.full((N, K // 32), 126, device=gpu, dtype=torch.uint8)
+    f8 = a.to(torch.float8_e4m3fn)[:1].expand(M, K), b.to(torch.float8_e4m3fn)[:1].expand(K, N)
+    got = tx.dot_scaled(f8[0], sc, "e4m3", f8[1], sbm, "e4m3")
+    want = tx.dot_scaled(f8[0].contiguous(), sc, "e4m3", f8[1].contiguous(), sbm, "e4m3")
+    assert torch.equal(got, want)
+    q = torch.randn((1, 4, 256, 64), generator=g, device=gpu).bfloat16()
+    k, v = (torch.randn((1, 1, 256, 64), generator=g, device=gpu).bfloat16().expand(1, 4, 256, 64)
+            for _ in range(2))
+    assert same(tx.attention(q, k, v, True, 0.125),
+                tx.attention(q, k.contiguous(), v.contiguous(), True, 0.125))

@@ -94,3 +94,76 @@ def test_plan_rejects_a_transposed_a():
     a = _t((64, 64)).t()[:, :32]          # columns contiguous: A must be row-major
     with pytest.raises(ValueError):
         txdot.plan_for(a, _t((32, 16)), tx.F32)
+
+
+def _overlapping(kind):
+    """Views of fewer elements than they show: 16 bytes apart or 0, on an aligned base."""
+    import torch
+    r = torch.arange(4096, dtype=torch.float32).to(torch.bfloat16)
+    return {"row": r[:320].expand(64, 320),                  # every row the same: stride 0
+            "col": r[:64, None].expand(64, 320),             # every column the same (rows of one value)
+            "kmajor": r[:64].expand(320, 64).t(),            # the same as a transposed view
+            "column": r[:1, None].expand(64, 1),
+            "window": r.unfold(0, 320, 8)[:64]}[kind]        # rows that share elements
+
+
+@pytest.mark.parametrize("kind", ["row", "col", "kmajor", "column", "window"])
+@pytest.mark.parametrize("col_ok", [False, True])
+def test_overlapping_rows_are_copied(kind, col_ok):
+    """A stride of 0 reads as "packed" in a descriptor: such a view, and rows that overlap, are
+    copied to storage of their own, and a plan of the view itself is refused."""
+    import torch
+    t = _overlapping(kind)
+    c = txdot.aligned_rows(t, col_ok=col_ok)
+    assert c is not t and torch.equal(c, t)
+    lies, ld = txdot._layout(c, col_ok)
+    n, length = c.shape if lies == "row" else c.shape[::-1]
+    assert ld >= length and ld % 8 == 0 and c.untyped_storage().nbytes() >= ((n - 1) * ld + length) * 2
+    other, ldc = _t((16, 64)), -(-t.shape[1] // 8) * 8
+    with pytest.raises(ValueError):
+        txdot.plan_for(other, t, tx.BF16, ldc=ldc)
+    assert txdot.plan_for(other, txdot.aligned_rows(t), tx.BF16, ldc=ldc).desc.K == 64
+    if kind in ("row", "window"):
+        with pytest.raises(ValueError):
+            txdot.plan_for(t, _t((320, 64)), tx.BF16)
+        a = txdot.aligned_rows(t, col_ok=False)
+        assert txdot.plan_for(a, _t((320, 64)), tx.BF16).desc.lda >= 320
+
+
+def test_single_rows_of_any_stride_are_not_copied():
+    import torch
+    t = torch.as_strided(_t((64,)), (1, 64), (0, 1))  # one row: its stride says nothing
+    assert txdot.aligned_rows(t, col_ok=False) is t
+    assert txdot.plan_for(t, _t((64, 64)), tx.BF16).desc.lda == 64
+
+
+@pytest.mark.parametrize("dtype_name", ["bfloat16", "float8_e5m2"])
+def test_attention_broadcast_heads_are_copied(dtype_name, monkeypatch):
+    """k and v of one head shown to all (a stride of 0) reach the plan as packed copies; a
+    dimension of size 1 may have any stride."""
+    import torch
+    seen = {}
+
+    class Planned(Exception):
+        pass
+
+    def plan(*args, strides=None, **kw):
+        seen.update(strides)
+        raise Planned
+
+    monkeypatch.setattr(txdot.capi, "attn_plan", plan)
+    q = _t((1, 4, 128, 32), dtype_name)
+    k = _t((1, 1, 128, 32), dtype_name).expand(1, 4, 128, 32)
+    v = _t((1, 1, 32, 128), dtype_name).expand(1, 4, 32, 128).permute(0, 1, 3, 2) \
+        if dtype_name == "float8_e5m2" else k
+    with pytest.raises(Planned):
+        txdot.attention(q, k, v, False, 0.5)
+    rows = 128 if dtype_name == "float8_e5m2" else 32
+    assert seen["k"][1:] == (128 * 32, 32) and seen["v"][1:] == (128 * 32, rows)
+
+
+def test_broadcast_out_is_refused():
+    import torch
+    with pytest.raises(ValueError, match="16 bytes apart"):
+        txdot._out_ldc(torch.zeros(1, 64).expand(16, 64))
+    assert txdot._out_ldc(torch.zeros(16, 64)) == 64

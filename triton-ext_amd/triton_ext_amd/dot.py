@@ -73,12 +73,13 @@ def _out_ldc(out):
     apart), or, for a single row, any 16-byte pitch (never used)."""
     if out.dim() != 2 or (out.shape[1] > 1 and out.stride(1) != 1):
         raise ValueError("out must be a row-major [M, N] tensor")
-    if out.shape[0] <= 1:
-        return _row_pitch(max(out.shape[1], 1), out.element_size())
-    if (out.stride(0) * out.element_size()) % 16 or out.data_ptr() % 16:
+    (M, N), ld, elt = out.shape, out.stride(0), out.element_size()
+    if M <= 1:
+        return _row_pitch(max(N, 1), elt)
+    if (ld * elt) % 16 or ld < N or out.data_ptr() % 16:
         raise ValueError("out's rows must start 16 bytes apart on a 16-byte aligned base "
                          "(new_output makes such a tensor)")
-    return out.stride(0)
+    return ld
 
 
 def _layout(t, col_ok=True):
@@ -98,6 +99,13 @@ def _layout(t, col_ok=True):
     if col_ok and (R <= 1 or s0 == 1):
         return "col", s1
     return None, 0
+
+
+def _overlaps(kind, ld, t):
+    """Whether the rows (kind "col": the columns) of t share elements: less than their length
+    apart, as a broadcast view's are (0, which a descriptor reads as "packed")."""
+    n, length = (t.shape[1], t.shape[0]) if kind == "col" else t.shape
+    return n > 1 and ld < length
 
 
 def _b_col_ok(b):
@@ -126,18 +134,28 @@ def _b_kmajor_ok(a, b, c_tx, scale_mode, block, flags):
             and _kmajor_plans(a, b, c_tx, scale_mode, block, flags))
 
 
+def _strides_nonzero(t):
+    """Whether every dimension of t but those of size 1 has a stride."""
+    st = t.stride()
+    return 0 not in st or all(s or n <= 1 for s, n in zip(st, t.shape))
+
+
 def _rows_aligned(t):
     """Whether t is plainly 2-D rows 16 bytes apart on a 16-byte aligned base:
     what aligned_rows() returns as it is, whatever col_ok."""
-    return (t.dim() == 2 and t.stride(1) == 1 and (t.stride(0) * t.element_size()) % 16 == 0
-            and t.data_ptr() % 16 == 0)
+    if t.dim() != 2:
+        return False
+    s0, s1 = t.stride()
+    return (s1 == 1 and (s0 * t.element_size()) % 16 == 0 and t.data_ptr() % 16 == 0
+            and (s0 >= t.size(1) or t.size(0) <= 1))
 
 
 def aligned_rows(t, col_ok=True):
     """t itself when its rows (or, for a transposed view and col_ok, its
-    columns) start 16 bytes apart on a 16-byte aligned base, else a copy in
-    padded storage of the same layout (row-major when not col_ok).  The
-    kernels read 16-byte chunks; K and N themselves may be any size."""
+    columns) start 16 bytes apart on a 16-byte aligned base and do not overlap,
+    else a copy in padded storage of the same layout (row-major when not
+    col_ok).  The kernels read 16-byte chunks; K and N themselves may be any
+    size."""
     import torch
     if t.dim() != 2 or t.numel() == 0:
         return t
@@ -145,7 +163,8 @@ def aligned_rows(t, col_ok=True):
         return t
     elt = t.element_size()
     kind, ld = _layout(t, col_ok)
-    if kind is not None and (ld * elt) % 16 == 0 and t.data_ptr() % 16 == 0:
+    if kind is not None and (ld * elt) % 16 == 0 and t.data_ptr() % 16 == 0 \
+            and not _overlaps(kind, ld, t):
         return t
     if kind == "col":  # [N][K] storage viewed as [K][N]
         return aligned_rows(t.t().contiguous()).t()
@@ -174,6 +193,8 @@ def plan_for(a, b, out_dtype_tx, scale_mode=capi.SCALE_NONE, block=(0, 0, 0), fl
     if a_kind != "row" or b_kind is None:
         raise ValueError("A rows must be contiguous, and B rows (or B's columns) too")
     b_kmajor = b_kind == "col"
+    if (a_ld < K and M > 1) or (b_ld < (K if b_kmajor else N) and (N if b_kmajor else K) > 1):
+        raise ValueError("A's or B's rows overlap (a broadcast view?); aligned_rows copies them")
     if b_kmajor:
         flags |= capi.FLAG_B_KMAJOR
     # an empty operand's strides are arbitrary: describe it as packed
@@ -251,6 +272,10 @@ def dot(a, b, out=None, out_dtype=None, scale_a=None, scale_b=None, scale_mode=N
         a = aligned_rows(a, col_ok=False)
         if not _rows_aligned(b):
             b = aligned_rows(b, col_ok=_b_kmajor_ok(a, b, c_tx, scale_mode, block, flags))
+    if scale_a is not None and not _strides_nonzero(scale_a):  # a broadcast scale
+        scale_a = scale_a.contiguous()
+    if scale_b is not None and not _strides_nonzero(scale_b):
+        scale_b = scale_b.contiguous()
     if acc is not None:
         if acc.dtype not in (torch.float32, torch.int32) or acc.dim() != 2:
             raise ValueError("acc must be an fp32 or int32 [M, N] tensor")
@@ -441,14 +466,20 @@ def attention(q, k, v, causal, sm_scale, USE_TMA=True, *, return_lse=False, plan
     if fp8 and v.stride(2) != 1:
         raise ValueError("v: float8_e5m2 v must be key-contiguous (stride 1 along N_CTX), "
                          "as v.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2) makes it")
+    qs, ks, vs = q.stride(), k.stride(), v.stride()
+    if 0 in qs or 0 in ks or 0 in vs:
+        # a broadcast view (heads of one k, say): its stride of 0 would be read as "packed"
+        q, k = (t if _strides_nonzero(t) else t.contiguous() for t in (q, k))
+        if not _strides_nonzero(v):
+            v = v.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2) if fp8 else v.contiguous()
+        qs, ks, vs = q.stride(), k.stride(), v.stride()
     Z, H, N = q.shape[:3]
     o = torch.empty_like(q, memory_format=torch.contiguous_format)
     M = torch.empty((Z, H, N), device=q.device, dtype=torch.float32)
     if plan is None:
-        st = {nm: (t.stride(0), t.stride(1), t.stride(2)) for nm, t in
-              (("q", q), ("k", k), ("v", v), ("o", o))}
-        if fp8:
-            st["v"] = (v.stride(0), v.stride(1), v.stride(3))  # dim rows of N_CTX keys
+        # (e5m2 v: dim rows of N_CTX keys)
+        st = {"q": qs[:3], "k": ks[:3], "v": vs[:2] + vs[3:] if fp8 else vs[:3],
+              "o": o.stride()[:3]}
         dt = capi.F8E5M2 if fp8 else capi.BF16 if q.dtype == torch.bfloat16 else capi.F16
         plan = capi.attn_plan(Z, H, N, HEAD_DIM, causal, sm_scale, dtype=dt, strides=st,
                               block=block)
