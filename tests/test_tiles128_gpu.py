@@ -173,3 +173,41 @@ def test_tiles128_wide_mxfp4(gpu):
         d = (got[:, n:n + 1024].double() - want[:, n:n + 1024].double()).abs()
         assert (d <= (K / 16 + 8) * 2.0 ** -23 * S).all()
     assert torch.isfinite(got).all() and float((got - want).abs().max()) < 1e-2 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "mxw"])
+def test_tiles128_noalloc_split(gpu, kind):
+    """The no-allocation launch splits K as the ring tiles do (2 ranges, 12 or 16 MiB of partials),
+    whatever the 256x256 tiles' own split would take (8 ranges, past the scratch): the bits of
+    the launch with a workspace, over several launches."""
+    import ctypes
+
+    import torch
+    M, N, K = (384, 4096, 4096) if kind == "mxw" else (256, 8192, 8192)
+    say(f"tiles128 noalloc split {kind} {M}x{N}x{K}")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(9)
+    sb = None
+    a = torch.randn((M, K), generator=g, device=gpu).bfloat16()
+    if kind == "mxw":
+        b = torch.randint(0, 256, (K // 2, N), generator=g, device=gpu, dtype=torch.uint8)
+        sb = torch.randint(124, 131, (N, K // 32), generator=g, device=gpu, dtype=torch.uint8)
+        p = tx.plan(tx.make_desc(M, N, K, tx.BF16, tx.F32, b_type=tx.F4E2M1,
+                                 scale_mode=tx.SCALE_MX32, ldb=N, ldc=N))
+        run = lambda: tx.dot_scaled(a, None, "bf16", b, sb, "e2m1", plan=p)
+    else:
+        b = torch.randn((K, N), generator=g, device=gpu).bfloat16()
+        if kind == "fp8":
+            a, b = a.to(torch.float8_e4m3fn), b.to(torch.float8_e4m3fn)
+        p = tx.plan_for(a, b, tx.F32)
+        run = lambda: tx.dot(a, b, plan=p, out=torch.empty((M, N), device=gpu))
+    assert p.desc.flags & tx.FLAG_TILES_128 and p.split_k == 8
+    assert p.workspace_bytes > tx.NOALLOC_SCRATCH_BYTES
+    want = run()
+    for _ in range(3):
+        got = torch.empty_like(want)
+        tx.check(tx.load().tx_dot_launch_noalloc(
+            ctypes.byref(p), a.data_ptr(), b.data_ptr(), got.data_ptr(), None,
+            None if sb is None else sb.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32))

@@ -393,6 +393,10 @@ int ringSplit(const tx_dot_desc &d) {
              ? 1
              : tx_ring_split_k(cdiv(d.M, 128) * cdiv(d.N, 128), cdiv(d.K, d.block_k));
 }
+// The K ranges a launch of a plan with `split` of them makes.
+int launchSplit(const tx_dot_desc &d, int split) {
+  return ringPlan(d) && split > ringSplit(d) ? ringSplit(d) : split;
+}
 // d: the dot the tile runs (for the MX x bf16 upcast, its bf16 dot: bfDot).
 int gemmSplit(const tx_dot_desc &d, int op, int64_t tiles) {
   if (ringPlan(d) && d.scale_mode == TX_SCALE_MX32)
@@ -713,8 +717,7 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
       plan.n_tiles <= 0 || plan.block_threads != c.wm * c.wn * 64 ||
       plan.grid_y != split)
     return fail(TX_ERR_INVALID, "plan launch shape does not match its tile");
-  if (ring && split > ringSplit(d))
-    split = ringSplit(d);
+  split = launchSplit(d, split);
   const GemmConfig *rc = nullptr;
   if (ring) {
     rc = findRing(op, split > 1 ? partialEpi(d, op) : epi, (d.flags & TX_FLAG_B_KMAJOR) != 0,
@@ -1211,19 +1214,23 @@ int launchPlanned(const tx_dot_plan *plan, const void *A, const void *B, void *C
   const int prc = checkPlan(*plan);
   if (prc != TX_OK)
     return prc;
-  // No allocation: a split-K tile plan whose partials do not fit the scratch
-  // runs unsplit (the same dot, one K range a tile).
-  tx_dot_plan unsplit;
+  // No allocation: a tile plan takes the K ranges its launch makes (ring tiles:
+  // their own, not the 256x256 tiles' of the plan), or, where the partials do
+  // not fit the scratch, one (the same dot, one K range a tile).
+  tx_dot_plan fits;
   if (noalloc && plan->split_k > 1 && plan->grid_y == plan->split_k &&
       plan->workspace_bytes > (int64_t)TX_NOALLOC_SCRATCH_BYTES &&
       (plan->kernel == TX_KERNEL_GEMM_16BIT || plan->kernel == TX_KERNEL_GEMM_I8 ||
        plan->kernel == TX_KERNEL_GEMM_F8 || plan->kernel == TX_KERNEL_GEMM_MX_BF16 ||
        plan->kernel == TX_KERNEL_GEMM_MX)) {
-    unsplit = *plan;
-    unsplit.split_k = 1;
-    unsplit.grid_y = 1;
-    unsplit.workspace_bytes = gemmWorkspace(plan->desc, 1);
-    plan = &unsplit;
+    int split = launchSplit(d, plan->split_k);
+    if (gemmWorkspace(d, split) > (int64_t)TX_NOALLOC_SCRATCH_BYTES)
+      split = 1;
+    fits = *plan;
+    fits.split_k = split;
+    fits.grid_y = split;
+    fits.workspace_bytes = gemmWorkspace(d, split);
+    plan = &fits;
   }
   if (noalloc && (plan->workspace_bytes < 0 ||
                   plan->workspace_bytes > (int64_t)TX_NOALLOC_SCRATCH_BYTES))
