@@ -63,3 +63,12 @@ def test_ring_bound(K, ld, ok):
     d = tx.make_desc(300, 512, K, tx.F8E4M3, tx.F32, ldb=ld, ldc=512, lda=128)
     p = tx.plan(d)
     assert ok or not p.desc.flags & capi.FLAG_TILES_128
+
+
+def test_ring_group_m():
+    """plan.group_m is what the launch takes: 4 tile rows on the ring tiles whatever K, 2 on the
+    8-bit 256x256 tile once K spans 8192 bytes."""
+    for block, gm in (((0, 0, 0), 4), ((256, 256, 128), 2)):
+        p = tx.plan(tx.make_desc(512, 8192, 8192, tx.I8, tx.BF16, scale_mode=tx.SCALE_ROWCOL,
+                                 block=block))
+        assert bool(p.desc.flags & capi.FLAG_TILES_128) == (gm == 4) and p.group_m == gm

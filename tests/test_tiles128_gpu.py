@@ -211,3 +211,19 @@ def test_tiles128_noalloc_split(gpu, kind):
             None if sb is None else sb.data_ptr(), torch.cuda.current_stream().cuda_stream))
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("M,N,K,split", [(700, 1100, 512, False), (300, 700, 8192, True)])
+def test_tiles128_group_m(gpu, M, N, K, split):
+    """A caller's plan.group_m, past the tile rows too, changes the tile order alone."""
+    import torch
+    say(f"tiles128 group_m {M}x{N}x{K}")
+    a, b = (torch.randint(-127, 128, s, device=gpu, dtype=torch.int8) for s in ((M, K), (K, N)))
+    b = tx.aligned_rows(b)
+    p = tx.plan_for(a, b, tx.I32, ldc=-(-N // 4) * 4)
+    assert p.desc.flags & tx.FLAG_TILES_128 and (p.split_k > 1) == split
+    want = a.double() @ b.double()
+    for gm in (1, 2, 3, 4, 100, 2 ** 31 - 1):
+        p.group_m = gm
+        out = tx.new_output(M, N, torch.int32, gpu)
+        assert torch.equal(tx.dot(a, b, plan=p, out=out).double(), want)

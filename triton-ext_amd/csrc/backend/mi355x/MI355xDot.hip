@@ -546,9 +546,11 @@ int txMi355xDotRun(tx_dot_plan *plan) {
   // Tile rows per group of the XCD-aware tile order: 4, except 2 on the 8-bit
   // tile once K spans 8192 bytes or more (a sweep of 1..32: mxfp8 8192^3 ran
   // 2365 TFLOP/s at 2 against 1930 at 4; 4096^3, C5 (K = 7168) and mxfp4
-  // 8192^3 (K = 4096 bytes) were as fast or faster at 4).
+  // 8192^3 (K = 4096 bytes) were as fast or faster at 4).  The 128x128 ring
+  // tiles keep 4: at K = 8192 4 / 2 take 48.7 / 48.7 us (W8A8, M = 512, N =
+  // 8192), 49.2 / 49.0 (fp8) and 40.7 / 40.8 (W8A8, M = 1024, N = 4096).
   const int64_t kbytes = d.K * tx_dtype_bits(d.a_type) / 8;
-  plan->group_m = c.dma == 5 && kbytes >= 8192 ? 2 : 4;
+  plan->group_m = c.dma == 5 && kbytes >= 8192 && !ringPlan(d) ? 2 : 4;
   plan->kernel = gemmKernelOf(d, op);
   plan->split_k = gemmSplit(bfDot(d), op, (int64_t)plan->m_tiles * plan->n_tiles);
   plan->grid_x = plan->m_tiles * plan->n_tiles;
@@ -778,7 +780,7 @@ int launchGemm(const tx_dot_plan &plan, const void *A, const void *B, void *C,
   if (ring) {
     a.tiles_m = (int32_t)cdiv(d.M, 128);
     a.tiles_n = (int32_t)cdiv(d.N, 128);
-    a.group_m = a.tiles_m < 4 ? a.tiles_m : 4;
+    a.group_m = a.tiles_m < gm ? a.tiles_m : gm;
   }
   a.sa_ld = (int32_t)(mx ? d.K / 32 : cdiv(d.K, 128));
   a.sb_ld = (int32_t)cdiv(d.N, 128);
