@@ -53,6 +53,14 @@ def test_header_declarations_are_exported():
     assert declared <= exported, sorted(declared - exported)
 
 
+def test_an_extension_name_change_rebuilds_its_objects():
+    """The name in triton-ext.conf is compiled into the backend's objects, so they depend on it."""
+    pkg = os.path.dirname(os.path.dirname(capi.lib_path("libmi355x_dot.so")))
+    out = subprocess.run(["make", "-n", "-W", "csrc/backend/mi355x/triton-ext.conf", "all"],
+                         cwd=pkg, check=True, capture_output=True, text=True).stdout
+    assert "-c -o obj/MI355xDot.o" in out
+
+
 def test_self_registration_and_enumeration():
     tx.load()
     names = tx.enumerate_passes()
