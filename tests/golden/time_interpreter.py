@@ -1,6 +1,6 @@
 """Time the reference's CPU execution of the tiled dot -- the Triton
 interpreter (TRITON_INTERPRET=1) running make_golden.py's tiled_dot_kernel --
-on BASELINE's configs, in the build container:
+on the benchmark's workloads, on a CPU:
 
     python tests/golden/time_interpreter.py
 

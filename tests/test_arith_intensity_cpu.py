@@ -1,4 +1,4 @@
-"""arith_intensity classifier vs closed forms (BASELINE figures)."""
+"""arith_intensity classifier vs closed forms (figures from the data sheet and from operand sizes)."""
 import pytest
 
 import triton_ext_amd as tx

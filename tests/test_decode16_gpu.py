@@ -2,7 +2,7 @@
 
 bf16 / fp16 dots with M <= 96 stream B once on the decode kernel: strips of
 64 columns (128 for slices of 32 .. 80 rows), 128-row K batches, split-K with the fp32 partials summed in split
-order.  Parity is the north_star's fp bar: |d| <= 1e-3 + 1e-2 |ref| for inputs
+order.  Parity is the fp bar: |d| <= 1e-3 + 1e-2 |ref| for inputs
 N(0,1)/sqrt(K), against the oracle at the plan's block; fp32 C is also held to
 the exact (float64) product within fp32 summation error.  Sums of fp32
 partials depend on order, so the kernel fixes it: two launches give the same

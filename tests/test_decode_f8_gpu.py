@@ -4,7 +4,7 @@ fp8 dots with M <= 64 stream B once on the decode kernel: unscaled fp8
 (e4m3 / e5m2 in any mix) to fp32 C, and e4m3 with 1x128 A-group and 128x128
 B-block scales (the block-scaled fp8 dot) to bf16 or fp32 C.  128-column
 strips, 128-row K batches (one scale block each), split-K with the fp32
-partials summed in split order.  The bar is the north_star's fp bar,
+partials summed in split order.  The bar is the fp bar,
 |d| <= 1e-3 s + 1e-2 |ref|: s = sqrt(K) for block-scaled inputs (N(0,1) before
 quantisation), s = sqrt(K) rms(a) rms(b) for unscaled full-range codes, as
 for the 8-bit tiles.

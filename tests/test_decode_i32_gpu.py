@@ -48,7 +48,7 @@ def run_i32(gpu, a, b, acc=None, block=(0, 0, 0)):
 
 @pytest.mark.parametrize("M", [1, 16, 64, 256])
 def test_decode_int32_sums_exact(gpu, M):
-    """BASELINE's W8A8 shapes (N = K = 8192) without the epilogue: every int32 sum."""
+    """The W8A8 decode shapes (N = K = 8192) without the epilogue: every int32 sum."""
     N = K = 8192
     say(f"int8->int32 decode M={M} N={N} K={K}")
     a = uniform_i8((M, K), 100 + M)

@@ -1,6 +1,6 @@
 """GPU parity: libmi355x_dot.so through the tx_dot C-ABI vs the CPU oracle.
 
-Tolerances (north_star): int8 -> int32 bit-exact; fp16/bf16/fp8 with fp32
+Tolerances: int8 -> int32 bit-exact; fp16/bf16/fp8 with fp32
 accumulation within |d| <= 1e-3 * s + 1e-2 * |ref|, s = 1 for inputs drawn
 N(0,1)/sqrt(K) (outputs ~ 1/sqrt(K)), s = sqrt(K) for unnormalised inputs.
 The oracle sums each K block in ascending k order; the MFMA sums in its own
@@ -372,7 +372,7 @@ def test_golden_fixture_on_gpu(gpu, name):
     Exact fixtures (every fp32 partial sum exact): the GPU output equals the
     oracle's bit for bit, and where the interpreter truncated to bf16, the
     GPU's fp32 accumulator truncated gives the fixture's bits.  Others: within
-    the north_star tolerance of the fixture."""
+    the fp tolerance of the fixture."""
     golden_on_gpu(gpu, name, None)
 
 

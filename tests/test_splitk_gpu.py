@@ -4,7 +4,7 @@ and add them in range order in a second kernel that applies the dot's epilogue.
 
 Against the oracle, with operands in padded storage whose padding holds NaN
 (floating point) or random bytes (int8): int8 -> int32 and W8A8 bit-exact (the
-int32 sums are exact in any order); fp16 / bf16 / fp8 within the north_star
+int32 sums are exact in any order); fp16 / bf16 / fp8 within the fp
 tolerance (|d| <= 1e-3 s + 1e-2 |ref|) and, for fp32 C, within fp32 summation
 error of the float64 product.  Ragged K puts the peeled K tail in the last
 range.  The partials are added in range order, so repeated launches give the

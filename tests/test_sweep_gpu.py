@@ -8,7 +8,7 @@ The targeted tests name the corners one by one; this sweep crosses them
 (dtype x epilogue x tile x K-major x ragged M/N/K; attention head dim x
 block x causal x dtype) at shapes nobody picked.
 Bars as elsewhere: int8 and W8A8 bit-exact; fp16/bf16/fp8 within the
-north_star tolerance (|d| <= 1e-3 s + 1e-2 |ref|); MX within the scaled
+fp tolerance (|d| <= 1e-3 s + 1e-2 |ref|); MX within the scaled
 MFMA's rigorous bound (test_mx_gpu.check_mx) and, on codes whose 32-product
 group sums are exact in the MFMA, within the fp32 running sum's rounding;
 attention as

@@ -8,7 +8,7 @@ whose padding holds NaN (floating point) or random bytes (int8), with extra
 rows past M (A) and past K (B) holding the same: an element past an edge
 that reached the MFMA would turn a result into NaN or change an integer sum.
 
-Bars: int8 and W8A8 bit-exact; fp16/bf16/fp8 within the north_star tolerance
+Bars: int8 and W8A8 bit-exact; fp16/bf16/fp8 within the fp tolerance
 (|d| <= 1e-3 s + 1e-2 |ref|, s as in test_dot_gpu.py).
 """
 import math

@@ -251,8 +251,9 @@ int analyse(const tx_dot_desc *d, tx_ai_report *out, bool *tiles128) {
     // C in their type or fp32, B row-major or K-major, M <= 96, N up to its
     // 16384 strips of 64 columns.  It streams B once with split-K.  Each wave
     // reads every row of the slice from LDS, so its time grows with M: at
-    // N = K = 8192 bf16, M = 80 / 96 / 112 / 128 44.1 / 48.6 / 53.9 / 57.6 us
-    // against the 256 tile with split-K's 51.9 / 51.9 / 54.1 / 56.6.
+    // N = K = 8192 bf16, M = 64 / 80 / 96 33.0 / 34.9 / 45.5 us against the
+    // 256x256 tiles with split-K's 46.6 / 48.0 / 49.1, from which the bound at 96
+    // was drawn, and the 128x128 ring tiles' 33.8 / 34.6 / 35.2.
     const bool decode16 =
         (d->a_type == TX_BF16 || d->a_type == TX_F16) && d->b_type == d->a_type &&
         d->scale_mode == TX_SCALE_NONE && (d->c_type == d->a_type || d->c_type == TX_F32) &&
@@ -336,9 +337,11 @@ int analyse(const tx_dot_desc *d, tx_ai_report *out, bool *tiles128) {
       t = tile16();
     else if (decode && d->M <= 256)
       // W8A8 decode (M <= 256, N up to its 4096 column strips; past it the
-      // 8-bit tiles with split-K: at N = K = 8192 M = 384 57.5 us, 512 63.9,
-      // against 76.0 and 78.7 for the row kernel's slices of 256), 128-column
-      // strips.  Up to M = 48 one row slice and 64-row K batches split among
+      // 8-bit tiles with split-K: at N = K = 8192 M = 384 57.5 us, 512 63.9 on
+      // the 256x256 ones, against 76.0 and 78.7 for the row kernel's slices of
+      // 256.  The bound is theirs: back to back, M = 96 / 128 / 192 / 256 take
+      // 26.0 / 26.4 / 38.1 / 38.6 here, 32.5 / 37.4 / 40.3 / 45.0 on them and
+      // 25.7 / 27.8 / 32.7 / 36.8 on the 128x128 ring tiles), 128-column strips.  Up to M = 48 one row slice and 64-row K batches split among
       // the waves; beyond, row slices whose waves all take every 128-row K
       // batch: of 64 rows up to M = 128, of 128 past it.  Measured at
       // N = K = 8192, in us: M = 32 20.1 / 22.1-22.7 (slices of 64), 48 22.0 /
