@@ -227,3 +227,26 @@ def test_tiles128_group_m(gpu, M, N, K, split):
         p.group_m = gm
         out = tx.new_output(M, N, torch.int32, gpu)
         assert torch.equal(tx.dot(a, b, plan=p, out=out).double(), want)
+
+
+@pytest.mark.parametrize("K,ld", [(100, 1 << 24), (126, (1 << 24) + 16)])
+def test_tiles128_long_rows(gpu, K, ld):
+    """A few columns of a matrix of 2^24 columns, rows past K up to just below 2^32 bytes: the
+    bits of the same dot on a copy of those columns."""
+    import torch
+    M, N = 300, 512
+    say(f"tiles128 {M}x{N}x{K} of rows {ld} bytes apart")
+    g = torch.Generator(device=gpu)
+    g.manual_seed(K)
+    a = torch.randn((M, K), generator=g, device=gpu).to(torch.float8_e4m3fn)
+    whole = torch.zeros((K, ld), device=gpu, dtype=torch.uint8)
+    whole.fill_(0x7F)  # NaN
+    b = whole.view(torch.float8_e4m3fn)[:, :N]
+    b.copy_(torch.randn((K, N), generator=g, device=gpu).to(torch.float8_e4m3fn))
+    a = tx.aligned_rows(a, col_ok=False)
+    p = tx.plan_for(a, b, tx.F32)
+    assert p.desc.flags & tx.FLAG_TILES_128 and p.desc.ldb == ld
+    got = tx.dot(a, b, plan=p, out=torch.empty((M, N), device=gpu))
+    assert torch.equal(got, tx.dot(a, b.contiguous(), out_dtype=torch.float32))
+    want = a.float().double() @ b.float().double()
+    assert (got.double() - want).norm() < 1e-4 * want.norm()
