@@ -146,3 +146,39 @@ def test_wq_decode_split_and_segments(gpu, lhs, rhs, fmt, M, N, K):
     bound = K * 2.0 ** -24 * (av @ bv) + 1e-30
     d = np.abs(got[:, cols].astype(np.float64) - ref)
     assert (d <= bound).all(), f"worst d/bound {(d / bound).max():.3g}"
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [("e4m3", 22, 6656, 7296), ("e4m3", 69, 3296, 4160),
+                                       ("e2m1", 16, 704, 8128), ("e2m1", 3, 17000, 4096),
+                                       ("e4m3", 9, 384, 2400)])
+def test_wq_decode_error(gpu, fmt, M, N, K):
+    """fp32 C against 64 bits: no further off than the upcast and the 256x256 bf16 tile (an
+    explicit block) are, over long ranges of K, uneven ones and 16 splits.  (Both errors are
+    2-norms over M N elements and three seeds: they scatter by about a percent, 2 at the
+    smallest.)"""
+    import torch
+    say(f"wq decode error {fmt} {M}x{N}x{K}")
+    mag = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6], device=gpu, dtype=torch.float64)
+    mag = torch.cat([mag, -mag])
+    err = [0.0, 0.0]
+    for seed in (1, 2, 3):
+        g = torch.Generator(device=gpu)
+        g.manual_seed(seed)
+        a = tx.aligned_rows(torch.randn((M, K), generator=g, device=gpu).bfloat16())
+        s = torch.randint(124, 131, (N, K // 32), generator=g, device=gpu, dtype=torch.uint8)
+        if fmt == "e2m1":
+            b = torch.randint(0, 256, (K // 2, N), generator=g, device=gpu, dtype=torch.uint8)
+            bv = mag[torch.stack([b & 15, b >> 4], 1).long()].view(K, N)
+        else:
+            b = torch.randn((K, N), generator=g, device=gpu).to(torch.float8_e4m3fn)
+            bv = b.float().double()
+        bv = bv * torch.exp2(s.double() - 127).repeat_interleave(32, 1).t()
+        want = a.double() @ bv
+        for i, block in enumerate(((0, 0, 0), (256, 256, 64))):
+            p = tx.plan(tx.make_desc(M, N, K, tx.BF16, tx.F32, b_type=FMT_TX[fmt],
+                                     scale_mode=tx.SCALE_MX32, block=block, lda=a.stride(0),
+                                     ldb=-(-N // 16) * 16, ldc=-(-N // 4) * 4))
+            assert p.kernel == (tx.KERNEL_GEMM_MX_BF16 if i else tx.KERNEL_DECODE_MX_BF16)
+            got = tx.dot_scaled(a, None, "bf16", tx.aligned_rows(b, col_ok=False), s, fmt, plan=p)
+            err[i] += float((got.double() - want).norm() / want.norm())
+    assert err[0] <= 1.03 * err[1], err

@@ -71,7 +71,12 @@
 // wave upcasts its B fragments in registers on the way to the MFMA (W = 128
 // strips), so B is read once in its own bytes instead of being written to
 // memory and read back as bf16.  The K order of the MFMAs is the plain
-// kernel's, so the sums are those of the bf16 dot of the upcast operand.
+// kernel's, their fp32 sums run in two chains that take 4 batches (512 K) each in
+// turn: up to 4 batches a split they are those of the bf16 dot of the upcast
+// operand, and past it no less exact than those of the upcast and the bf16
+// tile, which splits K further (bf16 x e4m3 22x6656x7296 against 64 bits: that
+// 1.03e-7, one chain 1.36e-7, two 1.01e-7).  16 splits are added in halves
+// (bf16 x e2m1 16x704x8128: that 6.4e-8, one sum of 16 7.5e-8, halves 6.1e-8).
 //  * B's batch is 128 K: 64 packed rows or 128 byte rows of 128 bytes, 16-byte
 //    chunk c of row r at c ^ swz(r).  ds_read_b64_tr_b8 hands a lane 8 rows of
 //    one column, and the 8 rows are the addressing lanes' choice: e2m1 takes
@@ -89,7 +94,8 @@
 //    than three, one branch for the upcast rather than one a fragment, load
 //    addresses kept and advanced rather than worked out, and a loop that is not
 //    unrolled by the ring (its code holds both upcasts): 0.55 us a batch.  M =
-//    32, N = K = 8192: 23.9 -> 19.3 us (e2m1), 25.2 -> 19.9 (e4m3).
+//    32, N = K = 8192: 23.9 -> 19.3 us (e2m1), 25.2 -> 19.9 (e4m3); with two
+//    chains of sums 19.5 -> 19.1 (e2m1).
 //  * Scales are staged per segment of 128 groups like decode_f8.h's MX form;
 //    columns past N and groups past K take a unit scale (their codes are 0).
 #pragma once
@@ -103,6 +109,7 @@ namespace txk {
 
 // B's format in the 16-bit decode kernel: A's type, or microscaled (WQ).
 enum { WQ_NONE = 0, WQ_MX_E2M1, WQ_MX_E4M3, WQ_MX_E5M2, WQ_NV_E2M1 };
+constexpr int kWqChain = 4; // batches that one of its two chains of fp32 sums takes in turn
 #define tx_unit_scales TX_TU_CAT(tx_unit_scales, TX_TU)
 __device__ uint32_t tx_unit_scales[2] = {0x7f7f7f7fu, 0x38383838u}; // e8m0 2^0; e4m3 1.0
 
@@ -728,7 +735,7 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
     for (int u = 0; u < Cfg::VPB; ++u)
       wq_src[u] += wq_step[u];
   };
-  auto wq_consume = [&](const uint8_t *slot, int i) {
+  auto wq_consume = [&](const uint8_t *slot, int i, f32x4_t (&sums)[JB][T]) {
     constexpr int T4 = T < 4 ? T : 4, NB = Cfg::FP4 ? 2 : 4;
     const uint32_t base = lds_addr(slot);
     const int b = b_begin + i;
@@ -778,7 +785,7 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
         for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
           for (int t = 0; t < T4; ++t)
-            acc[jj][t] = mfma16x16x32<BF>(bf[jj], a[ks][t], acc[jj][t]);
+            sums[jj][t] = mfma16x16x32<BF>(bf[jj], a[ks][t], sums[jj][t]);
         if constexpr (T > 4) { // slices past 64 rows: tiles 4 .. T - 1, two steps a read
           if (ks & 1)
             continue;
@@ -796,7 +803,8 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
             for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
               for (int t = 4; t < T; ++t)
-                acc[jj][t] = mfma16x16x32<BF>(h ? bn[jj] : bf[jj], am[h][t - 4], acc[jj][t]);
+                sums[jj][t] =
+                    mfma16x16x32<BF>(h ? bn[jj] : bf[jj], am[h][t - 4], sums[jj][t]);
         }
       }
     };
@@ -813,21 +821,39 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
 #pragma unroll
     for (int s = 0; s < S - 1; ++s)
       wq_issue(s, ring + s * SLOT);
-    // The loop below, not unrolled: a batch's code holds both upcasts.
+    // The loop below, unrolled by the two chains only: a batch's code holds both
+    // upcasts.
+    f32x4_t acc2[JB][T];
+#pragma unroll
+    for (int jj = 0; jj < JB; ++jj)
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        acc2[jj][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     int s = 0, sl = S - 1;
-    for (int i = 0; i < nb; ++i) {
-      if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
+    auto run = [&](int i, f32x4_t (&sums)[JB][T]) {
+      for (const int end = i + kWqChain < nb ? i + kWqChain : nb; i < end; ++i) {
+        if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
+          asm volatile("s_barrier" ::: "memory");
+          stage_scales(i);
+          wait_vmcnt<0>();
+        }
+        wait_vmcnt<(S - 2) * Cfg::VPB>();
         asm volatile("s_barrier" ::: "memory");
-        stage_scales(i);
-        wait_vmcnt<0>();
+        wq_issue(i + S - 1, ring + sl * SLOT);
+        wq_consume(ring + s * SLOT, i, sums);
+        s = s + 1 == S ? 0 : s + 1;
+        sl = sl + 1 == S ? 0 : sl + 1;
       }
-      wait_vmcnt<(S - 2) * Cfg::VPB>();
-      asm volatile("s_barrier" ::: "memory");
-      wq_issue(i + S - 1, ring + sl * SLOT);
-      wq_consume(ring + s * SLOT, i);
-      s = s + 1 == S ? 0 : s + 1;
-      sl = sl + 1 == S ? 0 : sl + 1;
+    };
+    for (int i = 0; i < nb; i += 2 * kWqChain) {
+      run(i, acc);
+      run(i + kWqChain, acc2);
     }
+#pragma unroll
+    for (int jj = 0; jj < JB; ++jj)
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        acc[jj][t] += acc2[jj][t];
     goto k_loop_done;
   }
 #pragma unroll
@@ -940,16 +966,28 @@ k_loop_done:
   __syncthreads();
   if (!*reinterpret_cast<volatile uint32_t *>(&last_flag))
     return;
-  // Last arrival: sum = partial 0 + partial 1 + .. in split order, its own
-  // from registers; NQ splits' loads in flight before any is used.
+  // Last arrival: sum = partial 0 + partial 1 + .. in split order (WQ: 16 of them
+  // in halves), its own from registers; NQ splits' loads in flight before any is used.
   f32x4_t sum[JB][T];
 #pragma unroll
   for (int jj = 0; jj < JB; ++jj)
 #pragma unroll
     for (int t = 0; t < T; ++t)
       sum[jj][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  [[maybe_unused]] f32x4_t low[JB][T]; // WQ: the first half of 16 splits
   constexpr int NQ = 4 / JB;
   for (int q0 = 0; q0 < p.ksplit; q0 += NQ) {
+    if constexpr (WQ != WQ_NONE) {
+      if (q0 == 8) {
+#pragma unroll
+        for (int jj = 0; jj < JB; ++jj)
+#pragma unroll
+          for (int t = 0; t < T; ++t) {
+            low[jj][t] = sum[jj][t];
+            sum[jj][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    }
     v4i_t v[NQ][JB][T];
 #pragma unroll
     for (int qq = 0; qq < NQ; ++qq)
@@ -971,6 +1009,15 @@ k_loop_done:
           for (int t = 0; t < T; ++t)
             sum[jj][t] +=
                 q0 + qq == split ? acc[jj][t] : __builtin_bit_cast(f32x4_t, v[qq][jj][t]);
+  }
+  if constexpr (WQ != WQ_NONE) {
+    if (p.ksplit > 8) {
+#pragma unroll
+      for (int jj = 0; jj < JB; ++jj)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          sum[jj][t] += low[jj][t];
+    }
   }
 #pragma unroll
   for (int jj = 0; jj < JB; ++jj)
