@@ -72,11 +72,11 @@
 // strips), so B is read once in its own bytes instead of being written to
 // memory and read back as bf16.  The K order of the MFMAs is the plain
 // kernel's, their fp32 sums run in two chains that take 4 batches (512 K) each in
-// turn: up to 4 batches a split they are those of the bf16 dot of the upcast
+// turn (halves of 5 to 7): up to 4 batches a split they are those of the bf16 dot of the upcast
 // operand, and past it no less exact than those of the upcast and the bf16
 // tile, which splits K further (bf16 x e4m3 22x6656x7296 against 64 bits: that
-// 1.03e-7, one chain 1.36e-7, two 1.01e-7).  16 splits are added in halves
-// (bf16 x e2m1 16x704x8128: that 6.4e-8, one sum of 16 7.5e-8, halves 6.1e-8).
+// 1.03e-7, one chain 1.36e-7, two 1.01e-7).  4 splits or more are added in halves
+// (16 of bf16 x e2m1 16x704x8128: that 6.4e-8, one row 7.5e-8, halves 6.1e-8).
 //  * B's batch is 128 K: 64 packed rows or 128 byte rows of 128 bytes, 16-byte
 //    chunk c of row r at c ^ swz(r).  ds_read_b64_tr_b8 hands a lane 8 rows of
 //    one column, and the 8 rows are the addressing lanes' choice: e2m1 takes
@@ -95,7 +95,7 @@
 //    addresses kept and advanced rather than worked out, and a loop that is not
 //    unrolled by the ring (its code holds both upcasts): 0.55 us a batch.  M =
 //    32, N = K = 8192: 23.9 -> 19.3 us (e2m1), 25.2 -> 19.9 (e4m3); with two
-//    chains of sums 19.5 -> 19.1 (e2m1).
+//    chains of sums 19.6 -> 19.4 (e2m1).
 //  * Scales are staged per segment of 128 groups like decode_f8.h's MX form;
 //    columns past N and groups past K take a unit scale (their codes are 0).
 #pragma once
@@ -109,7 +109,6 @@ namespace txk {
 
 // B's format in the 16-bit decode kernel: A's type, or microscaled (WQ).
 enum { WQ_NONE = 0, WQ_MX_E2M1, WQ_MX_E4M3, WQ_MX_E5M2, WQ_NV_E2M1 };
-constexpr int kWqChain = 4; // batches that one of its two chains of fp32 sums takes in turn
 #define tx_unit_scales TX_TU_CAT(tx_unit_scales, TX_TU)
 __device__ uint32_t tx_unit_scales[2] = {0x7f7f7f7fu, 0x38383838u}; // e8m0 2^0; e4m3 1.0
 
@@ -829,9 +828,10 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
 #pragma unroll
       for (int t = 0; t < T; ++t)
         acc2[jj][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int chain = nb > 4 && nb < 8 ? (nb + 1) / 2 : 4; // batches a turn
     int s = 0, sl = S - 1;
     auto run = [&](int i, f32x4_t (&sums)[JB][T]) {
-      for (const int end = i + kWqChain < nb ? i + kWqChain : nb; i < end; ++i) {
+      for (const int end = i + chain < nb ? i + chain : nb; i < end; ++i) {
         if (i > 0 && i % Cfg::SEG_B == 0) { // every wave has read the segment before
           asm volatile("s_barrier" ::: "memory");
           stage_scales(i);
@@ -845,9 +845,9 @@ __global__ void __launch_bounds__(kDecodeWaves * 64, 1) decode16_kernel(Decode16
         sl = sl + 1 == S ? 0 : sl + 1;
       }
     };
-    for (int i = 0; i < nb; i += 2 * kWqChain) {
+    for (int i = 0; i < nb; i += 2 * chain) {
       run(i, acc);
-      run(i + kWqChain, acc2);
+      run(i + chain, acc2);
     }
 #pragma unroll
     for (int jj = 0; jj < JB; ++jj)
@@ -966,19 +966,19 @@ k_loop_done:
   __syncthreads();
   if (!*reinterpret_cast<volatile uint32_t *>(&last_flag))
     return;
-  // Last arrival: sum = partial 0 + partial 1 + .. in split order (WQ: 16 of them
-  // in halves), its own from registers; NQ splits' loads in flight before any is used.
+  // Last arrival: sum = partial 0 + partial 1 + .. in split order (WQ: 4 or more in
+  // halves), its own from registers; NQ splits' loads in flight before any is used.
   f32x4_t sum[JB][T];
 #pragma unroll
   for (int jj = 0; jj < JB; ++jj)
 #pragma unroll
     for (int t = 0; t < T; ++t)
       sum[jj][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  [[maybe_unused]] f32x4_t low[JB][T]; // WQ: the first half of 16 splits
+  [[maybe_unused]] f32x4_t low[JB][T]; // WQ: the first half of 4 splits or more
   constexpr int NQ = 4 / JB;
   for (int q0 = 0; q0 < p.ksplit; q0 += NQ) {
     if constexpr (WQ != WQ_NONE) {
-      if (q0 == 8) {
+      if (q0 == p.ksplit / 2 && q0 > 1) {
 #pragma unroll
         for (int jj = 0; jj < JB; ++jj)
 #pragma unroll
@@ -1011,7 +1011,7 @@ k_loop_done:
                 q0 + qq == split ? acc[jj][t] : __builtin_bit_cast(f32x4_t, v[qq][jj][t]);
   }
   if constexpr (WQ != WQ_NONE) {
-    if (p.ksplit > 8) {
+    if (p.ksplit > 2) {
 #pragma unroll
       for (int jj = 0; jj < JB; ++jj)
 #pragma unroll
